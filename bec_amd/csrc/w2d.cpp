@@ -58,10 +58,9 @@ extern "C" int bec_run_2d(const bec_2d_params *pp, double *m, double *var, doubl
         ~StreamGuard() { (void)hipStreamDestroy(s); }
     } guard{s};
     Buffers buf;
-    double2 *d_gs = nullptr, *d_pv = nullptr;
+    double2 *d_gs = nullptr;
     double *d_rep = nullptr, *d_meas = nullptr, *d_avn = nullptr;
     BEC_HIP(buf.alloc((void **)&d_gs, sizeof(double2) * cells));
-    if (p.gs_rule == 2) BEC_HIP(buf.alloc((void **)&d_pv, sizeof(double2) * cells));
     BEC_HIP(buf.alloc((void **)&d_rep, sizeof(double) * 4));
     BEC_HIP(buf.alloc((void **)&d_meas, sizeof(double) * 3 * p.ne * p.n_meas));
     if (avn) BEC_HIP(buf.alloc((void **)&d_avn, sizeof(double) * cells * p.ne));
@@ -77,7 +76,7 @@ extern "C" int bec_run_2d(const bec_2d_params *pp, double *m, double *var, doubl
         }
     } eg{e0, e1};
     BEC_HIP(hipEventRecord(e0, s));
-    BEC_HIP(bec::run_w2d_ground_state(p, d_gs, d_pv, d_rep, s));
+    BEC_HIP(bec::run_w2d_ground_state(p, d_gs, d_rep, s));
     BEC_HIP(bec::run_w2d_ensemble(p, d_gs, d_meas, d_avn, s));
     BEC_HIP(hipEventRecord(e1, s));
     std::vector<double> h_rep(4), h_meas(3 * (size_t)p.ne * p.n_meas), h_avn(avn ? cells * p.ne : 0);
