@@ -134,4 +134,83 @@ template <int G> __device__ __forceinline__ double group_sum(double v)
     return v;
 }
 
+// ------------------------------------------------------ wave-wide sums
+// Sums across the 64 lanes through the vector unit's own lane moves (DPP within
+// rows of 16 lanes, permlane swaps between rows and halves) instead of LDS
+// permutes, whose latency (about 100 cycles each, two per double) is exposed in
+// the latency-bound kernels.  Fixed order: every run gives the same bits.
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141;   // quad_perm [1,0,3,2], [2,3,0,1]; i -> 7 - i
+constexpr int DPP_ROR8 = 0x128;                                            // row_ror:8, lane i <- lane i ^ 8
+
+typedef unsigned lane_pair_t __attribute__((ext_vector_type(2)));
+
+// Exchanges the upper 32 lanes of a with the lower 32 of b.
+__device__ __forceinline__ void swap32(double &a, double &b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const lane_pair_t lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const lane_pair_t hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    a = __longlong_as_double(((long long)hi.x << 32) | lo.x);
+    b = __longlong_as_double(((long long)hi.y << 32) | lo.y);
+}
+
+// Exchanges the odd rows (of 16 lanes) of a with the even rows of b.
+__device__ __forceinline__ void swap16(double &a, double &b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const lane_pair_t lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const lane_pair_t hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    a = __longlong_as_double(((long long)hi.x << 32) | lo.x);
+    b = __longlong_as_double(((long long)hi.y << 32) | lo.y);
+}
+
+// The sum over all 64 lanes, in every lane.
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += dpp_move<DPP_XOR1>(v);
+    v += dpp_move<DPP_XOR2>(v);
+    v += dpp_move<DPP_HALF_MIRROR>(v);
+    v += dpp_move<DPP_ROR8>(v);
+    double w = v;
+    swap16(v, w);
+    v += w;
+    w = v;
+    swap32(v, w);
+    return v + w;
+}
+
+// The sums of K <= 8 values over all 64 lanes: lane l returns sum l / 8 (0 for
+// l / 8 >= K).  The lanes halve the values they carry in the first three
+// exchanges, so eight sums cost ten exchanges instead of forty-eight.
+template <int K> __device__ __forceinline__ double wave_sums(const double (&v)[K])
+{
+    static_assert(K <= 8, "at most eight sums");
+    double a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = i < K ? v[i] : 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {   // lanes 0-31 keep a[i], lanes 32-63 a[i + 4]
+        swap32(a[i], a[i + 4]);
+        a[i] += a[i + 4];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {   // even rows keep a[i], odd rows a[i + 2]
+        swap16(a[i], a[i + 2]);
+        a[i] += a[i + 2];
+    }
+    const bool up = threadIdx.x & 8;   // the row's lower eight lanes keep a[0], its upper a[1]
+    const double keep = up ? a[1] : a[0], send = up ? a[0] : a[1];
+    double t = keep + dpp_move<DPP_ROR8>(send);
+    t += dpp_move<DPP_XOR1>(t);
+    t += dpp_move<DPP_XOR2>(t);
+    return t + dpp_move<DPP_HALF_MIRROR>(t);
+}
+
 } // namespace bec

@@ -75,10 +75,16 @@ __device__ __forceinline__ int freq_of(const Axis &a, int p)
     return p / sub + a.r1 * (p % sub);
 }
 
-__device__ __forceinline__ void sincos_any(double x, double *s, double *c)
+// the phase factors e^{i x}, e^{i y} of the two components
+__device__ __forceinline__ void phases(double x, double y, double2 &u, double2 &v)
 {
-    if (fabs(x) < DSINCOS_MAX) fast_sincos_f64(x, s, c);
-    else sincos(x, s, c);
+    if (fmax(fabs(x), fabs(y)) < DSINCOS_MAX) {
+        fast_sincos_f64(x, &u.y, &u.x);
+        fast_sincos_f64(y, &v.y, &v.x);
+    } else {
+        sincos(x, &u.y, &u.x);
+        sincos(y, &v.y, &v.x);
+    }
 }
 
 // A thread's butterfly of one stage: `on` when it has one, LDS offset of its
@@ -280,21 +286,18 @@ template <int RF, int RL, int NB> struct Fft {
     }
 };
 
-// Sum of K doubles over the workgroup (wave shuffles, then LDS across waves);
-// every thread receives the totals.
-template <int K> __device__ void block_sum(double (&v)[K], double *scratch)
+// Sums of K doubles over the workgroup (within the waves, then LDS across
+// them), in a fixed order; every thread receives the totals.
+template <int K> __device__ __forceinline__ void block_sum(double (&v)[K], double *scratch)
 {
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < K; ++k) scratch[wave * K + k] = v[k];
+    const double t = K == 1 ? wave_sum(v[0]) : wave_sums<K>(v);
+    if ((lane & 7) == 0 && lane / 8 < K) scratch[wave * K + lane / 8] = t;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         double s = 0.0;
+#pragma unroll
         for (int w = 0; w < THREADS / 64; ++w) s += scratch[w * K + k];
         v[k] = s;
     }
@@ -606,11 +609,10 @@ __global__ __launch_bounds__(THREADS) void w2d_ensemble_kernel(W2dParams p, cons
                     const double na = nrm(a), nb = nrm(b), base = p.mu - F.r2(m) / 4.0;
                     const double dA = -p.g11 * na - p.g12 * nb + base + 0.5 * p.E;
                     const double dB = -p.g22 * nb - p.g12 * na + base - 0.5 * p.E;
-                    double sa, ca, sb, cb;
-                    sincos_any(-p.dtW * dA, &sa, &ca);
-                    sincos_any(-p.dtW * dB, &sb, &cb);
-                    x[0][m] = cm(a, make_double2(ca, sa));
-                    x[1][m] = cm(b, make_double2(cb, sb));
+                    double2 ea, eb;
+                    phases(-p.dtW * dA, -p.dtW * dB, ea, eb);
+                    x[0][m] = cm(a, ea);
+                    x[1][m] = cm(b, eb);
                     __builtin_amdgcn_sched_barrier(0);   // one cell after the other: fewer registers
                 }
             F.to_k(x, k);
@@ -627,10 +629,9 @@ __global__ __launch_bounds__(THREADS) void w2d_ensemble_kernel(W2dParams p, cons
 #pragma unroll
                 for (int m = 0; m < RL; ++m) {
                     const double2 a = k[0][m], b = k[1][m];
-                    const double2 b1 = make_double2((b.x - a.y) / r2, (b.y + a.x) / r2);   // (b + i a)/sqrt 2
-                    const double2 aa = make_double2((a.x - b.y) / r2, (a.y + b.x) / r2);   // (a + i b)/sqrt 2
-                    s[0] += nrm(aa);
-                    s[1] += nrm(b1);
+                    // |(a + i b)/sqrt 2|^2, |(b + i a)/sqrt 2|^2
+                    s[0] += 0.5 * nrm(make_double2(a.x - b.y, a.y + b.x));
+                    s[1] += 0.5 * nrm(make_double2(b.x - a.y, b.y + a.x));
                     s[2] += a.x * b.x + a.y * b.y;
                     s[3] += a.x * b.y - a.y * b.x;
                     s[4] += nrm(a);
