@@ -2,15 +2,21 @@
 // the GPU: calculate_steady_state (wigner_1d.cpp:166-243) and main_loop
 // (wigner_1d.cpp:245-445), FP64.
 //
-// A trajectory is one wavefront.  Its state lives in registers: lane l holds
-// cells l, l + 64, ... (up to eight per lane, nv <= 512) of both components,
-// in whichever space the step is in.  The program's lattice has an odd,
-// generally prime, number of cells (41), so the transforms are direct DFTs:
-// the state is staged into LDS, and each lane accumulates its outputs
-// sum_j x_j w^(j k) over the staged inputs (broadcast reads) with the
-// exponent index (j k) mod nv stepped incrementally into a twiddle table in
-// LDS.  Both components share each table read.  HBM sees the ground state
-// read once per trajectory and the samples written.
+// A trajectory is one workgroup (one wavefront up to 63 cells).  The program's
+// lattice has an odd, generally prime, number n = 2 h + 1 of cells (41), so the
+// transforms are direct DFTs, folded about the middle: with
+// S_j = x_j + x_{n-j} and D_j = x_j - x_{n-j} (S_0 = x_0),
+//   X_k     = sum_{j<=h} S_j cos(2 pi j k / n) +- i sum_{j<=h} D_j sin(2 pi j k / n),
+//   X_{n-k} = the same with the other sign,
+// so a thread that owns cells k and n - k of one component forms both outputs
+// with 4 multiply-adds per j, a quarter of the plain sum's.  It stages its own
+// S_k and D_k into LDS; the j loop reads them as broadcasts.  Up to h = 32 the
+// thread keeps its cosines and sines in registers; longer lattices step
+// the index (j k) mod n into a table in LDS.  The components meet through their
+// densities (nonlinear step) and at the pulses, exchanged through LDS.  The
+// samples' six sums are reduced together, halving the values a lane carries
+// while the lanes combine, and the square root and division of a sample wait
+// until the run is over, when the lanes do them in parallel.
 //
 // Conventions of the program (and of the oracle's restatement): the k-space
 // factor is -k^2 with k = dk j for 2j <= nv else dk (j - nv), dk = pi/zmax;
@@ -20,13 +26,14 @@
 #include <math.h>
 
 #include "backend1d.hpp"
+#include "fastmath.hpp"
+#include "fft_reg.hpp"
 #include "philox.hpp"
 
 namespace bec {
 
 namespace {
 
-constexpr int LANES = 64;
 constexpr int MAXNV = W1D_MAX_NV;
 
 __device__ __forceinline__ double2 cm(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
@@ -35,289 +42,327 @@ __device__ __forceinline__ double nrm(double2 a) { return a.x * a.x + a.y * a.y;
 
 __device__ __forceinline__ double kval(int j, int n, double dk) { return (2 * j > n) ? dk * (j - n) : dk * j; }
 
-// tw[m] = exp(-2 pi i m / n)
-__device__ void make_twiddles(double2 *tw, int n)
+// the phase factors e^{i x}, e^{i y} (both at once: two independent chains)
+__device__ __forceinline__ void phases(double x, double y, double2 &u, double2 &v)
 {
-    for (int m = threadIdx.x; m < n; m += LANES) {
+    if (fmax(fabs(x), fabs(y)) < DSINCOS_MAX) {
+        fast_sincos_f64(x, &u.y, &u.x);
+        fast_sincos_f64(y, &v.y, &v.x);
+    } else {
+        sincos(x, &u.y, &u.x);
+        sincos(y, &v.y, &v.x);
+    }
+}
+
+// A thread's share of a line of n = 2 h + 1 values of NC components: the pair
+// (k, n - k) of component c (k = 0 alone), for the first NC (h + 1) threads.
+struct Line {
+    int n, h, hs, k, c;   // hs: stride between the components' LDS rows (odd: their broadcasts meet no bank twice)
+    bool on, two;         // has a pair; has a second cell
+    double2 *S, *D;       // [NC][hs]
+    const double2 *tw;    // (cos, sin)(2 pi m / n), m < n
+};
+
+// LDS row of S or D: h + 1 values and zeros up to a (non-zero) multiple of eight, an odd length
+__host__ __device__ constexpr int row_len(int n) { return (n < 2 ? 8 : (n / 2 + 7) & ~7) + 1; }
+
+// LDS: the factor table, then S and D (one row of each per component).
+template <int NC> __device__ __forceinline__ Line make_line(int n, double2 *lds)
+{
+    Line l;
+    l.n = n;
+    l.h = n >> 1;
+    l.hs = row_len(n);
+    l.c = NC > 1 && (int)threadIdx.x > l.h ? 1 : 0;
+    l.k = (int)threadIdx.x - l.c * (l.h + 1);
+    l.on = l.k <= l.h;
+    l.two = l.on && l.k > 0;
+    l.tw = lds;
+    l.S = lds + n;
+    l.D = l.S + NC * l.hs;
+    for (int m = threadIdx.x; m < n; m += blockDim.x) {
         double s, c;
-        sincospi(-2.0 * m / n, &s, &c);
-        tw[m] = make_double2(c, s);
+        sincospi(2.0 * m / n, &s, &c);
+        lds[m] = make_double2(c, s);
     }
+    for (int m = threadIdx.x; m < 2 * NC * l.hs; m += blockDim.x) l.S[m] = make_double2(0.0, 0.0);
+    if (!l.on) l.k = 0;
     __syncthreads();
+    return l;
 }
 
-// Stage the lane's cells of one or two vectors into LDS.
-template <int R, bool TWO>
-__device__ __forceinline__ void stage(const double2 (&a)[R], const double2 (&b)[R], double2 *sa, double2 *sb, int n)
-{
+// The cosines and sines of a thread's output pair, read once and held in
+// registers for lines of h <= H (H = 0: read from the table every time).
+template <int H> struct Factors {
+    double c[H + 1], s[H + 1];
+    __device__ __forceinline__ void load(const Line &l)
+    {
+        if constexpr (H > 0) {
+            int idx = 0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        if (k < n) {
-            sa[k] = a[r];
-            if (TWO) sb[k] = b[r];
-        }
-    }
-    __syncthreads();
-}
-
-// out[k] = sum_j s[j] exp(sign 2 pi i j k / n) for the lane's k, from the staged
-// inputs; ends with a barrier so the staging buffers may be overwritten.
-template <int R, bool TWO>
-__device__ __forceinline__ void dft(const double2 *sa, const double2 *sb, const double2 *tw, int n, int sign,
-                                    double2 (&oa)[R], double2 (&ob)[R])
-{
-    const double sg = sign < 0 ? 1.0 : -1.0;
-    int step[R], idx[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        step[r] = k < n ? k : 0;
-        idx[r] = 0;
-        oa[r] = make_double2(0.0, 0.0);
-        ob[r] = make_double2(0.0, 0.0);
-    }
-    // unrolled so that several table reads are in flight: one wavefront per
-    // trajectory leaves LDS latency exposed otherwise
-#pragma unroll 4
-    for (int j = 0; j < n; ++j) {
-        const double2 xa = sa[j];
-        const double2 xb = TWO ? sb[j] : xa;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            double2 w = tw[idx[r]];
-            w.y *= sg;
-            oa[r].x = fma(xa.x, w.x, fma(-xa.y, w.y, oa[r].x));
-            oa[r].y = fma(xa.x, w.y, fma(xa.y, w.x, oa[r].y));
-            if (TWO) {
-                ob[r].x = fma(xb.x, w.x, fma(-xb.y, w.y, ob[r].x));
-                ob[r].y = fma(xb.x, w.y, fma(xb.y, w.x, ob[r].y));
+            for (int j = 1; j <= H; ++j) {
+                idx += l.k;
+                idx -= idx >= l.n ? l.n : 0;
+                const double2 w = l.tw[idx];
+                c[j] = w.x;
+                s[j] = w.y;
             }
-            idx[r] += step[r];
-            idx[r] -= idx[r] >= n ? n : 0;
         }
     }
-    __syncthreads();
-}
+};
 
-// x -> k of the register state: the +i transform and 1/n
-template <int R, bool TWO>
-__device__ __forceinline__ void to_k(double2 (&a)[R], double2 (&b)[R], double2 *sa, double2 *sb, const double2 *tw,
-                                     int n)
+// (x_k, x_{n-k}) <- sum_j x_j exp(SIGN 2 pi i j k / n) of the thread's pair
+template <int SIGN, int H>
+__device__ __forceinline__ void dft_line(const Line &l, const Factors<H> &f, double2 &x, double2 &y)
 {
-    stage<R, TWO>(a, b, sa, sb, n);
-    dft<R, TWO>(sa, sb, tw, n, +1, a, b);
-    const double inv = 1.0 / n;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        a[r] = cs(a[r], inv);
-        b[r] = cs(b[r], inv);
+    if (l.on) {
+        l.S[l.c * l.hs + l.k] = l.two ? make_double2(x.x + y.x, x.y + y.y) : x;
+        l.D[l.c * l.hs + l.k] = make_double2(x.x - y.x, x.y - y.y);
     }
-}
-
-template <int R, bool TWO>
-__device__ __forceinline__ void to_x(double2 (&a)[R], double2 (&b)[R], double2 *sa, double2 *sb, const double2 *tw,
-                                     int n)
-{
-    stage<R, TWO>(a, b, sa, sb, n);
-    dft<R, TWO>(sa, sb, tw, n, -1, a, b);
-}
-
-template <int K> __device__ __forceinline__ void wave_sum(double (&v)[K])
-{
+    __syncthreads();
+    const double2 *S = l.S + l.c * l.hs, *D = l.D + l.c * l.hs;
+    double2 e = S[0], o = make_double2(0.0, 0.0);
+    auto add = [&](double2 sj, double2 dj, double c, double s) {
+        e.x = fma(sj.x, c, e.x);
+        e.y = fma(sj.y, c, e.y);
+        o.x = fma(dj.x, s, o.x);
+        o.y = fma(dj.y, s, o.y);
+    };
+    if constexpr (H > 0) {
+        // straight line over H terms (the rows end in zeros), so that the reads run ahead of the sums
 #pragma unroll
-    for (int k = 0; k < K; ++k)
-        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, LANES);
+        for (int j = 1; j <= H; ++j) add(S[j], D[j], f.c[j], f.s[j]);
+    } else {
+        int idx = 0;
+#pragma unroll 8
+        for (int j = 1; j <= l.h; ++j) {
+            idx += l.k;
+            idx -= idx >= l.n ? l.n : 0;
+            const double2 w = l.tw[idx];
+            add(S[j], D[j], w.x, w.y);
+        }
+    }
+    if (SIGN > 0) {
+        x = make_double2(e.x - o.y, e.y + o.x);
+        y = make_double2(e.x + o.y, e.y - o.x);
+    } else {
+        x = make_double2(e.x + o.y, e.y - o.x);
+        y = make_double2(e.x - o.y, e.y + o.x);
+    }
+    __syncthreads();   // the staging rows may be overwritten
+}
+
+// Sums of K <= 8 values over the workgroup, in a fixed order; thread t returns
+// sum t / 8 (in every wave).
+template <int K> __device__ __forceinline__ double block_sums(const double (&v)[K], double *scratch)
+{
+    const double t = wave_sums<K>(v);
+    const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+    if (waves == 1) return t;
+    if ((lane & 7) == 0) scratch[threadIdx.x >> 3] = t;
+    __syncthreads();
+    double s = 0.0;
+    for (int w = 0; w < waves; ++w) s += scratch[w * 8 + (lane >> 3)];
+    __syncthreads();
+    return s;
+}
+
+// the sum of one value, in every thread
+__device__ __forceinline__ double block_sum(double x, double *scratch)
+{
+    const double t = wave_sum(x);
+    const int waves = blockDim.x >> 6;
+    if (waves == 1) return t;
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = t;
+    __syncthreads();
+    double s = 0.0;
+    for (int w = 0; w < waves; ++w) s += scratch[w];
+    __syncthreads();
+    return s;
 }
 
 // calculate_steady_state (wigner_1d.cpp:166-243): uniform n0 start, ntG - 1
 // imaginary-time steps with the itmax midpoint iteration, the N series after
-// each pass; then the residual of the x-space result.  One wavefront.
-template <int R>
-__global__ __launch_bounds__(LANES) void w1d_ground_state_kernel(W1dParams p, int n, double2 *gs_out, double *ntot,
-                                                                 double *rep_out)
+// each pass; then the residual of the x-space result.  One workgroup.
+template <int H>
+__global__ __launch_bounds__(H ? 64 : 256) void w1d_ground_state_kernel(W1dParams p, int n, double2 *gs_out, double *ntot,
+                                                               double *rep_out)
 {
-    extern __shared__ double2 lds[];   // twiddles, then two staging vectors: 3 nv
-    double2 *tw = lds, *sa = lds + n, *sb = lds + 2 * n;
-    make_twiddles(tw, n);
-    const double dk = M_PI / p.zmax;
-    double2 a[R], u[R];
-    double propG[R], pG[R], k2[R], z[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        const double kv = kval(k, n, dk);
-        z[r] = -p.zmax + p.dz * k;
-        k2[r] = kv * kv;
-        propG[r] = exp(-k2[r] * p.dt / 2.0);
-        pG[r] = p.mu - z[r] * z[r] / 4.0;
-        a[r] = make_double2(k < n ? p.n0 : 0.0, 0.0);
-    }
-    to_k<R, false>(a, u, sa, sb, tw, n);
+    extern __shared__ double2 lds[];
+    __shared__ double scratch[32];
+    const Line l = make_line<1>(n, lds);
+    Factors<H> f;
+    f.load(l);
+    const double dk = M_PI / p.zmax, inv = 1.0 / n;
+    const double kv = kval(l.k, n, dk), k2 = kv * kv, propG = exp(-k2 * p.dt / 2.0);   // the same for n - k
+    const double z0 = -p.zmax + p.dz * l.k, z1 = -p.zmax + p.dz * (n - l.k);
+    const double pG0 = p.mu - z0 * z0 / 4.0, pG1 = p.mu - z1 * z1 / 4.0;
+    double2 a = make_double2(l.on ? p.n0 : 0.0, 0.0), b = make_double2(l.two ? p.n0 : 0.0, 0.0);
+    auto to_k = [&](double2 &u, double2 &v) {
+        dft_line<+1, H>(l, f, u, v);
+        u = cs(u, inv);
+        v = l.two ? cs(v, inv) : make_double2(0.0, 0.0);
+    };
+    auto to_x = [&](double2 &u, double2 &v) {
+        dft_line<-1, H>(l, f, u, v);
+        if (!l.two) v = make_double2(0.0, 0.0);
+    };
+    auto step = [&](double2 a1, double pG) {
+        double2 v = a1;
+        double da = 0.0;
+        for (int i = 0; i < p.itmax; ++i) {
+            da = exp(p.dt / 2.0 * (pG - p.g11 * nrm(v)));
+            v = cs(a1, da);
+        }
+        return cs(v, da);
+    };
+    to_k(a, b);
     double N0 = 0.0;
     for (int it = 0; it < p.ntG; ++it) {
         if (it > 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) a[r] = cs(a[r], propG[r]);
-            to_x<R, false>(a, u, sa, sb, tw, n);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const double2 a1 = a[r];
-                double2 v = a1;
-                double da = 0.0;
-                for (int i = 0; i < p.itmax; ++i) {
-                    da = exp(p.dt / 2.0 * (pG[r] - p.g11 * nrm(v)));
-                    v = cs(a1, da);
-                }
-                a[r] = cs(v, da);
-            }
-            to_k<R, false>(a, u, sa, sb, tw, n);
-#pragma unroll
-            for (int r = 0; r < R; ++r) a[r] = cs(a[r], propG[r]);
+            a = cs(a, propG);
+            b = cs(b, propG);
+            to_x(a, b);
+            a = step(a, pG0);
+            b = step(b, pG1);
+            to_k(a, b);
+            a = cs(a, propG);
+            b = cs(b, propG);
         }
-        double s[1] = {0.0};
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (threadIdx.x + LANES * r < n) s[0] += nrm(a[r]);
-        wave_sum<1>(s);
-        N0 = s[0] * p.dz * n;
+        N0 = block_sum(l.on ? nrm(a) + nrm(b) : 0.0, scratch) * p.dz * n;
         if (ntot && threadIdx.x == 0) ntot[it] = N0;
     }
-    to_x<R, false>(a, u, sa, sb, tw, n);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        if (k < n) gs_out[k] = a[r];
-    }
+    to_x(a, b);
+    if (l.on) gs_out[l.k] = a;
+    if (l.two) gs_out[n - l.k] = b;
     // residual of (-d^2/dz^2 + z^2/4 + g11 |psi|^2) psi = mu psi
-    double2 h[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) h[r] = a[r];
-    to_k<R, false>(h, u, sa, sb, tw, n);
-#pragma unroll
-    for (int r = 0; r < R; ++r) h[r] = cs(h[r], k2[r]);
-    to_x<R, false>(h, u, sa, sb, tw, n);
-    double s2[2] = {0.0, 0.0};
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if (threadIdx.x + LANES * r >= n) continue;
-        const double v = (p.mu - pG[r]) + p.g11 * nrm(a[r]);
-        h[r] = make_double2(h[r].x + v * a[r].x, h[r].y + v * a[r].y);
-        s2[0] += a[r].x * h[r].x + a[r].y * h[r].y;
-        s2[1] += nrm(a[r]);
-    }
-    wave_sum<2>(s2);
-    const double mu = s2[0] / s2[1];
-    double s1[1] = {0.0};
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-        if (threadIdx.x + LANES * r < n) s1[0] += nrm(make_double2(h[r].x - mu * a[r].x, h[r].y - mu * a[r].y));
-    wave_sum<1>(s1);
+    double2 h0 = a, h1 = b;
+    to_k(h0, h1);
+    h0 = cs(h0, k2);
+    h1 = cs(h1, k2);
+    to_x(h0, h1);
+    const double v0 = (p.mu - pG0) + p.g11 * nrm(a), v1 = (p.mu - pG1) + p.g11 * nrm(b);
+    h0 = make_double2(h0.x + v0 * a.x, h0.y + v0 * a.y);
+    h1 = make_double2(h1.x + v1 * b.x, h1.y + v1 * b.y);
+    const double num = block_sum(l.on ? a.x * h0.x + a.y * h0.y + (l.two ? b.x * h1.x + b.y * h1.y : 0.0) : 0.0, scratch);
+    const double den = block_sum(l.on ? nrm(a) + (l.two ? nrm(b) : 0.0) : 0.0, scratch);
+    const double mu = num / den;
+    const double r0 = nrm(make_double2(h0.x - mu * a.x, h0.y - mu * a.y));
+    const double r1 = nrm(make_double2(h1.x - mu * b.x, h1.y - mu * b.y));
+    const double rr = block_sum(l.on ? r0 + (l.two ? r1 : 0.0) : 0.0, scratch);
     if (threadIdx.x == 0) {
         rep_out[0] = N0;
-        rep_out[1] = sqrt(s1[0] / s2[1]) / fabs(mu);
+        rep_out[1] = sqrt(rr / den) / fabs(mu);
         rep_out[2] = mu;
     }
 }
 
-// main_loop (wigner_1d.cpp:245-445) for one trajectory per wavefront.  meas:
-// [traj][ntW][3] = {N1, N2, visibility}; avn: [traj][nv] x-space density
-// minus the vacuum term after the last step.
-template <int R>
-__global__ __launch_bounds__(LANES) void w1d_ensemble_kernel(W1dParams p, int n, const double2 *gs, double *meas,
-                                                             double *avn, uint32_t k0, uint32_t k1)
+// main_loop (wigner_1d.cpp:245-445) for one trajectory per workgroup.  meas:
+// [traj][ntW][5]; {N1, N2, visibility} of every sample in the first three on
+// return (the run stores the five sums they are made of); avn: [traj][nv]
+// x-space density minus the vacuum term after the last step.
+template <int H>
+__global__ __launch_bounds__(H ? 64 : 512) void w1d_ensemble_kernel(W1dParams p, int n, const double2 *gs, double *meas,
+                                                           double *avn, uint32_t k0, uint32_t k1)
 {
-    extern __shared__ double2 lds[];   // twiddles, then two staging vectors: 3 nv
-    double2 *tw = lds, *sa = lds + n, *sb = lds + 2 * n;
+    extern __shared__ double2 lds[];
+    __shared__ double scratch[64];
     const int traj = blockIdx.x;
-    make_twiddles(tw, n);
-    const double dk = M_PI / p.zmax, nd = p.noise_dev / 0.5;
-    double2 a[R], b[R], kw[R];
-    double base[R];
+    const Line l = make_line<2>(n, lds);
+    Factors<H> f;
+    f.load(l);
+    const double dk = M_PI / p.zmax, nd = p.noise_dev / 0.5, inv = 1.0 / n;
+    const double kv = kval(l.k, n, dk);   // k^2 is the same for n - k
+    double sn, co;
+    sincos(kv * kv * p.dt / 2.0, &sn, &co);
+    const double2 kw = make_double2(co, sn);   // exp(+i k^2 dt/2)
+    const double2 kwn = cs(kw, inv);
+    const double z0 = -p.zmax + p.dz * l.k, z1 = -p.zmax + p.dz * (n - l.k);
+    const double base0 = p.mu - z0 * z0 / 4.0, base1 = p.mu - z1 * z1 / 4.0;
+    const double gown = l.c ? p.g22 : p.g11, det = l.c ? -0.5 * p.E : 0.5 * p.E;
     // initial state: ground state + noise in x-space (:281-290), then to k-space
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        const double kv = kval(k, n, dk), z = -p.zmax + p.dz * k;
-        double sn, c;
-        sincos(kv * kv * p.dt / 2.0, &sn, &c);
-        kw[r] = make_double2(c, sn);   // exp(+i k^2 dt/2)
-        base[r] = p.mu - z * z / 4.0;
-        a[r] = b[r] = make_double2(0.0, 0.0);
-        if (k < n) {
-            double e[4];
-            noise4((uint32_t)k, (uint32_t)traj, 0u, k0, k1, e);
-            const double2 g = gs[k];
-            a[r] = make_double2(g.x + p.Va * nd * e[0], g.y + p.Va * nd * e[1]);
-            b[r] = make_double2(p.Vb * nd * e[2], p.Vb * nd * e[3]);
+    auto start = [&](int cell) {
+        double e[4];
+        noise4((uint32_t)cell, (uint32_t)traj, 0u, k0, k1, e);
+        if (l.c) return make_double2(p.Vb * nd * e[2], p.Vb * nd * e[3]);
+        const double2 g = gs[cell];
+        return make_double2(g.x + p.Va * nd * e[0], g.y + p.Va * nd * e[1]);
+    };
+    const double2 zero = make_double2(0.0, 0.0);
+    double2 x = l.on ? start(l.k) : zero, y = l.two ? start(n - l.k) : zero;
+    dft_line<+1, H>(l, f, x, y);
+    x = cs(x, inv);
+    y = l.two ? cs(y, inv) : zero;
+    // the other component's pair, through the staging rows
+    auto other = [&](double2 u, double2 v, double2 &ou, double2 &ov) {
+        if (l.on) {
+            l.S[l.c * l.hs + l.k] = u;
+            l.D[l.c * l.hs + l.k] = v;
         }
-    }
-    to_k<R, true>(a, b, sa, sb, tw, n);
+        __syncthreads();
+        ou = l.S[(1 - l.c) * l.hs + l.k];
+        ov = l.D[(1 - l.c) * l.hs + l.k];
+        __syncthreads();
+    };
     const double r2 = sqrt(2.0), V = (p.Va + p.Vb) / 2.0;
+    double *const mt = meas + (long)traj * p.ntW * 5;
     for (int nn = -p.ntW; nn < p.ntW; ++nn) {
         if (nn > -p.ntW) {
-            if (nn == 0) {   // pi/2 pulse (:308-318)
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const double2 x = a[r], y = b[r];
-                    b[r] = make_double2((y.x + x.y) / r2, (y.y - x.x) / r2);   // (b - i a)/sqrt 2
-                    a[r] = make_double2((x.x + y.y) / r2, (x.y - y.x) / r2);   // (a - i b)/sqrt 2
-                }
+            if (nn == 0) {   // pi/2 pulse (:308-318): (a - i b)/sqrt 2, (b - i a)/sqrt 2
+                double2 u, v;
+                other(x, y, u, v);
+                x = make_double2((x.x + u.y) / r2, (x.y - u.x) / r2);
+                y = make_double2((y.x + v.y) / r2, (y.y - v.x) / r2);
             }
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                a[r] = cm(a[r], kw[r]);
-                b[r] = cm(b[r], kw[r]);
-            }
-            to_x<R, true>(a, b, sa, sb, tw, n);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {   // single-shot nonlinear step (:331-337)
-                const double na = nrm(a[r]), nb = nrm(b[r]);
-                const double dA = -p.g11 * na - p.g12 * nb + base[r] + 0.5 * p.E;
-                const double dB = -p.g22 * nb - p.g12 * na + base[r] - 0.5 * p.E;
-                double sa_, ca, sb_, cb;
-                sincos(-p.dt * dA, &sa_, &ca);
-                sincos(-p.dt * dB, &sb_, &cb);
-                a[r] = cm(a[r], make_double2(ca, sa_));
-                b[r] = cm(b[r], make_double2(cb, sb_));
-            }
-            to_k<R, true>(a, b, sa, sb, tw, n);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                a[r] = cm(a[r], kw[r]);
-                b[r] = cm(b[r], kw[r]);
-            }
+            x = cm(x, kw);
+            y = cm(y, kw);
+            dft_line<-1, H>(l, f, x, y);
+            // single-shot nonlinear step (:331-337)
+            const double n0 = nrm(x), n1 = nrm(y);
+            double2 on, unused;
+            other(make_double2(n0, n1), zero, on, unused);
+            double2 e0, e1;
+            phases(-p.dt * (-gown * n0 - p.g12 * on.x + base0 + det), -p.dt * (-gown * n1 - p.g12 * on.y + base1 + det),
+                   e0, e1);
+            x = cm(x, e0);
+            y = l.two ? cm(y, e1) : zero;
+            dft_line<+1, H>(l, f, x, y);
+            x = cm(x, kwn);
+            y = l.two ? cm(y, kwn) : zero;
         }
         if (nn >= 0) {   // second pulse U^+ and measurement in k-space (:358-391)
-            double s[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                if (threadIdx.x + LANES * r >= n) continue;
-                const double2 x = a[r], y = b[r];
-                const double2 b1 = make_double2((y.x - x.y) / r2, (y.y + x.x) / r2);   // (b + i a)/sqrt 2
-                const double2 a1 = make_double2((x.x - y.y) / r2, (x.y + y.x) / r2);   // (a + i b)/sqrt 2
-                s[0] += nrm(a1);
-                s[1] += nrm(b1);
-                s[2] += x.x * y.x + x.y * y.y;
-                s[3] += x.x * y.y - x.y * y.x;
-                s[4] += nrm(x);
-                s[5] += nrm(y);
+            double2 u, v;
+            other(x, y, u, v);
+            double s[5] = {0, 0, 0, 0, 0};
+            if (l.on) {
+                // (own + i other)/sqrt 2 is the rotated component of both lines
+                const double2 q0 = make_double2(x.x - u.y, x.y + u.x), q1 = make_double2(y.x - v.y, y.y + v.x);
+                const double rot = 0.5 * (nrm(q0) + nrm(q1));
+                s[0] = l.c ? 0.0 : rot;
+                s[1] = l.c ? rot : 0.0;
+                if (!l.c) {
+                    s[2] = x.x * u.x + x.y * u.y + y.x * v.x + y.y * v.y;
+                    s[3] = x.x * u.y - x.y * u.x + y.x * v.y - y.y * v.x;
+                }
+                s[4] = nrm(x) + nrm(y);
             }
-            wave_sum<6>(s);
-            if (threadIdx.x == 0) {
-                double *m = meas + ((long)traj * p.ntW + nn) * 3;
-                m[0] = n * (s[0] * p.dz - 0.5 * V);
-                m[1] = n * (s[1] * p.dz - 0.5 * V);
-                m[2] = 2.0 * sqrt(s[2] * s[2] + s[3] * s[3]) / (s[4] + s[5]);
-            }
+            const double t = block_sums<5>(s, scratch);
+            if (threadIdx.x < 40 && (threadIdx.x & 7) == 0) mt[(long)nn * 5 + (threadIdx.x >> 3)] = t;
         }
     }
-    // mean density after the last step (:396-400)
-    to_x<R, false>(a, b, sa, sb, tw, n);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int k = threadIdx.x + LANES * r;
-        if (k < n) avn[(long)traj * n + k] = nrm(a[r]) - 0.5 * V / p.dz;
+    // mean density after the last step (:396-400), of component a
+    dft_line<-1, H>(l, f, x, y);
+    if (l.c == 0) {
+        if (l.on) avn[(long)traj * n + l.k] = nrm(x) - 0.5 * V / p.dz;
+        if (l.two) avn[(long)traj * n + n - l.k] = nrm(y) - 0.5 * V / p.dz;
+    }
+    __syncthreads();   // the sums are written
+    for (int t = threadIdx.x; t < p.ntW; t += blockDim.x) {
+        double *m = mt + (long)t * 5;
+        const double q[5] = {m[0], m[1], m[2], m[3], m[4]};
+        m[0] = n * (q[0] * p.dz - 0.5 * V);
+        m[1] = n * (q[1] * p.dz - 0.5 * V);
+        m[2] = 2.0 * sqrt(q[2] * q[2] + q[3] * q[3]) / q[4];
     }
 }
 
@@ -331,7 +376,7 @@ __global__ __launch_bounds__(256) void w1d_reduce_kernel(int ne, int ntW, int n,
     if (t < ntW) {
         double s[5] = {0, 0, 0, 0, 0};
         for (int j = 0; j < ne; ++j) {
-            const double *q = meas + ((long)j * ntW + t) * 3;
+            const double *q = meas + ((long)j * ntW + t) * 5;
             s[0] += q[0];
             s[1] += q[1];
             s[2] += q[0] * q[0];
@@ -347,42 +392,46 @@ __global__ __launch_bounds__(256) void w1d_reduce_kernel(int ne, int ntW, int n,
     }
 }
 
-size_t lds_bytes(int n) { return sizeof(double2) * 3 * (size_t)n; }
+// the factor table, then the rows S and D of every component
+size_t lds_bytes(int n, int nc) { return sizeof(double2) * (n + 2 * (size_t)nc * row_len(n)); }
 
-template <int R> hipError_t launch_gs(const W1dParams &p, int n, double2 *gs, double *ntot, double *rep, hipStream_t s)
-{
-    hipLaunchKernelGGL(w1d_ground_state_kernel<R>, dim3(1), dim3(LANES), lds_bytes(n), s, p, n, gs, ntot, rep);
-    return hipGetLastError();
-}
-
-template <int R>
-hipError_t launch_ens(const W1dParams &p, int n, const double2 *gs, double *meas, double *avn, hipStream_t s)
-{
-    const uint32_t k0 = (uint32_t)p.seed, k1 = (uint32_t)(p.seed >> 32);
-    hipLaunchKernelGGL(w1d_ensemble_kernel<R>, dim3((unsigned)p.ne), dim3(LANES), lds_bytes(n), s, p, n, gs, meas, avn,
-                       k0, k1);
-    return hipGetLastError();
-}
+// threads of a workgroup: one per pair and component, whole wavefronts
+int threads_for(int n, int nc) { return (nc * (n / 2 + 1) + 63) / 64 * 64; }
 
 } // namespace
+
+// Lines of h <= 31 run in one wavefront (both components) with their DFT
+// factors in registers, 32 of them per 8 terms; longer ones read the table.
+template <class Fn> static hipError_t with_terms(int n, Fn &&f)
+{
+    const int h = n / 2;
+    if (n > MAXNV) return hipErrorInvalidValue;
+    if (h <= 8) f(std::integral_constant<int, 8>{});
+    else if (h <= 16) f(std::integral_constant<int, 16>{});
+    else if (h <= 24) f(std::integral_constant<int, 24>{});
+    else if (h <= 31) f(std::integral_constant<int, 32>{});
+    else f(std::integral_constant<int, 0>{});
+    return hipGetLastError();
+}
 
 hipError_t run_w1d_ground_state(const W1dParams &p, int n, double2 *gs_out, double *ntot, double *rep_out,
                                 hipStream_t s)
 {
-    if (n <= 64) return launch_gs<1>(p, n, gs_out, ntot, rep_out, s);
-    if (n <= 128) return launch_gs<2>(p, n, gs_out, ntot, rep_out, s);
-    if (n <= 256) return launch_gs<4>(p, n, gs_out, ntot, rep_out, s);
-    if (n <= MAXNV) return launch_gs<8>(p, n, gs_out, ntot, rep_out, s);
-    return hipErrorInvalidValue;
+    return with_terms(n, [&](auto Ht) {
+        constexpr int H = decltype(Ht)::value;
+        hipLaunchKernelGGL(w1d_ground_state_kernel<H>, dim3(1), dim3(threads_for(n, 1)), lds_bytes(n, 1), s, p, n, gs_out,
+                           ntot, rep_out);
+    });
 }
 
 hipError_t run_w1d_ensemble(const W1dParams &p, int n, const double2 *gs, double *meas, double *avn, hipStream_t s)
 {
-    if (n <= 64) return launch_ens<1>(p, n, gs, meas, avn, s);
-    if (n <= 128) return launch_ens<2>(p, n, gs, meas, avn, s);
-    if (n <= 256) return launch_ens<4>(p, n, gs, meas, avn, s);
-    if (n <= MAXNV) return launch_ens<8>(p, n, gs, meas, avn, s);
-    return hipErrorInvalidValue;
+    const uint32_t k0 = (uint32_t)p.seed, k1 = (uint32_t)(p.seed >> 32);
+    return with_terms(n, [&](auto Ht) {
+        constexpr int H = decltype(Ht)::value;
+        hipLaunchKernelGGL(w1d_ensemble_kernel<H>, dim3((unsigned)p.ne), dim3(threads_for(n, 2)), lds_bytes(n, 2), s, p, n,
+                           gs, meas, avn, k0, k1);
+    });
 }
 
 hipError_t run_w1d_reduce(const W1dParams &p, int n, const double *meas, const double *avn, double *sums,

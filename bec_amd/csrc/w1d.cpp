@@ -14,7 +14,7 @@
 namespace {
 
 // the largest samples x trajectories product whose per-trajectory samples
-// (24 B each) are staged on the device
+// (40 B each) are staged on the device
 constexpr long long W1D_MAX_SAMPLES = 1LL << 26;
 
 int cells_1d(const bec_1d_params &p)
@@ -79,7 +79,7 @@ extern "C" int bec_run_1d(const bec_1d_params *pp, double *m, double *var, doubl
     BEC_HIP(buf.alloc((void **)&d_gs, sizeof(double2) * n));
     BEC_HIP(buf.alloc((void **)&d_rep, sizeof(double) * 3));
     BEC_HIP(buf.alloc((void **)&d_ntot, sizeof(double) * p.ntG));
-    BEC_HIP(buf.alloc((void **)&d_meas, sizeof(double) * 3 * (size_t)ne * nt));
+    BEC_HIP(buf.alloc((void **)&d_meas, sizeof(double) * 5 * (size_t)ne * nt));
     BEC_HIP(buf.alloc((void **)&d_avn, sizeof(double) * (size_t)ne * n));
     BEC_HIP(buf.alloc((void **)&d_sums, sizeof(double) * 5 * (size_t)nt));
     BEC_HIP(buf.alloc((void **)&d_avn_sum, sizeof(double) * n));

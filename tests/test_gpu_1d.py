@@ -108,3 +108,19 @@ def test_1d_edge_cases_follow_the_program(bec, oracle):
 def test_1d_rejects_lattices_beyond_one_wavefront(bec):
     with pytest.raises(bec.BecError):
         bec.run_1d(bec.params1d(zmax=64.0, dz=0.25, ne=1))
+
+
+@pytest.mark.parametrize("nv", [1, 3, 41, 61, 63, 65, 67, 127, 129, 511])
+def test_line_lengths_at_the_edges_match_oracle(bec, oracle, nv):
+    """One cell, the rows' remainders mod 4, the longest line whose factors a thread holds in registers
+    (65) and the first that does not (67), one and more wavefronts, the longest lattice; 3 trajectories,
+    12 steps each way, at the bars of the short runs above."""
+    h = nv // 2
+    dz = 20.0 / (h + 0.5) if h else 30.0
+    kw = dict(dz=dz, ne=3, tmaxGP=0.05, tmaxWig=0.11)
+    p = bec.params1d(**kw)
+    assert bec.cells_1d(p) == nv
+    got = bec.run_1d(p)
+    ref = oracle.run1d(oracle.Params1D(**{f: getattr(p, f) for f, _ in oracle.Params1D._fields_}))
+    for key, bar in (("gs", 1e-11), ("ntot", 1e-11), ("m", 1e-9), ("vis", 1e-9), ("avn", 1e-9)):
+        assert _rel(got[key], ref[key]) < bar, key
