@@ -655,6 +655,33 @@ __global__ __launch_bounds__(THREADS) void w2d_ensemble_kernel(W2dParams p, cons
     }
 }
 
+// Sums over trajectories in trajectory order, the products rounded on their own
+// (no contraction), as the program accumulates them: thread t < n_meas sums
+// sample t, the next threads the cells of avn.
+__global__ __launch_bounds__(256) void w2d_reduce_kernel(int ne, int nm, int cells, const double *meas,
+                                                         const double *avn, double *sums, double *avn_sum)
+{
+#pragma clang fp contract(off)
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < nm) {
+        double s[5] = {0, 0, 0, 0, 0};
+        for (int j = 0; j < ne; ++j) {
+            const double *q = meas + ((long)j * nm + t) * 3;
+            s[0] += q[0];
+            s[1] += q[1];
+            s[2] += q[0] * q[0];
+            s[3] += q[1] * q[1];
+            s[4] += q[2];
+        }
+        for (int i = 0; i < 5; ++i) sums[(long)i * nm + t] = s[i];
+    } else if (avn && t < nm + cells) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int j = 0; j < ne; ++j) s += avn[(long)j * cells + t - nm];
+        avn_sum[t - nm] = s;
+    }
+}
+
 // the radices of the first row stage and of the last column stage
 template <class Fn> hipError_t with_radices(const W2dParams &p, Fn &&f)
 {
@@ -690,6 +717,15 @@ hipError_t run_w2d_ensemble(const W2dParams &p, const double2 *gs, double *meas,
         hipLaunchKernelGGL((w2d_ensemble_kernel<RF, RL>), dim3((unsigned)p.ne), dim3(THREADS), 0, s, p, gs, meas, avn,
                            k0, k1);
     });
+}
+
+hipError_t run_w2d_reduce(const W2dParams &p, const double *meas, const double *avn, double *sums, double *avn_sum,
+                          hipStream_t s)
+{
+    const int cells = p.nvx * p.nvy, threads = p.n_meas + (avn ? cells : 0);
+    hipLaunchKernelGGL(w2d_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p.ne, p.n_meas,
+                       cells, meas, avn, sums, avn_sum);
+    return hipGetLastError();
 }
 
 } // namespace bec

@@ -35,18 +35,11 @@ int validate_1d(const bec_1d_params &p, int *nv)
     return BEC_OK;
 }
 
-struct Buffers {
-    std::vector<void *> p;
-    ~Buffers()
-    {
-        for (void *q : p) bec::dev_free(q);
-    }
-    hipError_t alloc(void **q, size_t bytes)
-    {
-        hipError_t e = bec::dev_alloc(q, bytes);
-        if (e == hipSuccess) p.push_back(*q);
-        return e;
-    }
+// The device memory of one call: the results first (one copy back), then the
+// per-trajectory values they are reduced from.
+struct Slab {
+    void *p = nullptr;
+    ~Slab() { bec::dev_free(p); }
 };
 
 } // namespace
@@ -72,17 +65,13 @@ extern "C" int bec_run_1d(const bec_1d_params *pp, double *m, double *var, doubl
         hipStream_t s;
         ~StreamGuard() { (void)hipStreamDestroy(s); }
     } guard{s};
-    Buffers buf;
-    double2 *d_gs = nullptr;
-    double *d_rep = nullptr, *d_ntot = nullptr, *d_meas = nullptr, *d_avn = nullptr, *d_sums = nullptr,
-           *d_avn_sum = nullptr;
-    BEC_HIP(buf.alloc((void **)&d_gs, sizeof(double2) * n));
-    BEC_HIP(buf.alloc((void **)&d_rep, sizeof(double) * 3));
-    BEC_HIP(buf.alloc((void **)&d_ntot, sizeof(double) * p.ntG));
-    BEC_HIP(buf.alloc((void **)&d_meas, sizeof(double) * 5 * (size_t)ne * nt));
-    BEC_HIP(buf.alloc((void **)&d_avn, sizeof(double) * (size_t)ne * n));
-    BEC_HIP(buf.alloc((void **)&d_sums, sizeof(double) * 5 * (size_t)nt));
-    BEC_HIP(buf.alloc((void **)&d_avn_sum, sizeof(double) * n));
+    // doubles: ground state, report, sums over trajectories, N series | samples and densities per trajectory
+    const size_t o_rep = 2 * (size_t)n, o_sums = o_rep + 3, o_avn = o_sums + 5 * (size_t)nt, o_ntot = o_avn + n;
+    const size_t n_res = o_ntot + p.ntG, o_meas = n_res, o_av = o_meas + 5 * (size_t)ne * nt;
+    Slab slab;
+    BEC_HIP(bec::dev_alloc(&slab.p, sizeof(double) * (o_av + (size_t)ne * n)));
+    double *d = (double *)slab.p;
+    double2 *d_gs = (double2 *)d;
     hipEvent_t e0, e1;
     BEC_HIP(hipEventCreate(&e0));
     BEC_HIP(hipEventCreate(&e1));
@@ -95,21 +84,17 @@ extern "C" int bec_run_1d(const bec_1d_params *pp, double *m, double *var, doubl
         }
     } eg{e0, e1};
     BEC_HIP(hipEventRecord(e0, s));
-    BEC_HIP(bec::run_w1d_ground_state(p, n, d_gs, d_ntot, d_rep, s));
-    BEC_HIP(bec::run_w1d_ensemble(p, n, d_gs, d_meas, d_avn, s));
-    BEC_HIP(bec::run_w1d_reduce(p, n, d_meas, d_avn, d_sums, d_avn_sum, s));
+    BEC_HIP(bec::run_w1d_ground_state(p, n, d_gs, d + o_ntot, d + o_rep, s));
+    BEC_HIP(bec::run_w1d_ensemble(p, n, d_gs, d + o_meas, d + o_av, s));
+    BEC_HIP(bec::run_w1d_reduce(p, n, d + o_meas, d + o_av, d + o_sums, d + o_avn, s));
     BEC_HIP(hipEventRecord(e1, s));
-    std::vector<double> h_rep(3), h_sums(5 * (size_t)nt), h_avn(n), h_ntot(p.ntG);
-    std::vector<double2> h_gs(n);
-    BEC_HIP(hipMemcpyAsync(h_rep.data(), d_rep, sizeof(double) * 3, hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_sums.data(), d_sums, sizeof(double) * h_sums.size(), hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_avn.data(), d_avn_sum, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_ntot.data(), d_ntot, sizeof(double) * p.ntG, hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_gs.data(), d_gs, sizeof(double2) * n, hipMemcpyDeviceToHost, s));
+    std::vector<double> res(n_res);
+    BEC_HIP(hipMemcpyAsync(res.data(), d, sizeof(double) * n_res, hipMemcpyDeviceToHost, s));
     BEC_HIP(hipStreamSynchronize(s));
     float ms = 0.0f;
     (void)hipEventElapsedTime(&ms, e0, e1);
 
+    const double *h_rep = &res[o_rep], *h_sums = &res[o_sums], *h_avn = &res[o_avn], *h_ntot = &res[o_ntot];
     // wigner_1d.cpp:405-413 as written: means, then sqrt((<N^2> - <N>^2) / (ne - 1))
     for (int i = 0; i < 2 * nt; ++i) {
         m[i] = h_sums[i] / ne;
@@ -123,10 +108,7 @@ extern "C" int bec_run_1d(const bec_1d_params *pp, double *m, double *var, doubl
     if (ntot)
         for (int i = 0; i < p.ntG; ++i) ntot[i] = h_ntot[i];
     if (gs_x)
-        for (int c = 0; c < n; ++c) {
-            gs_x[2 * c] = h_gs[c].x;
-            gs_x[2 * c + 1] = h_gs[c].y;
-        }
+        for (int i = 0; i < 2 * n; ++i) gs_x[i] = res[i];
     if (rep) {
         rep->N0 = h_rep[0];
         rep->nv = n;

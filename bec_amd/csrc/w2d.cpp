@@ -27,18 +27,11 @@ int validate_2d(const bec_2d_params &p)
     return BEC_OK;
 }
 
-struct Buffers {
-    std::vector<void *> p;
-    ~Buffers()
-    {
-        for (void *q : p) bec::dev_free(q);
-    }
-    hipError_t alloc(void **q, size_t bytes)
-    {
-        hipError_t e = bec::dev_alloc(q, bytes);
-        if (e == hipSuccess) p.push_back(*q);
-        return e;
-    }
+// The device memory of one call: the results first (one copy back), then the
+// per-trajectory values they are reduced from.
+struct Slab {
+    void *p = nullptr;
+    ~Slab() { bec::dev_free(p); }
 };
 
 } // namespace
@@ -57,13 +50,14 @@ extern "C" int bec_run_2d(const bec_2d_params *pp, double *m, double *var, doubl
         hipStream_t s;
         ~StreamGuard() { (void)hipStreamDestroy(s); }
     } guard{s};
-    Buffers buf;
-    double2 *d_gs = nullptr;
-    double *d_rep = nullptr, *d_meas = nullptr, *d_avn = nullptr;
-    BEC_HIP(buf.alloc((void **)&d_gs, sizeof(double2) * cells));
-    BEC_HIP(buf.alloc((void **)&d_rep, sizeof(double) * 4));
-    BEC_HIP(buf.alloc((void **)&d_meas, sizeof(double) * 3 * p.ne * p.n_meas));
-    if (avn) BEC_HIP(buf.alloc((void **)&d_avn, sizeof(double) * cells * p.ne));
+    const int nm = p.n_meas, ne = p.ne;
+    // doubles: ground state, report, sums over trajectories | samples and densities per trajectory
+    const size_t o_rep = 2 * (size_t)cells, o_sums = o_rep + 4, o_avn = o_sums + 5 * (size_t)nm;
+    const size_t n_res = o_avn + (avn ? cells : 0), o_meas = n_res, o_av = o_meas + 3 * (size_t)ne * nm;
+    Slab slab;
+    BEC_HIP(bec::dev_alloc(&slab.p, sizeof(double) * (o_av + (avn ? (size_t)ne * cells : 0))));
+    double *d = (double *)slab.p, *d_av = avn ? d + o_av : nullptr;
+    double2 *d_gs = (double2 *)d;
     hipEvent_t e0, e1;
     BEC_HIP(hipEventCreate(&e0));
     BEC_HIP(hipEventCreate(&e1));
@@ -76,51 +70,29 @@ extern "C" int bec_run_2d(const bec_2d_params *pp, double *m, double *var, doubl
         }
     } eg{e0, e1};
     BEC_HIP(hipEventRecord(e0, s));
-    BEC_HIP(bec::run_w2d_ground_state(p, d_gs, d_rep, s));
-    BEC_HIP(bec::run_w2d_ensemble(p, d_gs, d_meas, d_avn, s));
+    BEC_HIP(bec::run_w2d_ground_state(p, d_gs, d + o_rep, s));
+    BEC_HIP(bec::run_w2d_ensemble(p, d_gs, d + o_meas, d_av, s));
+    BEC_HIP(bec::run_w2d_reduce(p, d + o_meas, d_av, d + o_sums, d + o_avn, s));
     BEC_HIP(hipEventRecord(e1, s));
-    std::vector<double> h_rep(4), h_meas(3 * (size_t)p.ne * p.n_meas), h_avn(avn ? cells * p.ne : 0);
-    std::vector<double2> h_gs(cells);
-    BEC_HIP(hipMemcpyAsync(h_rep.data(), d_rep, sizeof(double) * 4, hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_meas.data(), d_meas, sizeof(double) * h_meas.size(), hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipMemcpyAsync(h_gs.data(), d_gs, sizeof(double2) * cells, hipMemcpyDeviceToHost, s));
-    if (avn) BEC_HIP(hipMemcpyAsync(h_avn.data(), d_avn, sizeof(double) * h_avn.size(), hipMemcpyDeviceToHost, s));
+    std::vector<double> res(n_res);
+    BEC_HIP(hipMemcpyAsync(res.data(), d, sizeof(double) * n_res, hipMemcpyDeviceToHost, s));
     BEC_HIP(hipStreamSynchronize(s));
     float ms = 0.0f;
     (void)hipEventElapsedTime(&ms, e0, e1);
 
+    const double *h_rep = &res[o_rep], *h_sums = &res[o_sums];
     // ensemble statistics (wigner.cpp:431-443): means, then sqrt(|<N^2> - <N>^2| / (ne - 1))
-    const int nm = p.n_meas, ne = p.ne;
-    for (int i = 0; i < 2 * nm; ++i) m[i] = var[i] = 0.0;
-    if (vis)
-        for (int i = 0; i < nm; ++i) vis[i] = 0.0;
-    for (int j = 0; j < ne; ++j)
-        for (int k = 0; k < nm; ++k) {
-            const double *q = &h_meas[((size_t)j * nm + k) * 3];
-            m[k] += q[0];
-            m[k + nm] += q[1];
-            var[k] += q[0] * q[0];
-            var[k + nm] += q[1] * q[1];
-            if (vis) vis[k] += q[2];
-        }
     for (int i = 0; i < 2 * nm; ++i) {
-        m[i] /= ne;
-        const double v = var[i] / ne - m[i] * m[i];
+        m[i] = h_sums[i] / ne;
+        const double v = h_sums[2 * (size_t)nm + i] / ne - m[i] * m[i];
         var[i] = ne > 1 ? sqrt(fabs(v) / (ne - 1)) : 0.0;
     }
     if (vis)
-        for (int i = 0; i < nm; ++i) vis[i] /= ne;
+        for (int i = 0; i < nm; ++i) vis[i] = h_sums[4 * (size_t)nm + i] / ne;
     if (avn)
-        for (long c = 0; c < cells; ++c) {
-            double t = 0.0;
-            for (int j = 0; j < ne; ++j) t += h_avn[(size_t)j * cells + c];
-            avn[c] = t / ne;
-        }
+        for (long c = 0; c < cells; ++c) avn[c] = res[o_avn + c] / ne;
     if (gs_x)
-        for (long c = 0; c < cells; ++c) {
-            gs_x[2 * c] = h_gs[c].x;
-            gs_x[2 * c + 1] = h_gs[c].y;
-        }
+        for (long i = 0; i < 2 * cells; ++i) gs_x[i] = res[i];
     if (rep) {
         rep->N0 = h_rep[0];
         rep->gs_iterations = (int)h_rep[1];
