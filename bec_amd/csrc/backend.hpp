@@ -77,13 +77,11 @@ hipError_t run_noise_init(const DevGroup &g, const void *gs, uint64_t seed, doub
 hipError_t run_pulse(const DevGroup &g, int kind, hipStream_t s);
 // (a, b) <- U (a, b) on every cell; u = {u00, u01, u10, u11} as (re, im) pairs
 hipError_t run_rotation(const DevGroup &g, const double u[8], hipStream_t s);
-// per-cell ensemble sums of vacuum-subtracted densities after halfPiRotate(alpha):
-// out[cell*2 + c], x-space
-hipError_t run_cell_density_sums(const DevGroup &g, double alpha, double vac, double *out,
-                                 hipStream_t s);
-// doubles of the projection workspace of a group: the per-cell sums [cells][2],
-// then xy [2][ny][nx], zy [2][ny][nz], axial [2][nz]
+// doubles of the projection workspace of a group: the results, then the partial
+// sums; it fits the fixed workspace of bec_projections_static for any ntraj
 long projection_doubles(const DevGroup &g);
+// doubles of the results: xy [2][ny][nx], zy [2][ny][nz], axial [2][nz]
+long projection_results(const DevGroup &g);
 // the density projections after halfPiRotate(alpha) into buf (projection_doubles(g) doubles)
 hipError_t run_projections(const DevGroup &g, double alpha, double vac, double *buf, hipStream_t s);
 // plain streaming copy (HBM counter calibration)

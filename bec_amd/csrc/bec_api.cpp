@@ -1037,14 +1037,15 @@ int ctx_projections(bec_ctx *ctx, int group, double alpha, double *buf, size_t c
     const long nx = g.calc.nvx, ny = g.calc.nvy, nz = g.calc.nvz;
     const double vac = g.calc.V / (2.0 * g.calc.dx * g.calc.dy * g.calc.dz);
     BEC_HIP(run_projections(g.dev, alpha, vac, buf, ctx->stream));
-    const double *xy = buf + 2 * g.cells, *zy = xy + 2 * nx * ny, *ax = zy + 2 * ny * nz;
-    double *dst[6] = {xy_a, xy_b, zy_a, zy_b, axial_a, axial_b};
-    const double *src[6] = {xy, xy + nx * ny, zy, zy + ny * nz, ax, ax + nz};
-    const long len[6] = {nx * ny, nx * ny, ny * nz, ny * nz, nz, nz};
-    for (int i = 0; i < 6; ++i)
-        if (dst[i])
-            BEC_HIP(hipMemcpyAsync(dst[i], src[i], sizeof(double) * len[i], hipMemcpyDeviceToHost, ctx->stream));
+    // one copy of all results, then the caller's arrays
+    std::vector<double> res(projection_results(g.dev));
+    BEC_HIP(hipMemcpyAsync(res.data(), buf, sizeof(double) * res.size(), hipMemcpyDeviceToHost, ctx->stream));
     BEC_HIP(hipStreamSynchronize(ctx->stream));
+    double *dst[6] = {xy_a, xy_b, zy_a, zy_b, axial_a, axial_b};
+    const long len[6] = {nx * ny, nx * ny, ny * nz, ny * nz, nz, nz};
+    const double *src = res.data();
+    for (int i = 0; i < 6; src += len[i], ++i)
+        if (dst[i]) memcpy(dst[i], src, sizeof(double) * len[i]);
     return BEC_OK;
 }
 } // namespace bec

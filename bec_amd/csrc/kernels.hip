@@ -420,112 +420,6 @@ hipError_t run_pulse(const DevGroup &g, int kind, hipStream_t s)
     return hipGetLastError();
 }
 
-// ----------------------------------------------------- density projections
-// Each workgroup owns 64/N planes at fixed z and loops over the trajectories,
-// accumulating the vacuum-subtracted densities after halfPiRotate(alpha)
-// (wigner_kernel.cu:283-286,344-360) in FP64; deterministic order.
-template <typename T, int N>
-__global__ void __launch_bounds__(64) cell_sums_kernel(const cpx<T> *__restrict__ a, const cpx<T> *__restrict__ b,
-                                                       int nz, int ntraj, double ca, double sa, double vac,
-                                                       double *__restrict__ out)
-{
-    constexpr int PPW = 64 / N;
-    __shared__ cpx<T> lds[PPW * N * (N + 1)];
-    const int lane = threadIdx.x, pl = lane / N, t = lane % N;
-    const int z = blockIdx.x * PPW + pl;
-    cpx<T> *tile = lds + pl * N * (N + 1);
-    const double r = 0.70710678118654752440;
-    double acc[2][N];
-#pragma unroll
-    for (int x = 0; x < N; ++x) acc[0][x] = acc[1][x] = 0.0;
-    for (int traj = 0; traj < ntraj; ++traj) {
-        const long base = ((long)traj * nz + z) * (N * N);
-        cpx<T> v[2][N];
-#pragma unroll
-        for (int y = 0; y < N; ++y) {
-            v[0][y] = a[base + y * N + t];
-            v[1][y] = b[base + y * N + t];
-        }
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            dft<T, N, -1>(v[c]);
-            col2row<T, N>(tile, t, v[c]);
-            dft<T, N, -1>(v[c]);
-        }
-#pragma unroll
-        for (int x = 0; x < N; ++x) {
-            const double ar = v[0][x].x, ai = v[0][x].y, br = v[1][x].x, bi = v[1][x].y;
-            // a' = (a + b (sin - i cos))/sqrt2, b' = (a (-sin - i cos) + b)/sqrt2
-            const double anr = (ar + br * sa + bi * ca) * r, ani = (ai + bi * sa - br * ca) * r;
-            const double bnr = (-ar * sa + ai * ca + br) * r, bni = (-ai * sa - ar * ca + bi) * r;
-            acc[0][x] += anr * anr + ani * ani - vac;
-            acc[1][x] += bnr * bnr + bni * bni - vac;
-        }
-    }
-#pragma unroll
-    for (int x = 0; x < N; ++x) {
-        const long cell = ((long)z * N + t) * N + x;
-        out[cell * 2] = acc[0][x];
-        out[cell * 2 + 1] = acc[1][x];
-    }
-}
-
-hipError_t run_cell_density_sums(const DevGroup &g, double alpha, double vac, double *out, hipStream_t s)
-{
-    double ca = cos(alpha), sa = sin(alpha);
-    return dispatch(g, [&](auto Tt, auto Nt, auto) -> hipError_t {
-        using T = typename decltype(Tt)::type;
-        constexpr int N = decltype(Nt)::value;
-        constexpr int PPW = 64 / N;
-        if (g.nz % PPW) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((cell_sums_kernel<T, N>), dim3(g.nz / PPW), dim3(64), 0, s, (const cpx<T> *)g.a,
-                           (const cpx<T> *)g.b, g.nz, g.ntraj, ca, sa, vac, out);
-        return hipGetLastError();
-    });
-}
-
-// Projections of the per-cell sums cs[cell*2 + c] (run_cell_density_sums):
-// out = {xy[2][ny][nx] (sum over z), zy[2][ny][nz] (sum over x),
-// axial[2][nz] (sum over y, then x)}, one thread per output value, each sum in
-// increasing index order (wigner.cu:279-303,388-410).
-__global__ void __launch_bounds__(256) projection_sums_kernel(const double *__restrict__ cs, int nx, int ny, int nz,
-                                                             double *__restrict__ out)
-{
-    const int nxy = nx * ny, nyz = ny * nz;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int n_out = 2 * (nxy + nyz + nz);
-    if (i >= n_out) return;
-    double s = 0.0;
-    if (i < 2 * nxy) {
-        const int c = i / nxy, q = i - c * nxy;   // q = y nx + x
-        for (int z = 0; z < nz; ++z) s += cs[((long)z * nxy + q) * 2 + c];
-    } else if (i < 2 * (nxy + nyz)) {
-        const int r = i - 2 * nxy, c = r / nyz, q = r - c * nyz, y = q / nz, z = q - y * nz;
-        for (int x = 0; x < nx; ++x) s += cs[(((long)z * ny + y) * nx + x) * 2 + c];
-    } else {
-        const int r = i - 2 * (nxy + nyz), c = r / nz, z = r - c * nz;
-        for (int q = 0; q < nxy; ++q) s += cs[((long)z * nxy + q) * 2 + c];
-    }
-    out[i] = s;
-}
-
-long projection_doubles(const DevGroup &g)
-{
-    const long cells = (long)g.nx * g.ny * g.nz;
-    return 2 * cells + 2 * ((long)g.nx * g.ny + (long)g.ny * g.nz + g.nz);
-}
-
-hipError_t run_projections(const DevGroup &g, double alpha, double vac, double *buf, hipStream_t s)
-{
-    hipError_t e = run_cell_density_sums(g, alpha, vac, buf, s);
-    if (e != hipSuccess) return e;
-    const long cells = (long)g.nx * g.ny * g.nz;
-    const int n_out = (int)(projection_doubles(g) - 2 * cells);
-    hipLaunchKernelGGL(projection_sums_kernel, dim3((n_out + 255) / 256), dim3(256), 0, s, buf, g.nx, g.ny, g.nz,
-                       buf + 2 * cells);
-    return hipGetLastError();
-}
-
 // ------------------------------------------------------------------- copy
 // A streaming copy for the achievable-bandwidth reference: one 16-byte
 // non-temporal load and store per thread over a grid that covers the buffer.

@@ -20,8 +20,8 @@ namespace bec {
 int ctx_projections(bec_ctx *ctx, int group, double alpha, double *buf, size_t cap, double *xy_a, double *xy_b,
                     double *zy_a, double *zy_b, double *axial_a, double *axial_b);
 
-// 4.25 MiB: the largest projection workspace of a supported lattice
-// (256 x 32 x 32: 2 x 262,144 cell sums + 18,944 projection values) with room
+// 4.25 MiB: the largest projection workspace (partial sums of at most 4 MiB, and
+// the 18,944 projection values of 256 x 32 x 32) with room
 static constexpr size_t SCRATCH_DOUBLES = 557056;
 static constexpr int MAX_DEVICES = 64;
 

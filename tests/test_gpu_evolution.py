@@ -321,3 +321,27 @@ def test_pulse_rotation_matches_oracle(bec, oracle, gs, prec, tol):
     ra, rb = oracle.rotation(a0, b0, 1.3, -0.8)
     assert rel_l2(a1, ra) < tol and rel_l2(b1, rb) < tol
     assert rel_l2(a2, a3) < tol and rel_l2(b2, b3) < tol
+
+
+@pytest.mark.parametrize("prec,nxy,nz,ne", [(0, 16, 64, 5), (0, 16, 128, 70), (0, 32, 256, 7), (0, 32, 64, 1),
+                                            (1, 16, 256, 3), (1, 32, 128, 13)])
+def test_projections_of_every_split_equal_the_states_sums(bec, prec, nxy, nz, ne):
+    """Projections whose trajectories are split over workgroups (one each, several each with a shorter
+    last share, a single trajectory) against FP64 sums of the x-space states."""
+    alpha = 0.7
+    c = gpu_calc(bec, **config1_model(bec, N=30000, nvx=nxy, nvy=nxy, nvz=nz, ne=ne, dt_evo=2e-5))
+    x = [np.arange(n) - n / 2 for n in (nz, nxy, nxy)]
+    psi = 6.0 * np.exp(-(x[2] / 4.0) ** 2 - (x[1][:, None] / 4.0) ** 2 - (x[0][:, None, None] / (nz / 5.0)) ** 2)
+    with bec.Solver(c, precision=prec) as s:
+        s.init_evolution(psi, 9)
+        s.propagate(2)
+        a, b = s.get_state(bec.SPACE_X)
+        p = s.projections(alpha=alpha)
+    w = np.sin(alpha) - 1j * np.cos(alpha)
+    vac = 1.0 / (2.0 * c.dx * c.dy * c.dz)
+    da = (np.abs(a + b * w) ** 2 / 2 - vac).sum(axis=0)
+    db = (np.abs(-a * np.conj(w) + b) ** 2 / 2 - vac).sum(axis=0)
+    for k, d in (("a", da), ("b", db)):
+        assert rel_l2(p["xy_" + k], d.sum(axis=0)) < 1e-9
+        assert rel_l2(p["zy_" + k], d.sum(axis=2).T) < 1e-9
+        assert rel_l2(p["axial_" + k], d.sum(axis=(1, 2))) < 1e-9
