@@ -126,14 +126,6 @@ template <typename T> __device__ __forceinline__ T potential_t(const TrajParams 
     return (T)0.5 * (xx * xx + yy * yy + zz * zz * (T)p.inv_lambda2);
 }
 
-// Wave-wide sum over a group of G consecutive lanes (G a power of two <= 64).
-template <int G> __device__ __forceinline__ double group_sum(double v)
-{
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // ------------------------------------------------------ wave-wide sums
 // Sums across the 64 lanes through the vector unit's own lane moves (DPP within
 // rows of 16 lanes, permlane swaps between rows and halves) instead of LDS

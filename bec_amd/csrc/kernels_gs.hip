@@ -25,7 +25,7 @@ __device__ __forceinline__ double psum(const double *partial, int per, int nsum,
     const double *p = partial + (long)traj * per * nsum + k;
     double s = 0.0;
     for (int j = (int)(threadIdx.x & 63); j < per; j += 64) s += p[(long)j * nsum];
-    return group_sum<64>(s);
+    return wave_sum(s);
 }
 
 // --------------------------------------------------------------- z-passes

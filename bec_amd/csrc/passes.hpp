@@ -175,10 +175,12 @@ __device__ __forceinline__ void xy_tile(const Op &op_, const XyGeom &g, double *
     op.apply(v, t, z, traj, base + (long)t * N, sums);
 
     if constexpr (Op::NSUM > 0) {
-#pragma unroll
-        for (int i = 0; i < Op::NSUM; ++i) {
-            double s = group_sum<64>(sums[i]);
-            if (lane == 0) partial[blk * Op::NSUM + i] = s;
+        if constexpr (Op::NSUM == 1) {
+            const double s = wave_sum(sums[0]);
+            if (lane == 0) partial[blk] = s;
+        } else {
+            const double s = wave_sums<Op::NSUM>(sums);
+            if ((lane & 7) == 0 && lane / 8 < Op::NSUM) partial[blk * Op::NSUM + lane / 8] = s;
         }
     }
 
