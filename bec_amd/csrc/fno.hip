@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/bec_fno.h"
+#include "fno_kernels.hpp"
 #include "host_common.hpp"
 
 namespace bec {
@@ -30,7 +31,7 @@ hipError_t run_gemm(const bec_gemm_desc &g, hipStream_t s);
 
 namespace {
 
-constexpr int KSPLIT = 256;
+constexpr int KSPLIT = WGRAD_SPLITS;
 
 bec_map2 m1(long stride)
 {
@@ -403,22 +404,27 @@ hipError_t rowgemm_bt(const bec_fno *f, const float *A, const float *Bt, float *
              nullptr, 1, nullptr, s);
 }
 
-// dWt[k][n] = sum_rows X[rows][k] D[rows][n]  (weight gradient, split K)
-hipError_t wgrad(const bec_fno *f, const float *X, int K, const float *D, int N, long rows, float *out,
-                 hipStream_t s)
+// dW[k][n] = sum_rows X[rows][k] D[rows][n] and, behind it, db[n] = sum_rows
+// D[rows][n] (a layer's weights and biases are adjacent in the parameters): the
+// fused kernel, or for the shapes it does not cover split-K GEMMs, the bias as
+// one against a constant-one A operand (stride 0)
+hipError_t layer_grad(const bec_fno *f, const float *X, int K, const float *D, int N, long rows, float *out,
+                      hipStream_t s)
 {
-    float *work = f->work;
-    return G(f, X, 0, D, 0, out, K, N, (int)rows, m1(1), m1(K), m1(N), m1(1), m1(N), m1(1), 1, m1(0), m1(0), m1(0), 0.0f,
-             nullptr, KSPLIT, work, s);
-}
-
-// db[n] = sum_rows D[rows][n]: a GEMM with a constant-one A operand (stride 0)
-hipError_t bgrad(const bec_fno *f, const float *D, int N, long rows, float *out, hipStream_t s)
-{
-    const float *one = f->one;
-    float *work = f->work;
-    return G(f, one, 0, D, 0, out, 1, N, (int)rows, m1(0), m1(0), m1(N), m1(1), m1(N), m1(1), 1, m1(0), m1(0), m1(0),
-             0.0f, nullptr, KSPLIT, work, s);
+    if (wgrad_covers(K, N, rows)) {
+        const long total = (long)K * N + N;
+        if (rows * K > room(f, X, 4) || rows * N > room(f, D, 4) || total > room(f, out, 4) ||
+            WGRAD_SPLITS * total > room(f, f->work, 4)) {
+            set_last_error("surrogate weight gradient exceeds its buffers");
+            return hipErrorInvalidValue;
+        }
+        return run_wgrad(X, K, D, N, rows, f->work, out, s);
+    }
+    hipError_t e = G(f, X, 0, D, 0, out, K, N, (int)rows, m1(1), m1(K), m1(N), m1(1), m1(N), m1(1), 1, m1(0), m1(0),
+                     m1(0), 0.0f, nullptr, KSPLIT, f->work, s);
+    if (e != hipSuccess) return e;
+    return G(f, f->one, 0, D, 0, out + (long)K * N, 1, N, (int)rows, m1(0), m1(0), m1(N), m1(1), m1(N), m1(1), 1, m1(0),
+             m1(0), m1(0), 0.0f, nullptr, KSPLIT, f->work, s);
 }
 
 struct Spec {
@@ -531,14 +537,12 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
     float *g = f->grads;
     hipError_t e;
     // projection: y = a1 Q2 + q2, a1 = gelu(g1), g1 = hL Q1 + q1
-    if ((e = wgrad(f, f->a1, H, f->dy, c.c_out, rows, g + f->oQ2, s)) != hipSuccess) return e;
-    if ((e = bgrad(f, f->dy, c.c_out, rows, g + f->oq2, s)) != hipSuccess) return e;
+    if ((e = layer_grad(f, f->a1, H, f->dy, c.c_out, rows, g + f->oQ2, s)) != hipSuccess) return e;
     float *da1 = f->dB;   // [rows][H]
     if ((e = rowgemm_bt(f, f->dy, f->params + f->oQ2, da1, rows, c.c_out, H, 0.0f, s)) != hipSuccess) return e;
     hipLaunchKernelGGL(gelu_bwd, grid1(rows * H), dim3(256), 0, s, f->g1, da1, rows * H);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = wgrad(f, f->h[L], W, da1, H, rows, g + f->oQ1, s)) != hipSuccess) return e;
-    if ((e = bgrad(f, da1, H, rows, g + f->oq1, s)) != hipSuccess) return e;
+    if ((e = layer_grad(f, f->h[L], W, da1, H, rows, g + f->oQ1, s)) != hipSuccess) return e;
     float *dh = f->dA;    // gradient w.r.t. the current layer output
     if ((e = rowgemm_bt(f, da1, f->params + f->oQ1, dh, rows, H, W, 0.0f, s)) != hipSuccess) return e;
     for (int l = L - 1; l >= 0; --l) {
@@ -548,8 +552,7 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         const float *hin = f->h[l];
-        if ((e = wgrad(f, hin, W, du, W, rows, g + f->oW[l], s)) != hipSuccess) return e;
-        if ((e = bgrad(f, du, W, rows, g + f->ob[l], s)) != hipSuccess) return e;
+        if ((e = layer_grad(f, hin, W, du, W, rows, g + f->oW[l], s)) != hipSuccess) return e;
         float *dhin = (dh == f->dA) ? f->dH : f->dA;
         if ((e = rowgemm_bt(f, du, f->params + f->oW[l], dhin, rows, W, W, 0.0f, s)) != hipSuccess) return e;
         // spectral path, adjoint order
@@ -571,8 +574,7 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
         dh = dhin;
     }
     // lift
-    if ((e = wgrad(f, x, c.c_in, dh, W, rows, g + f->oP, s)) != hipSuccess) return e;
-    return bgrad(f, dh, W, rows, g + f->op, s);
+    return layer_grad(f, x, c.c_in, dh, W, rows, g + f->oP, s);
 }
 
 int validate(const bec_fno_config &c)
@@ -689,7 +691,8 @@ int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
     FA(f->dB, fb * rows * c.hidden);
     FA(f->dE, fb * f->modes * 4 * W * W);
     long mn = std::max(std::max((long)c.c_in * W, W * W), std::max(W * (long)c.hidden, (long)c.hidden * c.c_out));
-    // split-K partials: the weight gradients (KSPLIT layers of at most mn) and the
+    mn += std::max({W, (long)c.hidden, (long)c.c_out});   // weights and biases of a layer
+    // split-K partials: the weight gradients (KSPLIT of at most mn) and the
     // small-batch splits of G (at most 8 layers of < 256 64 x 64 tiles)
     FA(f->work, fb * std::max((long)KSPLIT * mn, 8L * 256 * 64 * 64));
     FA(f->loss_part, sizeof(double) * ((rows * c.c_out + 255) / 256));
