@@ -225,6 +225,15 @@ __global__ void adam_kernel(float *p, const float *g, float *m, float *v, long n
     p[i] -= lr * (mh / (sqrtf(vh) + eps) + wd * p[i]);
 }
 
+// FP32 -> BF16, nearest even (finite values)
+unsigned short host_bf16(float f)
+{
+    unsigned int u;
+    memcpy(&u, &f, sizeof(u));
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (unsigned short)(u >> 16);
+}
+
 dim3 grid1(long n) { return dim3((unsigned)((n + 255) / 256)); }
 
 // splitmix64 -> uniform (-1, 1)
@@ -252,6 +261,7 @@ struct bec_fno {
     float *params = nullptr, *grads = nullptr, *adam_m = nullptr, *adam_v = nullptr;
     unsigned short *E = nullptr;      // [layers][modes][2W][2W] BF16
     float *Fz = nullptr, *Fxy = nullptr, *one = nullptr;
+    unsigned short *FxyB = nullptr, *FxyTB = nullptr;    // Fxy and its transpose as BF16 MFMA operands
     // activations
     std::vector<float *> h, u;        // h[0..L], u[0..L-1] (u[L-1] aliases h[L])
     float *zf = nullptr, *tm = nullptr, *zi = nullptr;   // spectral temporaries
@@ -340,6 +350,21 @@ long max_off(const bec_map2 &m, long n)
     return best;
 }
 
+// The K split of a GEMM that fills few workgroups (see G): 1 when it is not split.
+int small_split(int M, int N, int K, int batch)
+{
+    const long wgs = ((long)(N + 63) / 64) * ((M + 63) / 64) * batch;
+    if (wgs >= 256 || K < 128) return 1;
+    return (int)std::min<long>(std::min<long>(8, (1024 + wgs - 1) / wgs), K / 64);
+}
+
+// 32-value K tiles of each part of that split (0: not split)
+int split_tiles(int M, int N, int K, int batch)
+{
+    const int ks = small_split(M, N, K, batch);
+    return ks > 1 ? ((K + 31) / 32 + ks - 1) / ks : 0;
+}
+
 // One GEMM with the network's conventions.  Before the launch, the largest
 // offset each operand map reaches is checked on the host against the buffer
 // that holds the operand (every device buffer the network touches is
@@ -355,9 +380,8 @@ hipError_t G(const bec_fno *f, const void *A, int abf, const void *B, int bbf, f
     // single-sample forward pass) walks its K tiles in one dependent chain
     // per workgroup; split K to about 1024 workgroups (4 per CU; 512 left the
     // single-sample pass at 0.57 ms against 0.49), reduced in a fixed order.
-    const long wgs = ((long)(N + 63) / 64) * ((M + 63) / 64) * batch;
-    if (ksplit == 1 && wgs < 256 && K >= 128) {
-        ksplit = (int)std::min<long>(std::min<long>(8, (1024 + wgs - 1) / wgs), K / 64);
+    if (ksplit == 1 && small_split(M, N, K, batch) > 1) {
+        ksplit = small_split(M, N, K, batch);
         work = f->work;
     }
     bool ok = ea < room(f, A, abf ? 2 : 4) && eb < room(f, B, bbf ? 2 : 4) && ec < room(f, C, 4);
@@ -448,8 +472,17 @@ hipError_t xydft(const bec_fno *f, const Spec &q, const float *in, float *out, i
     const long rows_in = transpose ? 2 * q.mxy : 2 * q.P, rows_out = transpose ? 2 * q.P : 2 * q.mxy;
     const long lda = 2 * q.P;   // Fxy is [2 mxy][2 P]
     bec_map2 am = transpose ? m1(1) : m1(lda), ak = transpose ? m1(lda) : m1(1);
+    const int planes = q.B * (q.mz2 / 2);
+    if (plane_dft_covers((int)rows_out, (int)rows_in, q.W) && plane_dft_covers((int)rows_in, (int)rows_out, q.W)) {
+        if (planes * rows_in * q.W > room(f, in, 4) || planes * rows_out * q.W > room(f, out, 4)) {
+            set_last_error("surrogate plane transform exceeds its buffers");
+            return hipErrorInvalidValue;
+        }
+        return run_plane_dft(transpose ? f->FxyTB : f->FxyB, in, out, (int)rows_out, (int)rows_in, q.W, planes,
+                             split_tiles((int)rows_out, q.W, (int)rows_in, planes), s);
+    }
     return G(f, f->Fxy, 0, in, 0, out, (int)rows_out, q.W, (int)rows_in, am, ak, m1(q.W), m1(1), m1(q.W), m1(1),
-             q.B * (q.mz2 / 2), m1(0), m1(rows_in * q.W), m1(rows_out * q.W), 0.0f, nullptr, 1, nullptr, s);
+             planes, m1(0), m1(rows_in * q.W), m1(rows_out * q.W), 0.0f, nullptr, 1, nullptr, s);
 }
 
 // per-mode maps of the [b][kz][re/im][kxy][W] spectral layout
@@ -623,7 +656,14 @@ hipError_t build_tables(bec_fno *f)
                     fxy[(size_t)(mxy + r) * 2 * P + P + q] = cs;  // im <- im
                 }
         }
-    hipError_t e = hipMemcpy(f->Fz, fz.data(), fz.size() * sizeof(float), hipMemcpyHostToDevice);
+    std::vector<unsigned short> fb(fxy.size()), ft(fxy.size());
+    if (plane_dft_covers((int)(2 * mxy), (int)(2 * P), c.width) && plane_dft_covers((int)(2 * P), (int)(2 * mxy), c.width))
+        for (long r = 0; r < 2 * mxy; ++r)
+            for (long k = 0; k < 2 * P; ++k)
+                fb[operand_at(r, k, 2 * P)] = ft[operand_at(k, r, 2 * mxy)] = host_bf16(fxy[r * 2 * P + k]);
+    hipError_t e = hipMemcpy(f->FxyB, fb.data(), fb.size() * 2, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->FxyTB, ft.data(), ft.size() * 2, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->Fz, fz.data(), fz.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(f->Fxy, fxy.data(), fxy.size() * sizeof(float), hipMemcpyHostToDevice);
     return e;
 }
@@ -671,6 +711,8 @@ int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
     FA(f->E, sizeof(unsigned short) * L * f->modes * 4 * W * W);
     FA(f->Fz, fb * 2 * c.mz * c.nz);
     FA(f->Fxy, fb * 4 * f->mxy * f->P);
+    FA(f->FxyB, sizeof(unsigned short) * 4 * f->mxy * f->P);
+    FA(f->FxyTB, sizeof(unsigned short) * 4 * f->mxy * f->P);
     FA(f->one, fb);
     f->h.assign(L + 1, nullptr);
     f->u.assign(L, nullptr);

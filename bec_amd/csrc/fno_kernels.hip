@@ -127,6 +127,95 @@ __global__ __launch_bounds__(64) void sum_partials(const float *__restrict__ par
     out[i] = s;
 }
 
+// The 2D transforms of all retained kz planes: out[b] = A in[b] with the plane's
+// DFT matrix A (M x K, BF16, stored as the wavefronts' operands: [M / 16][K / 32]
+// [lane][8]) the same for every plane b.  A workgroup stages its plane's columns
+// (K x W) once in LDS, as BF16 and K contiguous, and its four wavefronts take
+// 16 MB rows of A each, straight from L2, 1 KB per load.  per > 0 splits K into chunks of `per` tiles that are added in order: the
+// rounding of the split-K GEMM it stands for.
+template <int NB, int MB, bool SPLIT>
+__global__ __launch_bounds__(256) void plane_dft_kernel(const unsigned short *__restrict__ A,
+                                                        const float *__restrict__ in, float *__restrict__ out, int M,
+                                                        int K, int W, int per)
+{
+    extern __shared__ __align__(16) unsigned short Bs[];   // [NB * 16][K + 8], column w at row (w % NB) 16 + w / NB
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ld = K + 8;
+    const int m0 = (blockIdx.x * 4 + wave) * 16 * MB;
+    const float *src = in + (long)blockIdx.y * K * W;
+    // G tiles of A are in flight: the first group under the staging loads
+    constexpr int G = 16 / MB;
+    const int tiles = K / 32;
+    const bool mine = m0 < M;   // M is a multiple of 16 MB
+    const unsigned short *afrag = A + (long)((mine ? m0 : 0) / 16) * tiles * 512 + lane * 8;
+    bf16x8_t a[G][MB], an[G][MB];
+    auto fetch = [&](bf16x8_t (&v)[G][MB], int t0) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) v[g][i] = *(const bf16x8_t *)(afrag + (i * tiles + min(t0 + g, tiles - 1)) * 512);
+    };
+    fetch(a, 0);
+#pragma unroll 4
+    for (int e = threadIdx.x; e < K / 8 * W; e += 256) {
+        const int w = e & (W - 1), k8 = e / W;
+        f32x8_t v;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = src[(k8 * 8 + i) * W + w];
+        *(bf16x8_t *)&Bs[((w % NB) * 16 + w / NB) * ld + k8 * 8] = to_bf16x8(v);
+    }
+    __syncthreads();
+    if (!mine) return;
+    const unsigned short *brow = Bs + (lane & 15) * ld + (lane >> 4) * 8;
+    f32x4_t acc[MB][NB], sum[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int t0 = 0; t0 < tiles; t0 += G) {
+        if (t0 + G < tiles) fetch(an, t0 + G);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int t = t0 + g;
+            if (t < tiles) {
+                bf16x8_t b[NB];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) b[j] = *(const bf16x8_t *)(brow + j * 16 * ld + t * 32);
+#pragma unroll
+                for (int i = 0; i < MB; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) acc[i][j] = mfma(a[g][i], b[j], acc[i][j]);
+                if (SPLIT && ((t + 1) % per == 0 || t + 1 == tiles)) {
+#pragma unroll
+                    for (int i = 0; i < MB; ++i)
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) {
+                            sum[i][j] += acc[i][j];
+                            acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                        }
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int i = 0; i < MB; ++i) a[g][i] = an[g][i];
+    }
+    float *dst = out + (long)blockIdx.y * M * W;
+    const int w0 = (lane & 15) * NB;
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float *row = dst + (long)(m0 + i * 16 + 4 * (lane >> 4) + q) * W + w0;
+            float v[NB];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) v[j] = SPLIT ? sum[i][j][q] : acc[i][j][q];
+            if (NB == 4) *(float4 *)row = make_float4(v[0], v[1 % NB], v[2 % NB], v[3 % NB]);
+            else if (NB == 2) *(float2 *)row = make_float2(v[0], v[1 % NB]);
+            else if (w0 < W) row[0] = v[0];
+        }
+}
+
 } // namespace
 
 bool wgrad_covers(int K, int N, long rows) { return K <= 64 && N <= 64 && rows % 32 == 0; }
@@ -148,6 +237,34 @@ hipError_t run_wgrad(const float *X, int K, const float *D, int N, long rows, fl
     const int total = K * N + N;
     hipLaunchKernelGGL(sum_partials, dim3((total + 63) / 64), dim3(64), 0, s, part, WGRAD_SPLITS, total, out);
     return hipGetLastError();
+}
+
+bool plane_dft_covers(int M, int K, int W)
+{
+    return M % 16 == 0 && K % 32 == 0 && W <= 64 && (W & (W - 1)) == 0 && K <= 1024;
+}
+
+hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, int M, int K, int W, int planes, int per,
+                         hipStream_t s)
+{
+    if (!plane_dft_covers(M, K, W) || planes < 1 || planes > 65535) return hipErrorInvalidValue;
+    // 64 rows of A per wavefront while that leaves two workgroups for every CU,
+    // else 16: the planes of a single sample would fill a quarter of the chip
+    const bool wide = M % 64 == 0 && (long)planes * (M / 64) >= 1024;
+    return with_blocks(W, [&](auto nb) {
+        constexpr int NB = decltype(nb)::value;
+        const size_t lds = sizeof(unsigned short) * NB * 16 * (K + 8);
+        auto go = [&](auto mb, auto split) {
+            constexpr int MB = decltype(mb)::value;
+            hipLaunchKernelGGL((plane_dft_kernel<NB, MB, decltype(split)::value>),
+                               dim3((M + 64 * MB - 1) / (64 * MB), planes), dim3(256), lds, s, A, in, out, M, K, W, per);
+            return hipGetLastError();
+        };
+        using M1 = std::integral_constant<int, 1>;
+        using M4 = std::integral_constant<int, 4>;
+        if (per > 0) return wide ? go(M4{}, std::true_type{}) : go(M1{}, std::true_type{});
+        return wide ? go(M4{}, std::false_type{}) : go(M1{}, std::false_type{});
+    });
 }
 
 } // namespace bec

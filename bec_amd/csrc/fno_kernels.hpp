@@ -15,4 +15,17 @@ constexpr int WGRAD_SPLITS = 256;
 bool wgrad_covers(int K, int N, long rows);
 hipError_t run_wgrad(const float *X, int K, const float *D, int N, long rows, float *part, float *out, hipStream_t s);
 
+// Offset of entry (m, k) of an M x K BF16 matrix stored as MFMA operands:
+// [M / 16][K / 32][lane][8], lane (m % 16) + 16 ((k % 32) / 8)
+constexpr long operand_at(long m, long k, long K)
+{
+    return ((m / 16 * (K / 32) + k / 32) * 64 + m % 16 + 16 * (k % 32 / 8)) * 8 + k % 8;
+}
+
+// out[p] = A in[p] for `planes` planes: A M x K in BF16 (operand_at), in[p] K x W, out[p] M x W; per > 0: K in chunks of `per` 32-value tiles, added in
+// order.  W a power of two up to 64, M a multiple of 16, K of 32 up to 1024.
+bool plane_dft_covers(int M, int K, int W);
+hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, int M, int K, int W, int planes, int per,
+                         hipStream_t s);
+
 } // namespace bec
