@@ -55,6 +55,8 @@ bec_map2 m2(long lo_count, long lo_stride, long hi_stride)
     return m;
 }
 
+long up(long v, long to) { return (v + to - 1) / to * to; }
+
 bool pow2(long v) { return v > 0 && (v & (v - 1)) == 0; }
 
 // ---------------------------------------------------------------- kernels
@@ -262,6 +264,7 @@ struct bec_fno {
     unsigned short *E = nullptr;      // [layers][modes][2W][2W] BF16
     float *Fz = nullptr, *Fxy = nullptr, *one = nullptr;
     unsigned short *FxyB = nullptr, *FxyTB = nullptr;    // Fxy and its transpose as BF16 MFMA operands
+    unsigned short *FzB = nullptr, *FzTB = nullptr;      // Fz and its transpose, likewise (padded with zeros)
     // activations
     std::vector<float *> h, u;        // h[0..L], u[0..L-1] (u[L-1] aliases h[L])
     float *zf = nullptr, *tm = nullptr, *zi = nullptr;   // spectral temporaries
@@ -459,6 +462,13 @@ struct Spec {
 // Zf = Fz h  (transpose = 0) or out = Fz^T zin (transpose = 1, beta)
 hipError_t zdft(const bec_fno *f, const Spec &q, const float *in, float *out, int transpose, float beta, hipStream_t s)
 {
+    if (!transpose && z_dft_covers(q.mz2, q.nz, q.PW)) {
+        if ((long)q.B * q.nz * q.PW > room(f, in, 4) || (long)q.B * q.mz2 * q.PW > room(f, out, 4)) {
+            set_last_error("surrogate z transform exceeds its buffers");
+            return hipErrorInvalidValue;
+        }
+        return run_z_dft(f->FzB, in, out, q.mz2, q.nz, (int)q.PW, q.B, split_tiles(q.mz2, (int)q.PW, q.nz, q.B), s);
+    }
     if (!transpose)
         return G(f, f->Fz, 0, in, 0, out, q.mz2, (int)q.PW, q.nz, m1(q.nz), m1(1), m1(q.PW), m1(1), m1(q.PW), m1(1), q.B,
                  m1(0), m1((long)q.nz * q.PW), m1((long)q.mz2 * q.PW), 0.0f, nullptr, 1, nullptr, s);
@@ -517,7 +527,24 @@ hipError_t mode_mix_row(const bec_fno *f, const float *A, const unsigned short *
     return hipGetLastError();
 }
 
-hipError_t forward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
+// The end of layer l on run_layer_out: forward from the spectral modes in zi,
+// input h and the layer's parameters; backward (back) from the output gradient h
+hipError_t layer_out(const bec_fno *f, const Spec &q, const float *h, int l, const float *u, float *r, float *g, int back,
+                     hipStream_t s)
+{
+    const long n = (long)q.B * q.nz * q.PW;
+    if (n > room(f, h, 4) || (u && n > room(f, u, 4)) || (r && n > room(f, r, 4)) || (g && n > room(f, g, 4)) ||
+        (long)q.B * q.mz2 * q.PW > room(f, f->zi, 4)) {
+        set_last_error("surrogate layer output exceeds its buffers");
+        return hipErrorInvalidValue;
+    }
+    return run_layer_out({f->FzTB, f->zi, h, f->params + f->oW[l], f->params + f->ob[l], u, r, g, q.mz2, q.nz, (int)q.P,
+                          q.W, q.B, back},
+                         s);
+}
+
+// keep: the layers' outputs before GELU are kept for a backward pass
+hipError_t forward_impl(bec_fno *f, int B, const float *x, bool keep, hipStream_t s)
 {
     const bec_fno_config &c = f->c;
     const int W = c.width, L = c.layers;
@@ -542,6 +569,11 @@ hipError_t forward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
                    hipSuccess)
             return e;
         if ((e = xydft(f, q, f->tm, f->zi, 1, s)) != hipSuccess) return e;
+        if (layer_out_covers(c.nz, W)) {
+            float *g = l < L - 1 ? f->h[l + 1] : nullptr;
+            if ((e = layer_out(f, q, hin, l, nullptr, g && !keep ? nullptr : ul, g, 0, s)) != hipSuccess) return e;
+            continue;
+        }
         if ((e = zdft(f, q, f->zi, ul, 1, 0.0f, s)) != hipSuccess) return e;
         if ((e = rowgemm(f, hin, f->params + f->oW[l], ul, rows, W, W, 1.0f, f->params + f->ob[l], s)) != hipSuccess)
             return e;
@@ -579,15 +611,16 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
     float *dh = f->dA;    // gradient w.r.t. the current layer output
     if ((e = rowgemm_bt(f, da1, f->params + f->oQ1, dh, rows, H, W, 0.0f, s)) != hipSuccess) return e;
     for (int l = L - 1; l >= 0; --l) {
-        float *du = dh;   // in place: du = dh * gelu'(u_l)
-        if (l < L - 1) {
+        float *du = dh;   // in place: du = dh * gelu'(u_l), by the layer above where it runs fused
+        const bool fused = layer_out_covers(c.nz, W);
+        if (l < L - 1 && !fused) {
             hipLaunchKernelGGL(gelu_bwd, grid1(rows * W), dim3(256), 0, s, f->u[l], du, rows * W);
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
         const float *hin = f->h[l];
         if ((e = layer_grad(f, hin, W, du, W, rows, g + f->oW[l], s)) != hipSuccess) return e;
         float *dhin = (dh == f->dA) ? f->dH : f->dA;
-        if ((e = rowgemm_bt(f, du, f->params + f->oW[l], dhin, rows, W, W, 0.0f, s)) != hipSuccess) return e;
+        if (!fused && (e = rowgemm_bt(f, du, f->params + f->oW[l], dhin, rows, W, W, 0.0f, s)) != hipSuccess) return e;
         // spectral path, adjoint order
         if ((e = zdft(f, q, du, f->zi, 0, 0.0f, s)) != hipSuccess) return e;          // dZi = Fz du
         if ((e = xydft(f, q, f->zi, f->tm, 0, s)) != hipSuccess) return e;            // dT = Fxy dZi
@@ -603,7 +636,11 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
                    (int)modes, mm.batch, m1(4L * W * W), mm.batch, 0.0f, nullptr, 1, nullptr, s)) != hipSuccess)
             return e;
         if ((e = xydft(f, q, f->zf, f->zi, 1, s)) != hipSuccess) return e;            // dZf = Fxy^T dSp
-        if ((e = zdft(f, q, f->zi, dhin, 1, 1.0f, s)) != hipSuccess) return e;        // dh += Fz^T dZf
+        if (fused)
+            e = layer_out(f, q, du, l, l > 0 ? f->u[l - 1] : nullptr, dhin, nullptr, 1, s);   // dh = du W^T + Fz^T dZf
+        else
+            e = zdft(f, q, f->zi, dhin, 1, 1.0f, s);   // dh += Fz^T dZf
+        if (e != hipSuccess) return e;
         dh = dhin;
     }
     // lift
@@ -661,7 +698,14 @@ hipError_t build_tables(bec_fno *f)
         for (long r = 0; r < 2 * mxy; ++r)
             for (long k = 0; k < 2 * P; ++k)
                 fb[operand_at(r, k, 2 * P)] = ft[operand_at(k, r, 2 * mxy)] = host_bf16(fxy[r * 2 * P + k]);
-    hipError_t e = hipMemcpy(f->FxyB, fb.data(), fb.size() * 2, hipMemcpyHostToDevice);
+    // (operands of dimensions that the fused kernels' shapes round up: zeros)
+    std::vector<unsigned short> zb((size_t)(up(2 * c.mz, 32) * up(c.nz, 32)), 0), zt(zb);
+    for (long r = 0; r < 2 * c.mz; ++r)
+        for (long z = 0; z < c.nz; ++z)
+            zb[operand_at(r, z, up(c.nz, 32))] = zt[operand_at(z, r, up(2 * c.mz, 32))] = host_bf16(fz[r * c.nz + z]);
+    hipError_t e = hipMemcpy(f->FzB, zb.data(), zb.size() * 2, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->FzTB, zt.data(), zt.size() * 2, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(f->FxyB, fb.data(), fb.size() * 2, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(f->FxyTB, ft.data(), ft.size() * 2, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(f->Fz, fz.data(), fz.size() * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(f->Fxy, fxy.data(), fxy.size() * sizeof(float), hipMemcpyHostToDevice);
@@ -713,6 +757,8 @@ int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
     FA(f->Fxy, fb * 4 * f->mxy * f->P);
     FA(f->FxyB, sizeof(unsigned short) * 4 * f->mxy * f->P);
     FA(f->FxyTB, sizeof(unsigned short) * 4 * f->mxy * f->P);
+    FA(f->FzB, sizeof(unsigned short) * up(2 * c.mz, 32) * up(c.nz, 32));
+    FA(f->FzTB, sizeof(unsigned short) * up(2 * c.mz, 32) * up(c.nz, 32));
     FA(f->one, fb);
     f->h.assign(L + 1, nullptr);
     f->u.assign(L, nullptr);
@@ -821,7 +867,7 @@ extern "C" int bec_fno_forward(bec_fno *f, int batch, const float *d_x, float *d
     if (!f || !d_x || !d_y || batch < 1 || batch > f->c.max_batch) return BEC_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}});
-    BEC_HIP(bec::forward_impl(f, batch, d_x, s));
+    BEC_HIP(bec::forward_impl(f, batch, d_x, false, s));
     BEC_HIP(hipMemcpyAsync(d_y, f->y, sizeof(float) * batch * f->S * f->c.c_out, hipMemcpyDeviceToDevice, s));
     return BEC_OK;
 }
@@ -847,7 +893,7 @@ extern "C" int bec_fno_loss_backward(bec_fno *f, int batch, const float *d_x, co
     if (!f || !d_x || !d_target || batch < 1 || batch > f->c.max_batch) return BEC_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}});
-    BEC_HIP(bec::forward_impl(f, batch, d_x, s));
+    BEC_HIP(bec::forward_impl(f, batch, d_x, true, s));
     const long n = (long)batch * f->S * f->c.c_out;
     const long blocks = (n + 255) / 256;
     hipLaunchKernelGGL(bec::mse_grad, dim3((unsigned)blocks), dim3(256), 0, s, f->y, d_target, f->dy, n,

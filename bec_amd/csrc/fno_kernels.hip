@@ -216,6 +216,180 @@ __global__ __launch_bounds__(256) void plane_dft_kernel(const unsigned short *__
         }
 }
 
+// Transform along z: out[b] = A in[b], A the M x K operand matrix (rows beyond M
+// zero), in[b] K x N, out[b] M x N.  A wavefront owns 64 columns, four adjacent
+// ones per lane (256-byte row segments), and reads them once.
+template <int MB, bool SPLIT>
+__global__ __launch_bounds__(256) void z_dft_kernel(const unsigned short *__restrict__ A, const float *__restrict__ in,
+                                                    float *__restrict__ out, int M, int K, int N, int per)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kq = (lane >> 4) * 8, tiles = K / 32;
+    const int n0 = (blockIdx.x * 4 + wave) * 64 + (lane & 15) * 4;
+    if (n0 - (lane & 15) * 4 >= N) return;   // N is a multiple of 64
+    const float *src = in + (long)blockIdx.y * K * N + (long)kq * N + n0;
+    const unsigned short *afrag = A + lane * 8;
+    f32x4_t acc[MB][4], sum[MB][4], v[8];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = *(const f32x4_t *)(src + (long)k * N);
+    for (int t = 0; t < tiles; ++t) {
+        f32x4_t vn[8];
+        bf16x8_t a[MB];
+        if (t + 1 < tiles)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) vn[k] = *(const f32x4_t *)(src + ((long)(t + 1) * 32 + k) * N);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) a[i] = *(const bf16x8_t *)(afrag + (i * tiles + t) * 512);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bf16x8_t b =
+                to_bf16x8((f32x8_t){v[0][j], v[1][j], v[2][j], v[3][j], v[4][j], v[5][j], v[6][j], v[7][j]});
+#pragma unroll
+            for (int i = 0; i < MB; ++i) acc[i][j] = mfma(a[i], b, acc[i][j]);
+        }
+        if (SPLIT && ((t + 1) % per == 0 || t + 1 == tiles)) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = vn[k];
+    }
+    float *dst = out + (long)blockIdx.y * M * N + n0;
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int m = i * 16 + 4 * (lane >> 4) + q;
+            if (m >= M) continue;
+            f32x4_t r;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) r[j] = SPLIT ? sum[i][j][q] : acc[i][j][q];
+            *(f32x4_t *)(dst + (long)m * N) = r;
+        }
+}
+
+__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
+
+// gelu'(x) = Phi(x) + x phi(x)
+__device__ __forceinline__ float gelu_slope(float x)
+{
+    const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
+    const float pdf = 0.39894228040143268f * expf(-0.5f * x * x);
+    return cdf + x * pdf;
+}
+
+template <int V> struct VecF;
+template <> struct VecF<1> { typedef float type __attribute__((ext_vector_type(1))); };
+template <> struct VecF<2> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct VecF<4> { typedef float type __attribute__((ext_vector_type(4))); };
+
+// What leaves a spectral layer: r = h W (+ b) + Fz^T s, one pass over h and s
+// (the z modes of the layer's spectral part), both products in one wavefront's
+// registers: 32 z values of one column (b, y, x).  BACK applies W^T and no bias.
+// EPI: 0 stores r; 1 stores r and gelu(r); 2 stores gelu(r) alone; 3 stores
+// r gelu'(u).  It stands for the transform, the per-cell GEMM that read its
+// result again and a GELU kernel (46 + 64 + 28 us at batch 16).
+template <int V, bool BACK, int EPI>
+__global__ __launch_bounds__(256) void layer_out_kernel(const unsigned short *__restrict__ FzT,
+                                                        const float *__restrict__ s, int ms,
+                                                        const float *__restrict__ h, const float *__restrict__ Wm,
+                                                        const float *__restrict__ bias, int nz, int P,
+                                                        const float *__restrict__ u, float *__restrict__ r_out,
+                                                        float *__restrict__ g_out)
+{
+    constexpr int W = 16 * V, WT = (W + 31) / 32, ZB = 2;
+    using vec = typename VecF<V>::type;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, kq = (lane >> 4) * 8;
+    const int p = blockIdx.x * 4 + wave, zb0 = blockIdx.y * ZB, w0 = c * V;
+    if (p >= P) return;
+    const long b = blockIdx.z;
+    const int st = (ms + 31) / 32;
+    // the layer input's rows first: the longest reads
+    f32x8_t ha[ZB][WT];
+#pragma unroll
+    for (int i = 0; i < ZB; ++i)
+#pragma unroll
+        for (int t = 0; t < WT; ++t) {
+            const float *row = h + ((b * nz + (zb0 + i) * 16 + c) * P + p) * W + t * 32 + kq;
+            ha[i][t] = (f32x8_t){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (W >= 32 || kq < W) {
+                const f32x4_t lo = *(const f32x4_t *)row, hi = *(const f32x4_t *)(row + 4);
+                ha[i][t] = (f32x8_t){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            }
+        }
+    f32x4_t az[ZB][V], aw[ZB][V];
+#pragma unroll
+    for (int i = 0; i < ZB; ++i)
+#pragma unroll
+        for (int j = 0; j < V; ++j) az[i][j] = aw[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < st; ++t) {
+        vec v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int m = t * 32 + kq + k;
+            v[k] = *(const vec *)(s + ((b * ms + min(m, ms - 1)) * P + p) * W + w0);
+            if (m >= ms) v[k] = (vec)(0.f);
+        }
+        bf16x8_t a[ZB];
+#pragma unroll
+        for (int i = 0; i < ZB; ++i) a[i] = *(const bf16x8_t *)(FzT + ((long)((zb0 + i) * st + t) * 64 + lane) * 8);
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const bf16x8_t bb =
+                to_bf16x8((f32x8_t){v[0][j], v[1][j], v[2][j], v[3][j], v[4][j], v[5][j], v[6][j], v[7][j]});
+#pragma unroll
+            for (int i = 0; i < ZB; ++i) az[i][j] = mfma(a[i], bb, az[i][j]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            f32x8_t w;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int i = t * 32 + kq + k;
+                w[k] = i < W ? (BACK ? Wm[(w0 + j) * W + i] : Wm[i * W + w0 + j]) : 0.f;
+            }
+            const bf16x8_t bb = to_bf16x8(w);
+#pragma unroll
+            for (int i = 0; i < ZB; ++i) aw[i][j] = mfma(to_bf16x8(ha[i][t]), bb, aw[i][j]);
+        }
+    vec bv = (vec)(0.f);
+    if (!BACK) bv = *(const vec *)(bias + w0);
+#pragma unroll
+    for (int i = 0; i < ZB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const long at = ((b * nz + (zb0 + i) * 16 + 4 * (lane >> 4) + q) * P + p) * W + w0;
+            vec r, g;
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                r[j] = aw[i][j][q] + az[i][j][q];
+                if (!BACK) r[j] += bv[j];
+            }
+            if (EPI == 3) {
+                const vec uv = *(const vec *)(u + at);
+#pragma unroll
+                for (int j = 0; j < V; ++j) r[j] *= gelu_slope(uv[j]);
+            }
+            if (EPI != 2) *(vec *)(r_out + at) = r;
+            if (EPI == 1 || EPI == 2) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) g[j] = gelu(r[j]);
+                *(vec *)(g_out + at) = g;
+            }
+        }
+}
+
 } // namespace
 
 bool wgrad_covers(int K, int N, long rows) { return K <= 64 && N <= 64 && rows % 32 == 0; }
@@ -264,6 +438,42 @@ hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, i
         using M4 = std::integral_constant<int, 4>;
         if (per > 0) return wide ? go(M4{}, std::true_type{}) : go(M1{}, std::true_type{});
         return wide ? go(M4{}, std::false_type{}) : go(M1{}, std::false_type{});
+    });
+}
+
+bool z_dft_covers(int M, int K, long N) { return M <= 64 && K % 32 == 0 && N % 64 == 0; }
+
+hipError_t run_z_dft(const unsigned short *A, const float *in, float *out, int M, int K, int N, int batch, int per,
+                     hipStream_t s)
+{
+    if (!z_dft_covers(M, K, N) || batch < 1 || batch > 65535) return hipErrorInvalidValue;
+    return with_blocks(M, [&](auto mb) {
+        constexpr int MB = decltype(mb)::value;
+        const dim3 grid((N / 64 + 3) / 4, batch);
+        if (per > 0) hipLaunchKernelGGL((z_dft_kernel<MB, true>), grid, dim3(256), 0, s, A, in, out, M, K, N, per);
+        else hipLaunchKernelGGL((z_dft_kernel<MB, false>), grid, dim3(256), 0, s, A, in, out, M, K, N, per);
+        return hipGetLastError();
+    });
+}
+
+bool layer_out_covers(int nz, int W) { return nz % 32 == 0 && (W == 16 || W == 32 || W == 64); }
+
+hipError_t run_layer_out(const LayerOut &a, hipStream_t s)
+{
+    if (!layer_out_covers(a.nz, a.W) || a.batch < 1 || a.batch > 65535) return hipErrorInvalidValue;
+    const dim3 grid((a.P + 3) / 4, a.nz / 32, a.batch);
+    return with_blocks(a.W, [&](auto v) {
+        constexpr int V = decltype(v)::value;
+        auto go = [&](auto back, auto epi) {
+            hipLaunchKernelGGL((layer_out_kernel<V, decltype(back)::value, decltype(epi)::value>), grid, dim3(256), 0, s,
+                               a.FzT, a.s, a.ms, a.h, a.Wm, a.bias, a.nz, a.P, a.u, a.r, a.g);
+            return hipGetLastError();
+        };
+        using E0 = std::integral_constant<int, 0>;
+        if (a.back) return a.u ? go(std::true_type{}, std::integral_constant<int, 3>{}) : go(std::true_type{}, E0{});
+        if (!a.g) return go(std::false_type{}, E0{});
+        return a.r ? go(std::false_type{}, std::integral_constant<int, 1>{})
+                   : go(std::false_type{}, std::integral_constant<int, 2>{});
     });
 }
 

@@ -28,4 +28,24 @@ bool plane_dft_covers(int M, int K, int W);
 hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, int M, int K, int W, int planes, int per,
                          hipStream_t s);
 
+// out[b] = A in[b]: A M x K operands (operand_at, M rounded up to 16 with zeros),
+// in[b] K x N, out[b] M x N; per as above.  M <= 64, K % 32 == 0, N % 64 == 0.
+bool z_dft_covers(int M, int K, long N);
+hipError_t run_z_dft(const unsigned short *A, const float *in, float *out, int M, int K, int N, int batch, int per,
+                     hipStream_t s);
+
+// What leaves a spectral layer, forward (back = 0): r = h W + bias + Fz^T s, and
+// with g set gelu(r) there (r may then be null); backward (back = 1):
+// r = h W^T + Fz^T s, times gelu'(u) when u is set.  h, r, g, u [batch][nz][P][W];
+// s [batch][ms][P][W]; FzT nz x ms operands (ms rounded up to 32 with zeros).
+// W 16, 32 or 64; nz % 32 == 0.
+struct LayerOut {
+    const unsigned short *FzT;
+    const float *s, *h, *Wm, *bias, *u;
+    float *r, *g;
+    int ms, nz, P, W, batch, back;
+};
+bool layer_out_covers(int nz, int W);
+hipError_t run_layer_out(const LayerOut &a, hipStream_t s);
+
 } // namespace bec
