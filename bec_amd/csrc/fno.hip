@@ -543,8 +543,8 @@ hipError_t layer_out(const bec_fno *f, const Spec &q, const float *h, int l, con
                          s);
 }
 
-// keep: the layers' outputs before GELU are kept for a backward pass
-hipError_t forward_impl(bec_fno *f, int B, const float *x, bool keep, hipStream_t s)
+// y: the output; keep: the values a backward pass reads are stored
+hipError_t forward_impl(bec_fno *f, int B, const float *x, float *y, bool keep, hipStream_t s)
 {
     const bec_fno_config &c = f->c;
     const int W = c.width, L = c.layers;
@@ -554,8 +554,11 @@ hipError_t forward_impl(bec_fno *f, int B, const float *x, bool keep, hipStream_
     const long modes = f->modes;
     hipError_t e;
     // lift
-    if ((e = rowgemm(f, x, f->params + f->oP, f->h[0], rows, c.c_in, W, 0.0f, f->params + f->op, s)) != hipSuccess)
-        return e;
+    if (lift_covers(c.c_in, W, rows) && (uintptr_t)x % 16 == 0 && rows * c.c_in <= room(f, x, 4))
+        e = run_lift(x, c.c_in, f->params + f->oP, f->params + f->op, W, rows, f->h[0], s);
+    else
+        e = rowgemm(f, x, f->params + f->oP, f->h[0], rows, c.c_in, W, 0.0f, f->params + f->op, s);
+    if (e != hipSuccess) return e;
     for (int l = 0; l < L; ++l) {
         const float *hin = f->h[l];
         float *ul = f->u[l];
@@ -583,12 +586,15 @@ hipError_t forward_impl(bec_fno *f, int B, const float *x, bool keep, hipStream_
         }
     }
     // projection
+    if (project_covers(W, c.hidden, c.c_out, rows) && rows * c.c_out <= room(f, y, 4))
+        return run_project(f->h[L], f->params + f->oQ1, f->params + f->oq1, f->params + f->oQ2, f->params + f->oq2, W,
+                           c.hidden, c.c_out, rows, keep ? f->g1 : nullptr, f->a1, y, s);
     if ((e = rowgemm(f, f->h[L], f->params + f->oQ1, f->g1, rows, W, c.hidden, 0.0f, f->params + f->oq1, s)) !=
         hipSuccess)
         return e;
     hipLaunchKernelGGL(gelu_fwd, grid1(rows * c.hidden), dim3(256), 0, s, f->g1, f->a1, rows * c.hidden);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    return rowgemm(f, f->a1, f->params + f->oQ2, f->y, rows, c.hidden, c.c_out, 0.0f, f->params + f->oq2, s);
+    return rowgemm(f, f->a1, f->params + f->oQ2, y, rows, c.hidden, c.c_out, 0.0f, f->params + f->oq2, s);
 }
 
 hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
@@ -604,12 +610,18 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
     // projection: y = a1 Q2 + q2, a1 = gelu(g1), g1 = hL Q1 + q1
     if ((e = layer_grad(f, f->a1, H, f->dy, c.c_out, rows, g + f->oQ2, s)) != hipSuccess) return e;
     float *da1 = f->dB;   // [rows][H]
-    if ((e = rowgemm_bt(f, f->dy, f->params + f->oQ2, da1, rows, c.c_out, H, 0.0f, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(gelu_bwd, grid1(rows * H), dim3(256), 0, s, f->g1, da1, rows * H);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = layer_grad(f, f->h[L], W, da1, H, rows, g + f->oQ1, s)) != hipSuccess) return e;
     float *dh = f->dA;    // gradient w.r.t. the current layer output
-    if ((e = rowgemm_bt(f, da1, f->params + f->oQ1, dh, rows, H, W, 0.0f, s)) != hipSuccess) return e;
+    const bool fused_p = project_covers(W, H, c.c_out, rows);
+    if (fused_p) {
+        e = run_project_back(f->dy, f->params + f->oQ1, f->params + f->oQ2, f->g1, W, H, c.c_out, rows, da1, dh, s);
+        if (e != hipSuccess) return e;
+    } else {
+        if ((e = rowgemm_bt(f, f->dy, f->params + f->oQ2, da1, rows, c.c_out, H, 0.0f, s)) != hipSuccess) return e;
+        hipLaunchKernelGGL(gelu_bwd, grid1(rows * H), dim3(256), 0, s, f->g1, da1, rows * H);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+    if ((e = layer_grad(f, f->h[L], W, da1, H, rows, g + f->oQ1, s)) != hipSuccess) return e;
+    if (!fused_p && (e = rowgemm_bt(f, da1, f->params + f->oQ1, dh, rows, H, W, 0.0f, s)) != hipSuccess) return e;
     for (int l = L - 1; l >= 0; --l) {
         float *du = dh;   // in place: du = dh * gelu'(u_l), by the layer above where it runs fused
         const bool fused = layer_out_covers(c.nz, W);
@@ -866,9 +878,17 @@ extern "C" int bec_fno_forward(bec_fno *f, int batch, const float *d_x, float *d
 {
     if (!f || !d_x || !d_y || batch < 1 || batch > f->c.max_batch) return BEC_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
-    bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}});
-    BEC_HIP(bec::forward_impl(f, batch, d_x, false, s));
-    BEC_HIP(hipMemcpyAsync(d_y, f->y, sizeof(float) * batch * f->S * f->c.c_out, hipMemcpyDeviceToDevice, s));
+    const size_t out = sizeof(float) * batch * f->S * f->c.c_out;
+    bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}, {d_y, out}});
+    // straight into the caller's buffer where it is a device allocation that holds
+    // the output; the copy reports what else it is given
+    void *base = nullptr;
+    size_t size = 0;
+    const bool direct = hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)d_y) == hipSuccess &&
+                        (uintptr_t)d_y % sizeof(float) == 0 && (char *)d_y + out <= (char *)base + size;
+    if (!direct) (void)hipGetLastError();
+    BEC_HIP(bec::forward_impl(f, batch, d_x, direct ? d_y : f->y, false, s));
+    if (!direct) BEC_HIP(hipMemcpyAsync(d_y, f->y, out, hipMemcpyDeviceToDevice, s));
     return BEC_OK;
 }
 
@@ -893,7 +913,7 @@ extern "C" int bec_fno_loss_backward(bec_fno *f, int batch, const float *d_x, co
     if (!f || !d_x || !d_target || batch < 1 || batch > f->c.max_batch) return BEC_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}});
-    BEC_HIP(bec::forward_impl(f, batch, d_x, true, s));
+    BEC_HIP(bec::forward_impl(f, batch, d_x, f->y, true, s));
     const long n = (long)batch * f->S * f->c.c_out;
     const long blocks = (n + 255) / 256;
     hipLaunchKernelGGL(bec::mse_grad, dim3((unsigned)blocks), dim3(256), 0, s, f->y, d_target, f->dy, n,

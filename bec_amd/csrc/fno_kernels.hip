@@ -390,6 +390,221 @@ __global__ __launch_bounds__(256) void layer_out_kernel(const unsigned short *__
         }
 }
 
+// Eight consecutive K values of a row-major FP32 operand row as BF16; zeros from
+// `width` on (a multiple of 8).
+__device__ __forceinline__ bf16x8_t row_operand(const float *row, int k, int width)
+{
+    f32x8_t v = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (k < width) {
+        const f32x4_t lo = *(const f32x4_t *)(row + k), hi = *(const f32x4_t *)(row + k + 4);
+        v = (f32x8_t){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    return to_bf16x8(v);
+}
+
+// The lift: out = x P + p, 16 rows at a time per wavefront, P in registers.
+template <int V>
+__global__ __launch_bounds__(256) void lift_kernel(const float *__restrict__ x, int K, const float *__restrict__ P,
+                                                   const float *__restrict__ bias, long tiles, float *__restrict__ out)
+{
+    constexpr int W = 16 * V;
+    using vec = typename VecF<V>::type;
+    const int lane = threadIdx.x & 63, c = lane & 15, kq = (lane >> 4) * 8, w0 = c * V;
+    bf16x8_t pb[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        f32x8_t w;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = kq + k < K ? P[(kq + k) * W + w0 + j] : 0.f;
+        pb[j] = to_bf16x8(w);
+    }
+    const vec bv = *(const vec *)(bias + w0);
+    for (long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6); t < tiles; t += (long)gridDim.x * 4) {
+        const bf16x8_t a = row_operand(x + (t * 16 + c) * K, kq, K);
+        f32x4_t acc[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[j] = mfma(a, pb[j], (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            vec r;
+#pragma unroll
+            for (int j = 0; j < V; ++j) r[j] = acc[j][q] + bv[j];
+            *(vec *)(out + (t * 16 + 4 * (lane >> 4) + q) * W + w0) = r;
+        }
+    }
+}
+
+// A 16-row tile of BF16 values between the result layout of one product (rows
+// 4 (l / 16) + q, columns V c + j) and the operand layout of the next (row
+// l % 16, eight consecutive columns), through this wavefront's LDS rows.
+template <int V>
+__device__ __forceinline__ void tile_put(unsigned short *T, int ld, int lane, int q, const float (&v)[V])
+{
+    typedef float fV __attribute__((ext_vector_type(V)));
+    typedef __bf16 bV __attribute__((ext_vector_type(V)));
+    fV f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) f[j] = v[j];
+    *(bV *)&T[(4 * (lane >> 4) + q) * ld + (lane & 15) * V] = __builtin_convertvector(f, bV);
+}
+
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// The projection y = gelu(h Q1 + q1) Q2 + q2 in one pass over h; with KEEP the
+// hidden values before and after GELU are stored for the backward pass.  As
+// three launches the hidden values (134 MB at batch 16) were written, read,
+// written and read again: 72 + 64 + 64 us.
+template <int VW, int VH, bool KEEP>
+__global__ __launch_bounds__(256) void project_kernel(const float *__restrict__ h, const float *__restrict__ Q1,
+                                                      const float *__restrict__ q1, const float *__restrict__ Q2,
+                                                      const float *__restrict__ q2, int co, long tiles,
+                                                      float *__restrict__ g1, float *__restrict__ a1,
+                                                      float *__restrict__ y)
+{
+    constexpr int W = 16 * VW, H = 16 * VH, WT = (W + 31) / 32, HT = (H + 31) / 32, LD = HT * 32 + 8;
+    using vec = typename VecF<VH>::type;
+    __shared__ __align__(16) unsigned short lds[4][16 * LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, kq = (lane >> 4) * 8, h0 = c * VH;
+    unsigned short *T = lds[wave];
+    for (int i = lane; i < 16 * LD; i += 64) T[i] = 0;   // columns beyond H stay zero
+    bf16x8_t w1[WT][VH], w2[HT];
+#pragma unroll
+    for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int j = 0; j < VH; ++j) {
+            f32x8_t w;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int i = t * 32 + kq + k;
+                w[k] = i < W ? Q1[i * H + h0 + j] : 0.f;
+            }
+            w1[t][j] = to_bf16x8(w);
+        }
+#pragma unroll
+    for (int t = 0; t < HT; ++t) {
+        f32x8_t w;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int i = t * 32 + kq + k;
+            w[k] = i < H && c < co ? Q2[i * co + c] : 0.f;
+        }
+        w2[t] = to_bf16x8(w);
+    }
+    const vec b1 = *(const vec *)(q1 + h0);
+    const float b2 = c < co ? q2[c] : 0.f;
+    wave_fence();
+    for (long t = (long)blockIdx.x * 4 + wave; t < tiles; t += (long)gridDim.x * 4) {
+        f32x4_t acc[VH], yo = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < VH; ++j) acc[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < WT; ++i) {
+            const bf16x8_t a = row_operand(h + (t * 16 + c) * W, i * 32 + kq, W);
+#pragma unroll
+            for (int j = 0; j < VH; ++j) acc[j] = mfma(a, w1[i][j], acc[j]);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const long at = (t * 16 + 4 * (lane >> 4) + q) * H + h0;
+            vec u, g;
+            float v[VH];
+#pragma unroll
+            for (int j = 0; j < VH; ++j) {
+                u[j] = acc[j][q] + b1[j];
+                g[j] = v[j] = gelu(u[j]);
+            }
+            if (KEEP) {
+                *(vec *)(g1 + at) = u;
+                *(vec *)(a1 + at) = g;
+            }
+            tile_put<VH>(T, LD, lane, q, v);
+        }
+        wave_fence();
+#pragma unroll
+        for (int i = 0; i < HT; ++i) yo = mfma(*(const bf16x8_t *)&T[c * LD + i * 32 + kq], w2[i], yo);
+        wave_fence();
+        if (c < co)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[(t * 16 + 4 * (lane >> 4) + q) * co + c] = yo[q] + b2;
+    }
+}
+
+// Its gradient: dg1 = (dy Q2^T) gelu'(g1) (kept for the weight gradients) and
+// dh = dg1 Q1^T, in one pass over g1.
+template <int VW, int VH>
+__global__ __launch_bounds__(256) void project_back_kernel(const float *__restrict__ dy, int co,
+                                                           const float *__restrict__ Q1, const float *__restrict__ Q2,
+                                                           const float *__restrict__ g1, long tiles,
+                                                           float *__restrict__ dg1, float *__restrict__ dh)
+{
+    constexpr int W = 16 * VW, H = 16 * VH, HT = (H + 31) / 32, LD = HT * 32 + 8;
+    using vec = typename VecF<VH>::type;
+    using vew = typename VecF<VW>::type;
+    __shared__ __align__(16) unsigned short lds[4][16 * LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, kq = (lane >> 4) * 8, h0 = c * VH;
+    unsigned short *T = lds[wave];
+    for (int i = lane; i < 16 * LD; i += 64) T[i] = 0;
+    bf16x8_t w2[VH], w1[HT][VW];
+#pragma unroll
+    for (int j = 0; j < VH; ++j) {
+        f32x8_t w;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) w[k] = kq + k < co ? Q2[(h0 + j) * co + kq + k] : 0.f;
+        w2[j] = to_bf16x8(w);
+    }
+#pragma unroll
+    for (int t = 0; t < HT; ++t)
+#pragma unroll
+        for (int j = 0; j < VW; ++j) w1[t][j] = row_operand(Q1 + (c * VW + j) * H, t * 32 + kq, H);
+    wave_fence();
+    for (long t = (long)blockIdx.x * 4 + wave; t < tiles; t += (long)gridDim.x * 4) {
+        f32x8_t d;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d[k] = kq + k < co ? dy[(t * 16 + c) * co + kq + k] : 0.f;
+        const bf16x8_t a = to_bf16x8(d);
+        f32x4_t acc[VH], ao[VW];
+#pragma unroll
+        for (int j = 0; j < VH; ++j) acc[j] = mfma(a, w2[j], (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const long at = (t * 16 + 4 * (lane >> 4) + q) * H + h0;
+            const vec u = *(const vec *)(g1 + at);
+            vec g;
+            float v[VH];
+#pragma unroll
+            for (int j = 0; j < VH; ++j) g[j] = v[j] = acc[j][q] * gelu_slope(u[j]);
+            *(vec *)(dg1 + at) = g;
+            tile_put<VH>(T, LD, lane, q, v);
+        }
+        wave_fence();
+#pragma unroll
+        for (int j = 0; j < VW; ++j) ao[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < HT; ++i) {
+            const bf16x8_t b = *(const bf16x8_t *)&T[c * LD + i * 32 + kq];
+#pragma unroll
+            for (int j = 0; j < VW; ++j) ao[j] = mfma(b, w1[i][j], ao[j]);
+        }
+        wave_fence();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            vew r;
+#pragma unroll
+            for (int j = 0; j < VW; ++j) r[j] = ao[j][q];
+            *(vew *)(dh + (t * 16 + 4 * (lane >> 4) + q) * W + c * VW) = r;
+        }
+    }
+}
+
+// workgroups of a kernel whose wavefronts walk `tiles` tiles: eight per CU
+int row_grid(long tiles) { return (int)std::min<long>(2048, (tiles + 3) / 4); }
+
+bool vec_width(int n) { return n == 16 || n == 32 || n == 64; }
+
 } // namespace
 
 bool wgrad_covers(int K, int N, long rows) { return K <= 64 && N <= 64 && rows % 32 == 0; }
@@ -474,6 +689,55 @@ hipError_t run_layer_out(const LayerOut &a, hipStream_t s)
         if (!a.g) return go(std::false_type{}, E0{});
         return a.r ? go(std::false_type{}, std::integral_constant<int, 1>{})
                    : go(std::false_type{}, std::integral_constant<int, 2>{});
+    });
+}
+
+bool lift_covers(int K, int W, long rows) { return K % 8 == 0 && K <= 32 && vec_width(W) && rows % 16 == 0; }
+
+hipError_t run_lift(const float *x, int K, const float *P, const float *bias, int W, long rows, float *out, hipStream_t s)
+{
+    if (!lift_covers(K, W, rows)) return hipErrorInvalidValue;
+    return with_blocks(W, [&](auto v) {
+        hipLaunchKernelGGL(lift_kernel<decltype(v)::value>, dim3(row_grid(rows / 16)), dim3(256), 0, s, x, K, P, bias,
+                           rows / 16, out);
+        return hipGetLastError();
+    });
+}
+
+bool project_covers(int W, int H, int co, long rows)
+{
+    return vec_width(W) && vec_width(H) && co <= 16 && rows % 16 == 0;
+}
+
+hipError_t run_project(const float *h, const float *Q1, const float *q1, const float *Q2, const float *q2, int W, int H,
+                       int co, long rows, float *g1, float *a1, float *y, hipStream_t s)
+{
+    if (!project_covers(W, H, co, rows)) return hipErrorInvalidValue;
+    return with_blocks(W, [&](auto vw) {
+        return with_blocks(H, [&](auto vh) {
+            constexpr int VW = decltype(vw)::value, VH = decltype(vh)::value;
+            const dim3 grid(row_grid(rows / 16));
+            if (g1)
+                hipLaunchKernelGGL((project_kernel<VW, VH, true>), grid, dim3(256), 0, s, h, Q1, q1, Q2, q2, co, rows / 16,
+                                   g1, a1, y);
+            else
+                hipLaunchKernelGGL((project_kernel<VW, VH, false>), grid, dim3(256), 0, s, h, Q1, q1, Q2, q2, co,
+                                   rows / 16, g1, a1, y);
+            return hipGetLastError();
+        });
+    });
+}
+
+hipError_t run_project_back(const float *dy, const float *Q1, const float *Q2, const float *g1, int W, int H, int co,
+                            long rows, float *dg1, float *dh, hipStream_t s)
+{
+    if (!project_covers(W, H, co, rows)) return hipErrorInvalidValue;
+    return with_blocks(W, [&](auto vw) {
+        return with_blocks(H, [&](auto vh) {
+            hipLaunchKernelGGL((project_back_kernel<decltype(vw)::value, decltype(vh)::value>), dim3(row_grid(rows / 16)),
+                               dim3(256), 0, s, dy, co, Q1, Q2, g1, rows / 16, dg1, dh);
+            return hipGetLastError();
+        });
     });
 }
 

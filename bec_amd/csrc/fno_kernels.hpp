@@ -48,4 +48,17 @@ struct LayerOut {
 bool layer_out_covers(int nz, int W);
 hipError_t run_layer_out(const LayerOut &a, hipStream_t s);
 
+// out[rows][W] = x[rows][K] P + bias.  K % 8 == 0 up to 32; W 16, 32 or 64; rows % 16 == 0.
+bool lift_covers(int K, int W, long rows);
+hipError_t run_lift(const float *x, int K, const float *P, const float *bias, int W, long rows, float *out, hipStream_t s);
+
+// y[rows][co] = gelu(h Q1 + q1) Q2 + q2; with g1 set the hidden values before and
+// after GELU go to g1 and a1 [rows][H].  W, H 16, 32 or 64; co <= 16; rows % 16 == 0.
+bool project_covers(int W, int H, int co, long rows);
+hipError_t run_project(const float *h, const float *Q1, const float *q1, const float *Q2, const float *q2, int W, int H,
+                       int co, long rows, float *g1, float *a1, float *y, hipStream_t s);
+// its gradient: dg1 = (dy Q2^T) gelu'(g1), dh = dg1 Q1^T
+hipError_t run_project_back(const float *dy, const float *Q1, const float *Q2, const float *g1, int W, int H, int co,
+                            long rows, float *dg1, float *dh, hipStream_t s);
+
 } // namespace bec
