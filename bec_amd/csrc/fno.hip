@@ -107,55 +107,6 @@ __global__ void mse_grad(const float *y, const float *t, float *dy, long n, floa
     if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
 }
 
-__device__ __forceinline__ long map_off(const bec_map2 &m, long i)
-{
-    return (i >> m.lg) * m.hi + (i & ((1L << m.lg) - 1)) * m.lo;
-}
-
-// The per-mode channel mixing for a single sample (one row per mode) with
-// 2W = 64 channels: C[t][n] = sum_k bf16(A[t][k]) E[t][k][n].  One wave per
-// mode t; lane L owns the channels n = 8 (L & 7) + i (i < 8) and the rows
-// k = (L >> 3) + 8 j, and reads E[t] in 16-byte pieces, so one load of the
-// wave covers 8 whole rows.  The 8 partial sums of a channel are combined
-// across lanes in a fixed butterfly order.  The operands are rounded as the
-// GEMM rounds them (A to BF16 nearest even, E already BF16); the products are
-// exact in FP32.
-__global__ __launch_bounds__(256) void mode_row_mix64(const float *A, const unsigned short *E, float *C, bec_map2 ab,
-                                                      bec_map2 ak, long ebatch, bec_map2 cb, bec_map2 cn, int K,
-                                                      long modes)
-{
-    const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= modes) return;   // t is the same for the whole wave
-    const int lane = threadIdx.x & 63, nb = lane & 7, kp = lane >> 3;
-    const float *a = A + map_off(ab, t);
-    const unsigned short *e = E + t * ebatch + nb * 8;
-    float acc[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-#pragma unroll 4
-    for (int k = kp; k < K; k += 8) {
-        const float x = a[map_off(ak, k)];
-        const unsigned int u = __float_as_uint(x);
-        const float xr = (u & 0x7f800000u) == 0x7f800000u ? x : __uint_as_float((unsigned int)to_bf16(x) << 16);
-        const uint4 w = *(const uint4 *)(e + (long)k * 64);
-        const unsigned int ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[2 * i] = fmaf(xr, __uint_as_float(ws[i] << 16), acc[2 * i]);
-            acc[2 * i + 1] = fmaf(xr, __uint_as_float(ws[i] & 0xffff0000u), acc[2 * i + 1]);
-        }
-    }
-#pragma unroll
-    for (int off = 8; off < 64; off <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += __shfl_xor(acc[i], off);
-    if (kp == 0) {
-        const long cbase = map_off(cb, t);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) C[cbase + map_off(cn, nb * 8 + i)] = acc[i];
-    }
-}
-
 struct Gs2Lattice {
     int nx, ny, nz;
     double xmax, ymax, zmax, dx, dy, dz, lambda, mu;
@@ -332,8 +283,10 @@ void layout(bec_fno *f)
     f->n_params = o;
 }
 
+// (only where the mixing reads the expanded matrices)
 hipError_t expand_all(bec_fno *f, hipStream_t s)
 {
+    if (mode_covers(f->c.width)) return hipSuccess;
     const long per = f->modes * f->c.width * f->c.width;
     for (int l = 0; l < f->c.layers; ++l) {
         hipLaunchKernelGGL(expand_modes, grid1(per), dim3(256), 0, s, f->params + f->oR[l],
@@ -508,23 +461,18 @@ ModeMaps mode_maps(const Spec &q)
     return m;
 }
 
-// The channel mixing of a batch-1 forward pass with 2W = 64 on mode_row_mix64
-// instead of 64 x 64 GEMM tiles that would hold one row each; the operand
-// extents are checked as G checks them.
-hipError_t mode_mix_row(const bec_fno *f, const float *A, const unsigned short *El, float *C, int W2,
-                        const ModeMaps &mm, long modes, hipStream_t s)
+// The channel mixing of layer l on run_mode_mix, or with D on run_mode_back (the
+// gradient with respect to the modes into C, to the matrices into the gradients)
+hipError_t mode_mix(const bec_fno *f, const Spec &q, int l, const float *A, const float *D, float *C, hipStream_t s)
 {
-    const long eb = (modes - 1) * (long)W2 * W2 + (long)W2 * W2 - 1;
-    const long ea = max_off(mm.batch, modes) + max_off(mm.ch, W2);
-    const long ec = max_off(mm.batch, modes) + max_off(mm.ch, W2);
-    if (W2 != 64 || ((uintptr_t)El & 15) != 0 ||
-        !(ea < room(f, A, 4) && eb < room(f, El, 2) && ec < room(f, C, 4))) {
-        set_last_error("surrogate mode mixing exceeds its buffer");
+    const long n = (long)q.B * q.mz2 * q.mxy * q.W;
+    if (n > room(f, A, 4) || (D && n > room(f, D, 4)) || n > room(f, C, 4)) {
+        set_last_error("surrogate mode mixing exceeds its buffers");
         return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(mode_row_mix64, dim3((unsigned)((modes + 3) / 4)), dim3(256), 0, s, A, El, C, mm.batch, mm.ch,
-                       (long)W2 * W2, mm.batch, mm.ch, W2, modes);
-    return hipGetLastError();
+    const float *R = f->params + f->oR[l];
+    if (D) return run_mode_back(A, D, R, C, f->grads + f->oR[l], q.W, q.mxy, q.mz2 / 2, q.B, s);
+    return run_mode_mix(A, R, C, q.W, q.mxy, q.mz2 / 2, q.B, s);
 }
 
 // The end of layer l on run_layer_out: forward from the spectral modes in zi,
@@ -565,8 +513,8 @@ hipError_t forward_impl(bec_fno *f, int B, const float *x, float *y, bool keep, 
         if ((e = zdft(f, q, hin, f->zf, 0, 0.0f, s)) != hipSuccess) return e;
         if ((e = xydft(f, q, f->zf, f->sp[l], 0, s)) != hipSuccess) return e;
         const unsigned short *El = f->E + (long)l * modes * 4 * W * W;
-        if (B == 1 && 2 * W == 64) {
-            if ((e = mode_mix_row(f, f->sp[l], El, f->tm, 2 * W, mm, modes, s)) != hipSuccess) return e;
+        if (mode_covers(W)) {
+            if ((e = mode_mix(f, q, l, f->sp[l], nullptr, f->tm, s)) != hipSuccess) return e;
         } else if ((e = G(f, f->sp[l], 0, El, 1, f->tm, B, 2 * W, 2 * W, mm.row, mm.ch, m1(2 * W), m1(1), mm.row,
                           mm.ch, (int)modes, mm.batch, m1(4L * W * W), mm.batch, 0.0f, nullptr, 1, nullptr, s)) !=
                    hipSuccess)
@@ -636,17 +584,21 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
         // spectral path, adjoint order
         if ((e = zdft(f, q, du, f->zi, 0, 0.0f, s)) != hipSuccess) return e;          // dZi = Fz du
         if ((e = xydft(f, q, f->zi, f->tm, 0, s)) != hipSuccess) return e;            // dT = Fxy dZi
-        const unsigned short *El = f->E + (long)l * modes * 4 * W * W;
-        // dE[t] = Sp[t]^T dT[t]  (K = batch)
-        if ((e = G(f, f->sp[l], 0, f->tm, 0, f->dE, 2 * W, 2 * W, B, mm.ch, mm.row, mm.row, mm.ch, m1(2 * W), m1(1),
-                   (int)modes, mm.batch, mm.batch, m1(4L * W * W), 0.0f, nullptr, 1, nullptr, s)) != hipSuccess)
-            return e;
-        hipLaunchKernelGGL(fold_modes, grid1(modes * W * W), dim3(256), 0, s, f->dE, g + f->oR[l], W, modes);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        // dSp = dT E^T
-        if ((e = G(f, f->tm, 0, El, 1, f->zf, B, 2 * W, 2 * W, mm.row, mm.ch, m1(1), m1(2 * W), mm.row, mm.ch,
-                   (int)modes, mm.batch, m1(4L * W * W), mm.batch, 0.0f, nullptr, 1, nullptr, s)) != hipSuccess)
-            return e;
+        if (mode_covers(W)) {
+            if ((e = mode_mix(f, q, l, f->sp[l], f->tm, f->zf, s)) != hipSuccess) return e;   // dSp, dR
+        } else {
+            const unsigned short *El = f->E + (long)l * modes * 4 * W * W;
+            // dE[t] = Sp[t]^T dT[t]  (K = batch)
+            if ((e = G(f, f->sp[l], 0, f->tm, 0, f->dE, 2 * W, 2 * W, B, mm.ch, mm.row, mm.row, mm.ch, m1(2 * W), m1(1),
+                       (int)modes, mm.batch, mm.batch, m1(4L * W * W), 0.0f, nullptr, 1, nullptr, s)) != hipSuccess)
+                return e;
+            hipLaunchKernelGGL(fold_modes, grid1(modes * W * W), dim3(256), 0, s, f->dE, g + f->oR[l], W, modes);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+            // dSp = dT E^T
+            if ((e = G(f, f->tm, 0, El, 1, f->zf, B, 2 * W, 2 * W, mm.row, mm.ch, m1(1), m1(2 * W), mm.row, mm.ch,
+                       (int)modes, mm.batch, m1(4L * W * W), mm.batch, 0.0f, nullptr, 1, nullptr, s)) != hipSuccess)
+                return e;
+        }
         if ((e = xydft(f, q, f->zf, f->zi, 1, s)) != hipSuccess) return e;            // dZf = Fxy^T dSp
         if (fused)
             e = layer_out(f, q, du, l, l > 0 ? f->u[l - 1] : nullptr, dhin, nullptr, 1, s);   // dh = du W^T + Fz^T dZf
@@ -764,7 +716,7 @@ int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
     FA(f->grads, fb * f->n_params);
     FA(f->adam_m, fb * f->n_params);
     FA(f->adam_v, fb * f->n_params);
-    FA(f->E, sizeof(unsigned short) * L * f->modes * 4 * W * W);
+    if (!bec::mode_covers(W)) FA(f->E, sizeof(unsigned short) * L * f->modes * 4 * W * W);
     FA(f->Fz, fb * 2 * c.mz * c.nz);
     FA(f->Fxy, fb * 4 * f->mxy * f->P);
     FA(f->FxyB, sizeof(unsigned short) * 4 * f->mxy * f->P);
@@ -789,7 +741,7 @@ int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
     FA(f->dA, fb * rows * W);
     FA(f->dH, fb * rows * W);
     FA(f->dB, fb * rows * c.hidden);
-    FA(f->dE, fb * f->modes * 4 * W * W);
+    if (!bec::mode_covers(W)) FA(f->dE, fb * f->modes * 4 * W * W);
     long mn = std::max(std::max((long)c.c_in * W, W * W), std::max(W * (long)c.hidden, (long)c.hidden * c.c_out));
     mn += std::max({W, (long)c.hidden, (long)c.c_out});   // weights and biases of a layer
     // split-K partials: the weight gradients (KSPLIT of at most mn) and the

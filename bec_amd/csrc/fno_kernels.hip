@@ -600,6 +600,259 @@ __global__ __launch_bounds__(256) void project_back_kernel(const float *__restri
     }
 }
 
+// Where the values of mode t lie: the real channels of sample b at
+// b * sample + t's offset, the imaginary ones `part` floats behind.
+struct ModeAt {
+    long base, part;
+};
+__device__ __forceinline__ ModeAt mode_at(long t, long mxy, int W)
+{
+    return {(t / mxy * 2 * mxy + t % mxy) * W, mxy * W};
+}
+
+// Eight samples from b0 on of V channels of one part, as V operands whose K is the sample.
+template <int V>
+__device__ __forceinline__ void sample_operands(const float *A, long sample, int b0, int B, bf16x8_t (&out)[V])
+{
+    using vec = typename VecF<V>::type;
+    vec v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        vec z;
+#pragma unroll
+        for (int j = 0; j < V; ++j) z[j] = 0.f;
+        v[k] = b0 + k < B ? *(const vec *)(A + (b0 + k) * sample) : z;
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j)
+        out[j] = to_bf16x8((f32x8_t){v[0][j], v[1][j], v[2][j], v[3][j], v[4][j], v[5][j], v[6][j], v[7][j]});
+}
+
+// The operand of a product over 2 W channels of sample b (K tile i of 32).
+template <int V>
+__device__ __forceinline__ bf16x8_t channel_operand(const float *A, long sample, const ModeAt &m, int b, int B, int k)
+{
+    f32x8_t v = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (b < B) {
+        const float *r = A + b * sample + m.base + (k < 16 * V ? k : m.part + k - 16 * V);
+        const f32x4_t lo = *(const f32x4_t *)r, hi = *(const f32x4_t *)(r + 4);
+        v = (f32x8_t){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    return to_bf16x8(v);
+}
+
+// C = A (re + i im) for the 2 W channels of 16 samples at a time, given the
+// products' operands: re[i][j], im[i][j] of K tile i (of the W input channels;
+// with W = 16 one tile holds both parts, already signed) and output column
+// 16 V-wide block j.  `conj` the other sign of im (the adjoint).
+template <int V, bool CONJ>
+__device__ __forceinline__ void mix_samples(const float *A, float *C, long sample, const ModeAt &m, int B,
+                                            const bf16x8_t (&re)[(V + 1) / 2][V], const bf16x8_t (&im)[(V + 1) / 2][V],
+                                            const bf16x8_t (&nim)[(V + 1) / 2][V])
+{
+    using vec = typename VecF<V>::type;
+    constexpr int T = V / 2;
+    const int lane = threadIdx.x & 63, c = lane & 15, kq = (lane >> 4) * 8;
+    for (int b0 = 0; b0 < B; b0 += 16) {
+        f32x4_t acc[2][V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[0][j] = acc[1][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const bf16x8_t a = channel_operand<V>(A, sample, m, b0 + c, B, i * 32 + kq);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                if (V == 1 || i < T) {
+                    acc[0][j] = mfma(a, re[i][j], acc[0][j]);
+                    acc[1][j] = mfma(a, V > 1 && CONJ ? nim[i][j] : im[i][j], acc[1][j]);
+                } else {
+                    acc[0][j] = mfma(a, CONJ ? im[i - T][j] : nim[i - T][j], acc[0][j]);
+                    acc[1][j] = mfma(a, re[i - T][j], acc[1][j]);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int b = b0 + 4 * (lane >> 4) + q;
+            if (b < B)
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    vec v;
+#pragma unroll
+                    for (int j = 0; j < V; ++j) v[j] = acc[r][j][q];
+                    *(vec *)(C + b * sample + m.base + r * m.part + c * V) = v;
+                }
+        }
+    }
+}
+
+// The channel mixing of every retained mode, C[b][t] = A[b][t] R[t] (complex):
+// bound by memory (R is read once, 33 MB per layer at width 32 and 4096 modes).
+// One wavefront per mode holds R[t] in registers as BF16 operands, read straight
+// from the FP32 parameters in whole rows; as a GEMM over the expanded real
+// matrices it took 31 us at batch 16 and the matrices another 16 us per change
+// of the parameters.
+template <int V>
+__global__ __launch_bounds__(256) void mode_mix_kernel(const float *__restrict__ A, const float *__restrict__ R,
+                                                       float *__restrict__ C, long mxy, long sample, int B, long modes)
+{
+    constexpr int W = 16 * V, I = (V + 1) / 2;
+    typedef float vec2 __attribute__((ext_vector_type(2 * V)));
+    const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= modes) return;
+    const int lane = threadIdx.x & 63, c = lane & 15, kq = (lane >> 4) * 8;
+    const bool second = V == 1 && kq >= W;   // width 16: these lanes' K is the imaginary part
+    const float *r = R + t * (2 * W * W) + c * 2 * V;
+    bf16x8_t re[I][V], im[I][V], nim[I][V];
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+        vec2 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = *(const vec2 *)(r + (i * 32 + (kq & (V == 1 ? 15 : 31)) + k) * 2 * W);
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            f32x8_t x, y;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                x[k] = second ? -v[k][2 * j + 1] : v[k][2 * j];
+                y[k] = second ? v[k][2 * j] : v[k][2 * j + 1];
+            }
+            re[i][j] = to_bf16x8(x);
+            im[i][j] = to_bf16x8(y);
+            nim[i][j] = to_bf16x8(-y);
+        }
+    }
+    mix_samples<V, false>(A, C, sample, mode_at(t, mxy, W), B, re, im, nim);
+}
+
+// Its gradient, per mode: dA = dC conj(R)^T and dR = A^T-products of A and dC
+// over the samples (re: AreDre + AimDim, im: AreDim - AimDre), in one pass over
+// R, A and dC.  As two GEMMs and a fold of the four real products: 35 + 16 + 31 us.
+template <int V>
+__global__ __launch_bounds__(256) void mode_back_kernel(const float *__restrict__ A, const float *__restrict__ D,
+                                                        const float *__restrict__ R, float *__restrict__ dA,
+                                                        float *__restrict__ dR, long mxy, long sample, int B, long modes)
+{
+    constexpr int W = 16 * V, I = (V + 1) / 2, JS = V < 2 ? V : 2;
+    const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= modes) return;
+    const int lane = threadIdx.x & 63, c = lane & 15, kq = (lane >> 4) * 8;
+    const bool second = V == 1 && kq >= W;
+    const ModeAt m = mode_at(t, mxy, W);
+    {
+        bf16x8_t re[I][V], im[I][V], nim[I][V];
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const float *r = R + t * (2 * W * W) + (c * V + j) * 2 * W + (i * 32 + (kq & (V == 1 ? 15 : 31))) * 2;
+                f32x8_t x, y;
+#pragma unroll
+                for (int k = 0; k < 8; k += 2) {
+                    const f32x4_t v = *(const f32x4_t *)(r + 2 * k);
+                    x[k] = second ? v[1] : v[0];
+                    y[k] = second ? v[0] : -v[1];
+                    x[k + 1] = second ? v[3] : v[2];
+                    y[k + 1] = second ? v[2] : -v[3];
+                }
+                re[i][j] = to_bf16x8(x);
+                nim[i][j] = to_bf16x8(y);
+                im[i][j] = V == 1 ? nim[i][j] : to_bf16x8(-y);
+            }
+        mix_samples<V, true>(D, dA, sample, m, B, re, im, nim);
+    }
+    for (int jb = 0; jb < V; jb += JS) {
+        typedef float vecj __attribute__((ext_vector_type(2 * JS)));
+        f32x4_t acc[4][V][JS];   // re re, im im, re im, im re
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+#pragma unroll
+                for (int j = 0; j < JS; ++j) acc[p][i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        for (int b0 = 0; b0 < B; b0 += 32) {
+            bf16x8_t ar[V], ai[V], dr[JS], di[JS];
+            const float *a = A + m.base + c * V, *d = D + m.base + c * V + jb;
+            sample_operands<V>(a, sample, b0 + kq, B, ar);
+            sample_operands<V>(a + m.part, sample, b0 + kq, B, ai);
+            sample_operands<JS>(d, sample, b0 + kq, B, dr);
+            sample_operands<JS>(d + m.part, sample, b0 + kq, B, di);
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+#pragma unroll
+                for (int j = 0; j < JS; ++j) {
+                    acc[0][i][j] = mfma(ar[i], dr[j], acc[0][i][j]);
+                    acc[1][i][j] = mfma(ai[i], di[j], acc[1][i][j]);
+                    acc[2][i][j] = mfma(ar[i], di[j], acc[2][i][j]);
+                    acc[3][i][j] = mfma(ai[i], dr[j], acc[3][i][j]);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                vecj v;
+#pragma unroll
+                for (int j = 0; j < JS; ++j) {
+                    v[2 * j] = acc[0][i][j][q] + acc[1][i][j][q];
+                    v[2 * j + 1] = acc[2][i][j][q] - acc[3][i][j][q];
+                }
+                *(vecj *)(dR + t * (2 * W * W) + ((4 * (lane >> 4) + q) * V + i) * 2 * W + (c * V + jb) * 2) = v;
+            }
+    }
+}
+
+// The mixing for a single sample at width 32 (a product would use one row of
+// 16): one wavefront per mode, lane l owns the outputs 4 (l % 8) + i and the
+// inputs l / 8 + 8 j, so one load covers whole rows of R; the partial sums are
+// combined over the lanes in a fixed butterfly order.  Operands rounded to BF16
+// as the products round them, products exact in FP32.
+__global__ __launch_bounds__(256) void mode_row_kernel(const float *__restrict__ A, const float *__restrict__ R,
+                                                       float *__restrict__ C, long mxy, long modes)
+{
+    const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= modes) return;
+    const int lane = threadIdx.x & 63, o = 4 * (lane & 7), kp = lane >> 3;
+    const ModeAt m = mode_at(t, mxy, 32);
+    f32x8_t w[4], acc[2] = {};   // acc: re outputs, im outputs (4 each used)
+    float xr[4], xi[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float *r = R + t * 2048 + (kp + 8 * j) * 64 + 2 * o;
+        const f32x4_t lo = *(const f32x4_t *)r, hi = *(const f32x4_t *)(r + 4);
+        w[j] = __builtin_convertvector(to_bf16x8((f32x8_t){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), f32x8_t);
+        xr[j] = A[m.base + kp + 8 * j];
+        xi[j] = A[m.base + m.part + kp + 8 * j];
+    }
+    const f32x8_t x = __builtin_convertvector(
+        to_bf16x8((f32x8_t){xr[0], xr[1], xr[2], xr[3], xi[0], xi[1], xi[2], xi[3]}), f32x8_t);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[0][i] = fmaf(x[j], w[j][2 * i], acc[0][i]);
+            acc[1][i] = fmaf(x[j], w[j][2 * i + 1], acc[1][i]);
+        }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[0][i] = fmaf(x[4 + j], -w[j][2 * i + 1], acc[0][i]);
+            acc[1][i] = fmaf(x[4 + j], w[j][2 * i], acc[1][i]);
+        }
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            acc[0][i] += __shfl_xor(acc[0][i], off);
+            acc[1][i] += __shfl_xor(acc[1][i], off);
+        }
+    if (kp < 2) {
+        const f32x8_t v = acc[kp ? 1 : 0];
+        *(f32x4_t *)(C + m.base + kp * m.part + o) = (f32x4_t){v[0], v[1], v[2], v[3]};
+    }
+}
+
 // workgroups of a kernel whose wavefronts walk `tiles` tiles: eight per CU
 int row_grid(long tiles) { return (int)std::min<long>(2048, (tiles + 3) / 4); }
 
@@ -738,6 +991,35 @@ hipError_t run_project_back(const float *dy, const float *Q1, const float *Q2, c
                                dim3(256), 0, s, dy, co, Q1, Q2, g1, rows / 16, dg1, dh);
             return hipGetLastError();
         });
+    });
+}
+
+bool mode_covers(int W) { return vec_width(W); }
+
+hipError_t run_mode_mix(const float *A, const float *R, float *C, int W, long mxy, long mz, int B, hipStream_t s)
+{
+    if (!mode_covers(W)) return hipErrorInvalidValue;
+    const long modes = mz * mxy, sample = 2 * modes * W;
+    const dim3 grid((unsigned)((modes + 3) / 4));
+    if (B == 1 && W == 32) {
+        hipLaunchKernelGGL(mode_row_kernel, grid, dim3(256), 0, s, A, R, C, mxy, modes);
+        return hipGetLastError();
+    }
+    return with_blocks(W, [&](auto v) {
+        hipLaunchKernelGGL(mode_mix_kernel<decltype(v)::value>, grid, dim3(256), 0, s, A, R, C, mxy, sample, B, modes);
+        return hipGetLastError();
+    });
+}
+
+hipError_t run_mode_back(const float *A, const float *D, const float *R, float *dA, float *dR, int W, long mxy, long mz,
+                         int B, hipStream_t s)
+{
+    if (!mode_covers(W)) return hipErrorInvalidValue;
+    const long modes = mz * mxy, sample = 2 * modes * W;
+    return with_blocks(W, [&](auto v) {
+        hipLaunchKernelGGL(mode_back_kernel<decltype(v)::value>, dim3((unsigned)((modes + 3) / 4)), dim3(256), 0, s, A, D,
+                           R, dA, dR, mxy, sample, B, modes);
+        return hipGetLastError();
     });
 }
 

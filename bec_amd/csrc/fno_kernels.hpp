@@ -61,4 +61,12 @@ hipError_t run_project(const float *h, const float *Q1, const float *q1, const f
 hipError_t run_project_back(const float *dy, const float *Q1, const float *Q2, const float *g1, int W, int H, int co,
                             long rows, float *dg1, float *dh, hipStream_t s);
 
+// The channel mixing of the mz * mxy retained modes (layout [sample][mz][re, im]
+// [mxy][W]): C = A R[mode] with the FP32 parameters R[mode][W][W][re, im], and its
+// gradient dA = D conj(R)^T, dR = conj(A)^T-sums over the samples.  W 16, 32 or 64.
+bool mode_covers(int W);
+hipError_t run_mode_mix(const float *A, const float *R, float *C, int W, long mxy, long mz, int B, hipStream_t s);
+hipError_t run_mode_back(const float *A, const float *D, const float *R, float *dA, float *dR, int W, long mxy, long mz,
+                         int B, hipStream_t s);
+
 } // namespace bec

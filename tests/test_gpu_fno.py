@@ -108,3 +108,38 @@ def test_production_size_forward_matches_oracle(bec):
         err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
         print(f"batch {b}: forward rel L2 vs FP64 oracle {err:.2e}")
         assert np.abs(ref).max() > 0 and err < 1e-2
+
+
+@pytest.mark.parametrize(
+    "nz,n,mz,m,width,layers,c_in,hidden,batch",
+    [
+        (32, 8, 8, 8, 16, 2, 16, 32, 3),      # width 16: both parts of a mode in one K tile
+        (64, 8, 6, 4, 32, 2, 16, 64, 1),      # one sample, fewer plane modes than points
+        (128, 8, 16, 4, 32, 3, 16, 32, 2),
+        (32, 4, 8, 4, 32, 1, 32, 16, 33),     # more samples than one K tile, 16 in the last rows
+        (32, 8, 8, 8, 64, 1, 16, 16, 2),      # the widest network
+        (48, 6, 8, 4, 32, 2, 5, 24, 2),       # shapes that some of the fused kernels do not cover
+    ],
+)
+def test_network_shapes_match_oracle(bec, nz, n, mz, m, width, layers, c_in, hidden, batch):
+    """The fused kernels at the edges of the shapes they cover.  The bars are those of
+    the small network above: BF16 operands round at 2^-9, a dozen products deep."""
+    from bec_amd import fno as F
+    from oracle import fno_oracle as FO
+    net = F.FNO(seed=3, nz=nz, ny=n, nx=n, mz=mz, my=m, mx=m, width=width, layers=layers, c_in=c_in, c_out=2,
+                hidden=hidden, max_batch=batch)
+    ocfg = FO.Config.from_struct(net.cfg)
+    rng = np.random.default_rng(3)
+    x = rng.normal(size=(batch, nz * n * n, c_in)).astype(np.float32)
+    t = rng.normal(size=(batch, nz * n * n, 2)).astype(np.float32)
+    flat = net.get_params().astype(np.float64)
+    y = net.predict(x)
+    ref = FO.forward(ocfg, flat, _grid(x, ocfg)).reshape(y.shape)
+    assert np.linalg.norm(y - ref) < 2e-2 * np.linalg.norm(ref)
+    net.loss_backward(F.DeviceArray(x.shape, np.float32, x), F.DeviceArray(t.shape, np.float32, t), batch)
+    g = net.get_grads().astype(np.float64)
+    _, g_ref = FO.loss_and_grads(ocfg, flat, _grid(x, ocfg), _grid(t, ocfg))
+    for name, sl in _blocks(ocfg):
+        a, b = g[sl], g_ref[sl]
+        rel = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+        assert rel < 5e-2 and a @ b > 0.998 * np.linalg.norm(a) * np.linalg.norm(b), (name, rel)
