@@ -12,8 +12,9 @@ bool shape_supported(int nx, int ny, int nz)
 
 size_t elem_size(int prec) { return prec == 0 ? 8 : 16; }
 
-long xy_workgroups(const DevGroup &g, int ntraj) { return (long)ntraj * g.nz / (64 / g.nx); }
-int xy_wg_per_traj(const DevGroup &g) { return g.nz / (64 / g.nx); }
+// one slot per wavefront: 64 / nx planes in FP32, nx / 16 to a plane in FP64
+int xy_wg_per_traj(const DevGroup &g) { return g.prec ? g.nz * (g.nx / 16) : g.nz / (64 / g.nx); }
+long xy_workgroups(const DevGroup &g, int ntraj) { return (long)ntraj * xy_wg_per_traj(g); }
 
 int default_pw(int prec, int nx, int nz)
 {
@@ -305,24 +306,21 @@ hipError_t run_z_fft(const DevGroup &g, const void *in, void *out, int ntraj, in
 
 // ------------------------------------------------------------- reductions
 
-__global__ void reduce_partials_kernel(const double *__restrict__ partial, int per_traj, int ntraj,
-                                       int nsum, double *__restrict__ out)
+__global__ __launch_bounds__(64) void reduce_partials_kernel(const double *__restrict__ partial, int per_traj, int nsum,
+                                                             double *__restrict__ out)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ntraj * nsum) return;
-    int traj = i / nsum, k = i % nsum;
-    const double *p = partial + (long)traj * per_traj * nsum + k;
+    const double *p = partial + (long)(blockIdx.x / nsum) * per_traj * nsum + blockIdx.x % nsum;
     double s = 0.0;
-    for (int j = 0; j < per_traj; ++j) s += p[(long)j * nsum];
-    out[i] = s;
+    for (int j = threadIdx.x; j < per_traj; j += 64) s += p[(long)j * nsum];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 hipError_t run_reduce_partials(const double *partial, int per_traj, int ntraj, int nsum, double *out,
                                hipStream_t s)
 {
-    int n = ntraj * nsum;
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((n + 255) / 256), dim3(256), 0, s, partial, per_traj,
-                       ntraj, nsum, out);
+    hipLaunchKernelGGL(reduce_partials_kernel, dim3((unsigned)(ntraj * nsum)), dim3(64), 0, s, partial, per_traj, nsum,
+                       out);
     return hipGetLastError();
 }
 

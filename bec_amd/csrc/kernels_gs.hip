@@ -128,15 +128,17 @@ template <typename T, int N> struct OpGsNonlinIm : SkipDone {
     int rec_shift;
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return psi; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int y, int z, int traj, long, double *) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int y, int z, int traj, long, double *) const
     {
         const TrajParams &p = P[traj >> rec_shift];
         const T hdt = (T)(0.5 * p.dt_steady), g11 = (T)p.g11, scale = (T)(1.0 / (N * N));
         const int itmax = p.itmax;
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
             const T V = potential_t<T>(p, x, y, z);
-            const cpx<T> a0 = r[0][x];
+            const cpx<T> a0 = r[0][i];
             cpx<T> a = a0;
             T da = (T)0;
             for (int it = 0; it < itmax; ++it) {
@@ -144,7 +146,7 @@ template <typename T, int N> struct OpGsNonlinIm : SkipDone {
                 else da = exp(hdt * (-V - g11 * cnorm<T>(a)));
                 a = cscale<T>(a0, da);
             }
-            r[0][x] = cscale<T>(a, da * scale);
+            r[0][i] = cscale<T>(a, da * scale);
         });
     }
 };
@@ -160,14 +162,16 @@ template <typename T, int N> struct OpGsMeasureRef : SkipDone {
     int rec_shift, nz;
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return nullptr; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int y, int z, int traj, long row, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int y, int z, int traj, long row, double *s) const
     {
         const int rec = traj >> rec_shift;
         const TrajParams &p = P[rec];
         const double ezv = ez[(long)rec * nz + z];
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
-            const double ar = r[0][x].x, ai = r[0][x].y;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
+            const double ar = r[0][i].x, ai = r[0][i].y;
             const double n = ar * ar + ai * ai;
             const cpx<T> k = kcopy[row + x];
             const double e = exy[(long)rec * N * N + y * N + x] + ezv;
@@ -215,11 +219,12 @@ template <typename T, int N> struct OpGsForward : SkipDone {
     __device__ __forceinline__ bool skip(int traj) const { return (done && done[traj]) || bad; }
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return w; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int, int, int traj, long, double *) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int traj, long, double *) const
     {
         const T s = (T)(s_v / (N * N));
 #pragma unroll
-        for (int x = 0; x < N; ++x) r[0][x] = cscale<T>(r[0][x], s);
+        for (int i = 0; i < M; ++i) r[0][i] = cscale<T>(r[0][i], s);
     }
 };
 
@@ -239,23 +244,25 @@ template <typename T, int N> struct OpGsHam : SkipDone {
     long cells;
     __device__ const cpx<T> *src(int) const { return w; }
     __device__ cpx<T> *dst(int) const { return w; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int y, int z, int traj, long row, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int y, int z, int traj, long row, double *s) const
     {
         const TrajParams &p = P[traj >> rec_shift];
         const T sc = (T)scale[traj];
         const T g = (T)((pair && (traj & 1)) ? p.g22 : p.g11), g12 = (T)p.g12;
         const T scp = pair ? (T)scale[traj ^ 1] : (T)0;
         const long poff = (traj & 1) ? -cells : cells;
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
             const cpx<T> ps = cscale<T>(psi[row + x], sc);
             const T n = cnorm<T>(ps);
             const T V = potential_t<T>(p, x, y, z);
             T coup = (T)0;
             if (pair) coup = g12 * cnorm<T>(cscale<T>(psi[row + poff + x], scp));
-            const cpx<T> kp = r[0][x];
+            const cpx<T> kp = r[0][i];
             const cpx<T> h = cadd<T>(kp, cscale<T>(ps, V + g * n + coup));
-            r[0][x] = h;
+            r[0][i] = h;
             s[0] += (double)ps.x * h.x + (double)ps.y * h.y;
             s[1] += (double)n;
             s[2] += (double)ps.x * kp.x + (double)ps.y * kp.y;
@@ -291,17 +298,19 @@ template <typename T, int N> struct OpGsResid : SkipDone {
     }
     __device__ const cpx<T> *src(int) const { return w; }
     __device__ cpx<T> *dst(int) const { return w; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int, int, int traj, long row, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int traj, long row, double *s) const
     {
         const double sc = scale[traj], m = mu_v;
         const T inv = (T)(1.0 / (N * N));
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
             const cpx<T> p = psi[row + x];
-            const double rr = (double)r[0][x].x - m * sc * (double)p.x;
-            const double ri = (double)r[0][x].y - m * sc * (double)p.y;
+            const double rr = (double)r[0][i].x - m * sc * (double)p.x;
+            const double ri = (double)r[0][i].y - m * sc * (double)p.y;
             s[0] += rr * rr + ri * ri;
-            r[0][x] = mk<T>((T)rr * inv, (T)ri * inv);
+            r[0][i] = mk<T>((T)rr * inv, (T)ri * inv);
         });
     }
 };
@@ -316,14 +325,16 @@ template <typename T, int N> struct OpGsUpdate : SkipDone {
     T tau, beta;
     __device__ const cpx<T> *src(int) const { return w; }
     __device__ cpx<T> *dst(int) const { return nullptr; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int, int, int traj, long row, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int traj, long row, double *s) const
     {
         const T sc = (T)scale[traj];
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
             const cpx<T> ps = cscale<T>(psi[row + x], sc);
             const cpx<T> pv = prev[row + x];
-            const cpx<T> d = r[0][x];
+            const cpx<T> d = r[0][i];
             const cpx<T> nw = mk<T>(ps.x - tau * d.x + beta * (ps.x - pv.x), ps.y - tau * d.y + beta * (ps.y - pv.y));
             prev[row + x] = ps;
             psi[row + x] = nw;
@@ -339,10 +350,11 @@ template <typename T, int N> struct OpGsNorm : SkipDone {
     const cpx<T> *psi;
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return nullptr; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int, int, int, long, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int, long, double *s) const
     {
 #pragma unroll
-        for (int x = 0; x < N; ++x) s[0] += (double)r[0][x].x * r[0][x].x + (double)r[0][x].y * r[0][x].y;
+        for (int i = 0; i < M; ++i) s[0] += (double)r[0][i].x * r[0][i].x + (double)r[0][i].y * r[0][i].y;
     }
 };
 

@@ -76,11 +76,15 @@ template <typename T, int N, class Op, bool NT = false, int MINW = 1>
 inline hipError_t launch_xy(const DevGroup &g, const Op &op, int ntraj, double *partial, hipStream_t s,
                             int xcd = 0)
 {
-    constexpr int PPW = 64 / N;
     XyGeom geo{g.nz, (long)ntraj * g.nz, (xcd && ntraj % 8 == 0) ? 1 : 0};
-    if (geo.n_planes % PPW) return hipErrorInvalidValue;
-    dim3 grid((unsigned)(geo.n_planes / PPW)), block(64);
-    hipLaunchKernelGGL((xy_kernel<T, N, Op, NT, MINW>), grid, block, 0, s, op, geo, partial);
+    if constexpr (sizeof(T) == 8) {
+        hipLaunchKernelGGL((xy_quad_kernel<N, Op>), dim3((unsigned)geo.n_planes), dim3(4 * N), 0, s, op, geo, partial);
+    } else {
+        constexpr int PPW = 64 / N;
+        if (geo.n_planes % PPW) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((xy_kernel<T, N, Op, NT, MINW>), dim3((unsigned)(geo.n_planes / PPW)), dim3(64), 0, s, op, geo,
+                           partial);
+    }
     return hipGetLastError();
 }
 

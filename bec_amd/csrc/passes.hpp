@@ -116,7 +116,13 @@ struct XyGeom {
 //   static constexpr bool WRITE;     write the components back
 //   static constexpr int NSUM;       per-WG FP64 partial sums produced
 //   const cpx<T>* src(int c); cpx<T>* dst(int c);
-//   void apply(cpx<T> (&rows)[NC][N], int y, int z, int traj, long row_index, double* sums)
+//   void apply(cpx<T> (&rows)[NC][M], Xs xs, int y, int z, int traj, long row_index, double* sums)
+//     (the lane's M values of row y: value i is cell xs(i) of the row)
+// The lane holds its whole row.
+struct WholeRow {
+    __device__ __forceinline__ constexpr int operator()(int i) const { return i; }
+};
+
 // MINW: minimum waves per SIMD the register allocation must allow.
 // One tile (the 64/N planes blk*PPW ..) of the xy pass, by one 64-lane
 // workgroup, exchanging through `lds` (PPW * N * (N + 1) complex values).
@@ -135,6 +141,19 @@ xy_kernel(Op op, XyGeom g, double *partial)
     __shared__ cpx<T> lds[PPW * N * (N + 1)];
     const long blk = g.xcd ? xcd_remap(blockIdx.x, g.nz / PPW) : (long)blockIdx.x;
     xy_tile<T, N, Op, NT>(op, g, partial, blk, lds, threadIdx.x);
+}
+
+// One wavefront's FP64 sums into its slot of the partials.
+template <int NSUM, int K> __device__ __forceinline__ void store_sums(double *partial, long slot, const double (&sums)[K])
+{
+    const int lane = threadIdx.x & 63;
+    if constexpr (NSUM == 1) {
+        const double s = wave_sum(sums[0]);
+        if (lane == 0) partial[slot] = s;
+    } else if constexpr (NSUM > 1) {
+        const double s = wave_sums<NSUM>(sums);
+        if ((lane & 7) == 0 && lane / 8 < NSUM) partial[slot * NSUM + lane / 8] = s;
+    }
 }
 
 template <typename T, int N, class Op, bool NT>
@@ -172,17 +191,8 @@ __device__ __forceinline__ void xy_tile(const Op &op_, const XyGeom &g, double *
     double sums[Op::NSUM > 0 ? Op::NSUM : 1];
 #pragma unroll
     for (int i = 0; i < (Op::NSUM > 0 ? Op::NSUM : 1); ++i) sums[i] = 0.0;
-    op.apply(v, t, z, traj, base + (long)t * N, sums);
-
-    if constexpr (Op::NSUM > 0) {
-        if constexpr (Op::NSUM == 1) {
-            const double s = wave_sum(sums[0]);
-            if (lane == 0) partial[blk] = s;
-        } else {
-            const double s = wave_sums<Op::NSUM>(sums);
-            if ((lane & 7) == 0 && lane / 8 < Op::NSUM) partial[blk * Op::NSUM + lane / 8] = s;
-        }
-    }
+    op.apply(v, WholeRow{}, t, z, traj, base + (long)t * N, sums);
+    store_sums<Op::NSUM>(partial, blk, sums);
 
     if constexpr (Op::WRITE) {
 #pragma unroll
@@ -196,6 +206,167 @@ __device__ __forceinline__ void xy_tile(const Op &op_, const XyGeom &g, double *
             cpx<T> *d = op.dst(c);
 #pragma unroll
             for (int y = 0; y < N; ++y) st<NT, T>(d + base + y * N + t, v[c][y]);
+        }
+    }
+}
+
+// ------------------------------------------------------- FP64 xy-plane pass
+// In FP64 a whole row per lane costs 128 registers a component at 32 points, and
+// a plane of 16 fills a quarter of a wavefront: one or two wavefronts per SIMD,
+// and 32 wavefronts for one state.  Here four lanes share a line.  Lane (t, q),
+// t the line, q = 0..3 (16 lanes apart), carries N/4 of its values in one of two
+// forms: "strided", n = q + 4 j, or "blocked", n = q N/16 + i + m N/4.  A
+// transform from strided to blocked is an N/4-point one in registers, twiddles, a
+// 4 x 4 transposition among the four lanes by lane swaps and a 4-point one; from
+// blocked to strided the same steps backwards.  Rows and columns change through
+// LDS as in xy_tile.  A plane of 16 is one wavefront, one of 32 two.
+// Measured on the real-time step of 16 trajectories of 128x32x32: 106 -> 46 us
+// (268 MB of state traffic and about 2000 FP64 operations per cell pair); on the
+// ground state's passes over one 128x16x16 state 7.3 -> 3.9 us.
+template <int N> struct Quad {
+    static constexpr int R = N / 4, KP = R / 4;
+    static __device__ __forceinline__ int strided(int q, int j) { return q + 4 * j; }
+    // value e = m KP + i of the blocked form
+    static __device__ __forceinline__ int blocked(int q, int e) { return q * KP + e % KP + R * (e / KP); }
+};
+
+// cos and sin of 2 pi q k / N, q < 4, k < N/4
+template <int N> struct QuadTable {
+    double v[N][2];
+    constexpr QuadTable() : v()
+    {
+        for (int q = 0; q < 4; ++q)
+            for (int k = 0; k < N / 4; ++k) {
+                v[q * (N / 4) + k][0] = ccos2pi(q * k, N);
+                v[q * (N / 4) + k][1] = csin2pi(q * k, N);
+            }
+    }
+};
+template <int N> __device__ const QuadTable<N> quad_table;
+
+// Value m of lane q <- value q of lane m, among the four lanes of a line.
+__device__ __forceinline__ void quad_transpose(double2 &a, double2 &b, double2 &c, double2 &d)
+{
+    swap32(a.x, c.x);
+    swap32(a.y, c.y);
+    swap32(b.x, d.x);
+    swap32(b.y, d.y);
+    swap16(a.x, b.x);
+    swap16(a.y, b.y);
+    swap16(c.x, d.x);
+    swap16(c.y, d.y);
+}
+
+// the line's twiddles w[k] = exp(2 pi i q k / N); SIGN the transform's
+template <int N, int SIGN> __device__ __forceinline__ void quad_twiddle(double2 (&v)[N / 4], const double2 (&w)[N / 4])
+{
+#pragma unroll
+    for (int k = 1; k < N / 4; ++k) v[k] = cmul<double>(v[k], make_double2(w[k].x, SIGN > 0 ? w[k].y : -w[k].y));
+}
+
+template <int N, int SIGN> __device__ __forceinline__ void dft_to_blocked(double2 (&v)[N / 4], const double2 (&w)[N / 4])
+{
+    constexpr int R = N / 4, KP = R / 4;
+    dft<double, R, SIGN>(v);
+    quad_twiddle<N, SIGN>(v, w);
+    double2 r[R];
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+        double2 x[4] = {v[i], v[KP + i], v[2 * KP + i], v[3 * KP + i]};
+        quad_transpose(x[0], x[1], x[2], x[3]);
+        dft<double, 4, SIGN>(x);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) r[m * KP + i] = x[m];
+    }
+#pragma unroll
+    for (int e = 0; e < R; ++e) v[e] = r[e];
+}
+
+template <int N, int SIGN> __device__ __forceinline__ void dft_to_strided(double2 (&v)[N / 4], const double2 (&w)[N / 4])
+{
+    constexpr int R = N / 4, KP = R / 4;
+    double2 r[R];
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+        double2 x[4] = {v[i], v[KP + i], v[2 * KP + i], v[3 * KP + i]};
+        dft<double, 4, SIGN>(x);
+        quad_transpose(x[0], x[1], x[2], x[3]);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) r[m * KP + i] = x[m];
+    }
+    quad_twiddle<N, SIGN>(r, w);
+    dft<double, R, SIGN>(r);
+#pragma unroll
+    for (int e = 0; e < R; ++e) v[e] = r[e];
+}
+
+// The lane's cells of its row (blocked form).
+template <int N> struct QuadRow {
+    int q;
+    __device__ __forceinline__ int operator()(int i) const { return Quad<N>::blocked(q, i); }
+};
+
+template <int N, class Op>
+__global__ void __launch_bounds__(4 * N) xy_quad_kernel(Op op, XyGeom g, double *partial)
+{
+    using T = double;
+    using Q = Quad<N>;
+    constexpr int R = Q::R, NC = Op::NC;
+    __shared__ double2 tile[N * (N + 1)];
+    const long plane = g.xcd ? xcd_remap(blockIdx.x, g.nz) : (long)blockIdx.x;
+    const int z = (int)(plane % g.nz), traj = (int)(plane / g.nz);
+    op.begin(traj, z == 0);
+    if (op.skip(traj)) return;   // the same for the whole workgroup
+    const int q = (threadIdx.x >> 4) & 3, t = (int)(threadIdx.x & 15) + 16 * (int)(threadIdx.x >> 6);
+    const long base = plane * (long)(N * N);
+
+    double2 v[NC][R], w[R];
+    auto load_w = [&]() {   // reloaded behind the operator rather than held across it
+        const double *tw = quad_table<N>.v[opaque_index(q) * R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) w[k] = make_double2(tw[2 * k], tw[2 * k + 1]);
+    };
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const double2 *s = op.src(c);
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[c][j] = s[base + Q::strided(q, j) * N + t];
+    }
+    load_w();
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if constexpr (Op::SIGN_IN != 0) dft_to_blocked<N, Op::SIGN_IN>(v[c], w);
+#pragma unroll
+        for (int j = 0; j < R; ++j) tile[(Op::SIGN_IN ? Q::blocked(q, j) : Q::strided(q, j)) * (N + 1) + t] = v[c][j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[c][j] = tile[t * (N + 1) + (Op::SIGN_IN ? Q::strided(q, j) : Q::blocked(q, j))];
+        __syncthreads();
+        if constexpr (Op::SIGN_IN != 0) dft_to_blocked<N, Op::SIGN_IN>(v[c], w);
+    }
+
+    double sums[Op::NSUM > 0 ? Op::NSUM : 1];
+#pragma unroll
+    for (int i = 0; i < (Op::NSUM > 0 ? Op::NSUM : 1); ++i) sums[i] = 0.0;
+    op.apply(v, QuadRow<N>{q}, t, z, traj, base + (long)t * N, sums);
+    store_sums<Op::NSUM>(partial, plane * (N / 16) + (threadIdx.x >> 6), sums);
+
+    if constexpr (Op::WRITE) {
+        load_w();
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if constexpr (Op::SIGN_OUT != 0) dft_to_strided<N, Op::SIGN_OUT>(v[c], w);
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+                tile[t * (N + 1) + (Op::SIGN_OUT ? Q::strided(q, j) : Q::blocked(q, j))] = v[c][j];
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < R; ++j) v[c][j] = tile[(Op::SIGN_OUT ? Q::blocked(q, j) : Q::strided(q, j)) * (N + 1) + t];
+            if (c + 1 < NC) __syncthreads();
+            if constexpr (Op::SIGN_OUT != 0) dft_to_strided<N, Op::SIGN_OUT>(v[c], w);
+            double2 *d = op.dst(c);
+#pragma unroll
+            for (int j = 0; j < R; ++j) d[base + Q::strided(q, j) * N + t] = v[c][j];
         }
     }
 }
@@ -261,7 +432,8 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
         da = cscale<T>(w1, b11);
         db = mk<T>(b21.x * w1.x - b21.y * w1.y + b22 * w2.x, b21.x * w1.y + b21.y * w1.x + b22 * w2.y);
     }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[2][N], int y, int z, int traj, long, double *) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[2][M], Xs xs, int y, int z, int traj, long, double *) const
     {
         const TrajParams &p = P[traj >> rec_shift];
         const T half_dt = (T)(0.5 * p.dt);
@@ -280,14 +452,14 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
             ws = (T)(sqrt(p.dt / (2.0 * p.dx * p.dy * p.dz)) / (N * N));
         }
         const uint32_t cell0 = (uint32_t)((z * N + y) * N);
-        auto add_noise = [&](int x, cpx<T> a0, cpx<T> b0) {
+        auto add_noise = [&](int i, int x, cpx<T> a0, cpx<T> b0) {
             if constexpr (NOISE) {
                 T zn[4];
                 loss_noise4<T>(cell0 + (uint32_t)x, (uint32_t)traj, st, group, k0, k1, zn);
                 cpx<T> da, db;
                 loss_increment(l111, l12, l22, a0, b0, zn, ws, da, db);
-                r[0][x] = mk<T>(r[0][x].x + da.x, r[0][x].y + da.y);
-                r[1][x] = mk<T>(r[1][x].x + db.x, r[1][x].y + db.y);
+                r[0][i] = mk<T>(r[0][i].x + da.x, r[0][i].y + da.y);
+                r[1][i] = mk<T>(r[1][i].x + db.x, r[1][i].y + db.y);
             }
         };
         if constexpr (IT1) {
@@ -298,36 +470,45 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
             const T g11d = (T)(p.g11 * dt), g12d = (T)(p.g12 * dt), g22d = (T)(p.g22 * dt);
             const T n111 = (T)(-0.5 * p.l111 * dt), n12 = (T)(-0.5 * p.l12 * dt), n22 = (T)(-0.5 * p.l22 * dt);
             const T detd = (T)(p.detuning * dt);
-            static_for<0, N>([&](auto X_) {
-                constexpr int x = decltype(X_)::value;
+            static_for<0, M>([&](auto X_) {
+                constexpr int i = decltype(X_)::value;
+                const int x = xs(i);
                 const T xx = (T)(-p.xmax) + (T)p.dx * (T)x;
                 const T Vd = half_dt * fma_t(xx, xx, vyz);     // V dt
-                const cpx<T> a0 = r[0][x], b0 = r[1][x];
+                const cpx<T> a0 = r[0][i], b0 = r[1][i];
                 const T na = cnorm<T>(a0), nb = cnorm<T>(b0);
                 const T pha = fma_t(g11d, na, fma_t(g12d, nb, Vd));
                 const T phb = fma_t(g22d, nb, fma_t(g12d, na, Vd - detd));
                 const T ya = fma_t(n111, na * na, n12 * nb);
                 const T yb = fma_t(n22, nb, n12 * na);
                 T sa, ca, sb, cb;
-                sincos2_scaled_t(pha, scale, &sa, &ca);
-                sincos2_scaled_t(phb, scale, &sb, &cb);
+                if constexpr (sizeof(T) == 4) {
+                    sincos2_scaled_t(pha, scale, &sa, &ca);
+                    sincos2_scaled_t(phb, scale, &sb, &cb);
+                } else {
+                    sincos_pair(pha, phb, &sa, &ca, &sb, &cb);
+                    sa *= scale, ca *= scale, sb *= scale, cb *= scale;
+                }
                 const T ta = expm1_small_t(ya), tb = expm1_small_t(yb);
                 const cpx<T> va = cmul<T>(a0, mk<T>(ca, sa));
                 const cpx<T> vb = cmul<T>(b0, mk<T>(cb, sb));
-                r[0][x] = mk<T>(fma_t(va.x, ta, va.x), fma_t(va.y, ta, va.y));
-                r[1][x] = mk<T>(fma_t(vb.x, tb, vb.x), fma_t(vb.y, tb, vb.y));
-                add_noise(x, a0, b0);
+                r[0][i] = mk<T>(fma_t(va.x, ta, va.x), fma_t(va.y, ta, va.y));
+                r[1][i] = mk<T>(fma_t(vb.x, tb, vb.x), fma_t(vb.y, tb, vb.y));
+                add_noise(i, x, a0, b0);
+                // one cell after the other in FP64: half the registers
+                if constexpr (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
             });
             return;
         }
         // itmax = 0 never forms the factor: the output is zero, as the reference's
         // uninitialised factor (quirk Q10) and the oracle give
         const T scale_out = itmax > 0 ? scale : (T)0;
-        static_for<0, N>([&](auto X_) {
-            constexpr int x = decltype(X_)::value;
+        static_for<0, M>([&](auto X_) {
+            constexpr int i = decltype(X_)::value;
+            const int x = xs(i);
             const T xx = (T)(-p.xmax) + (T)p.dx * (T)x;
             const T V = (T)0.5 * (xx * xx + vyz);
-            const cpx<T> a0 = r[0][x], b0 = r[1][x];
+            const cpx<T> a0 = r[0][i], b0 = r[1][i];
             // d = m e^{i phi}; the output psi0 d^2 = psi0 e^{2 i phi} (1 + t) with
             // t = m^2 - 1 = expm1(2 Re(p) dt/2) formed directly, so that the small
             // loss increments (|t| ~ 1e-6 per step) keep full relative precision
@@ -354,9 +535,10 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
             }
             const cpx<T> va = cscale<T>(cmul<T>(a0, cmul<T>(ea, ea)), scale_out);
             const cpx<T> vb = cscale<T>(cmul<T>(b0, cmul<T>(eb, eb)), scale_out);
-            r[0][x] = mk<T>(fma_t(va.x, ta, va.x), fma_t(va.y, ta, va.y));
-            r[1][x] = mk<T>(fma_t(vb.x, tb, vb.x), fma_t(vb.y, tb, vb.y));
-            add_noise(x, a0, b0);
+            r[0][i] = mk<T>(fma_t(va.x, ta, va.x), fma_t(va.y, ta, va.y));
+            r[1][i] = mk<T>(fma_t(vb.x, tb, vb.x), fma_t(vb.y, tb, vb.y));
+            add_noise(i, x, a0, b0);
+            if constexpr (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
         });
     }
     // The IT1 step of one component c (0: a, 1: b) of a row, given the other
@@ -393,14 +575,19 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
     }
     // S sin x and S cos x of the doubled phase (IT1 path), S a power of two (the
     // 1/N^2 of the xy transform pair): exactly the rounded sin and cos times S
-    static __device__ __forceinline__ void sincos2_scaled_t(T x, T S, T *s, T *c)
+    static __device__ __forceinline__ void sincos2_scaled_t(float x, float S, float *s, float *c)
     {
-        if constexpr (sizeof(T) == 4) {
-            fast_sincos_pi_scaled(x, S, s, c);
+        fast_sincos_pi_scaled(x, S, s, c);
+    }
+    // both components' sines and cosines; the library's beyond the fast range
+    static __device__ __forceinline__ void sincos_pair(double x, double y, double *sx, double *cx, double *sy, double *cy)
+    {
+        if (__builtin_expect(fmax(fabs(x), fabs(y)) < DSINCOS_MAX, 1)) {
+            fast_sincos_f64(x, sx, cx);
+            fast_sincos_f64(y, sy, cy);
         } else {
-            sincos(x, s, c);
-            *s *= S;
-            *c *= S;
+            sincos(x, sx, cx);
+            sincos(y, sy, cy);
         }
     }
     // expm1 for the IT1 path: a cubic (relative truncation error y^3/24 <
@@ -417,7 +604,15 @@ template <typename T, int N, bool IT1 = true, bool NOISE = false> struct OpNonli
             if (__any(big)) t = big ? __expf(y) - 1.0f : t;
             return t;
         } else {
-            return expm1(y);
+            // to y^6: relative truncation error y^6 / 5040 < 8e-19
+            double p = fma(y, 1.0 / 720.0, 1.0 / 120.0);
+            p = fma(y, p, 1.0 / 24.0);
+            p = fma(y, p, 1.0 / 6.0);
+            p = fma(y, p, 0.5);
+            p = fma(y * y, p, y);
+            const bool big = !(fabs(y) < 0.00390625);
+            if (__any(big)) p = big ? expm1(y) : p;
+            return p;
         }
     }
     // expm1: a degree-4 Taylor polynomial for |y| < 1/64 (truncation error
@@ -509,9 +704,10 @@ template <typename T, int N> struct OpSample : NoSkip {
     const cpx<T> *a, *b;
     __device__ const cpx<T> *src(int c) const { return c == 0 ? a : b; }
     __device__ cpx<T> *dst(int) const { return nullptr; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[2][N], int, int, int, long, double *s) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[2][M], Xs, int, int, int, long, double *s) const
     {
-        static_for<0, N>([&](auto X_) {
+        static_for<0, M>([&](auto X_) {
             constexpr int x = decltype(X_)::value;
             const double ar = r[0][x].x, ai = r[0][x].y, br = r[1][x].x, bi = r[1][x].y;
             s[0] += ar * ar + ai * ai;
@@ -531,11 +727,12 @@ template <typename T, int N, int SIGN> struct OpFftXY : NoSkip {
     T scale;
     __device__ const cpx<T> *src(int) const { return in; }
     __device__ cpx<T> *dst(int) const { return out; }
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][N], int, int, int, long, double *) const
+    template <int M, class Xs>
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs, int, int, int, long, double *) const
     {
         if (scale != (T)1)
 #pragma unroll
-            for (int x = 0; x < N; ++x) r[0][x] = cscale<T>(r[0][x], scale);
+            for (int x = 0; x < M; ++x) r[0][x] = cscale<T>(r[0][x], scale);
     }
 };
 

@@ -345,3 +345,24 @@ def test_projections_of_every_split_equal_the_states_sums(bec, prec, nxy, nz, ne
         assert rel_l2(p["xy_" + k], d.sum(axis=0)) < 1e-9
         assert rel_l2(p["zy_" + k], d.sum(axis=2).T) < 1e-9
         assert rel_l2(p["axial_" + k], d.sum(axis=(1, 2))) < 1e-9
+
+
+@pytest.mark.parametrize("itmax", [1, 2])
+@pytest.mark.parametrize("nz,n,ne", [(64, 16, 1), (128, 16, 3), (256, 16, 2), (64, 32, 3), (256, 32, 1)])
+def test_fp64_planes_match_oracle(bec, oracle, nz, n, ne, itmax):
+    """The FP64 plane pass (four lanes to a line) on every plane size, with odd counts of
+    trajectories and both forms of the nonlinear step, and its sampled sums."""
+    c, oc = _pair(bec, oracle, 1, ne=ne, nvx=n, nvy=n, nvz=nz, itmax=itmax)
+    rng = np.random.default_rng(nz + n)
+    start = 5.0 * (rng.normal(size=(nz, n, n)) + 1j * rng.normal(size=(nz, n, n)))
+    with bec.Solver(c, precision=1) as s:
+        s.init_evolution(start, SEED, equilibrate=False)
+        sums = s.propagate(3, sample_every=3)
+        ax, bx = s.get_state(bec.SPACE_X)
+    oa, ob = oracle.init_evolution(oc, start, SEED, equilibrate=False)
+    oa, ob = oracle.propagate(oc, oa, ob, oc.dt_evo, 3)
+    assert rel_l2(ax, oracle.to_xspace(oc, oa), axis=(1, 2, 3)).max() < 1e-11
+    assert rel_l2(bx, oracle.to_xspace(oc, ob), axis=(1, 2, 3)).max() < 1e-11
+    got = np.asarray(sums).reshape(-1, ne, 4)[-1]
+    np.testing.assert_allclose(got[:, 0], (np.abs(ax) ** 2).sum(axis=(1, 2, 3)), rtol=1e-12)
+    np.testing.assert_allclose(got[:, 1], (np.abs(bx) ** 2).sum(axis=(1, 2, 3)), rtol=1e-12)
