@@ -18,7 +18,7 @@ namespace {
 
 struct GsWork {
     Group g;
-    void *X = nullptr, *W = nullptr, *P = nullptr, *KC = nullptr;
+    void *X = nullptr, *W = nullptr, *P = nullptr, *KC = nullptr, *Q = nullptr;
     double *ph = nullptr, *pr = nullptr, *pm = nullptr, *pn = nullptr;
     double *sums = nullptr;        // [batch][8] reduced sums
     double *exy = nullptr, *ez = nullptr, *mu_tf = nullptr, *ones = nullptr;
@@ -183,35 +183,42 @@ hipError_t residual_pass(GsWork &w, const GsScalars &sc, double tol, int check, 
     return gs_scalar_residual(d, w.ph, w.pr, sc, tol, check, s);
 }
 
-int split_step_iteration(GsWork &w, const bec_gs_options &o, int it, hipStream_t s)
+// One split-step iteration in three launches: the x-space step (on Q, where the
+// previous z pass left the state half a kinetic step ahead), the z pass that ends
+// this iteration in P and begins the next in Q, and the energy integral.  Its
+// test and renormalisation run inside the next x-space step (*pending: they are
+// still to do), so nothing waits on a launch of its own: five launches before,
+// each about 2 us behind the other for a state that fills few CUs.
+int split_step_iteration(GsWork &w, const bec_gs_options &o, int it, bool *pending, hipStream_t s)
 {
     const DevGroup &d = w.g.dev;
-    GsScalars once = w.sc;
-    once.s = w.ones;
+    const int rule = o.rule == BEC_GS_RULE_REFERENCE;
     GsTables t{w.exy, w.ez};
-    GS_HIP(gs_z_imag(d, w.P, w.sc, nullptr, s));          // K/2 with the pending renormalisation
-    GS_HIP(gs_xy_nonlinear_imag(d, w.P, w.sc, s));        // x-space step
-    GS_HIP(gs_z_imag(d, w.P, once, w.KC, s));             // K/2, keep psi_k for the energy integral
+    GS_HIP(gs_xy_nonlinear_imag(d, w.Q, w.sc, s, *pending ? w.pm : nullptr, o.tol, rule));
+    GS_HIP(gs_z_step(d, w.Q, w.P, w.KC, w.sc, s));
     GS_HIP(gs_xy_measure_ref(d, w.P, w.KC, w.sc, t, w.pm, s));
-    GS_HIP(gs_scalar_ref(d, w.pm, w.sc, o.tol, o.rule == BEC_GS_RULE_REFERENCE, s));
+    *pending = true;
     if (o.rule == BEC_GS_RULE_RESIDUAL && (it + 1) % std::max(1, o.check_every) == 0) {
+        GS_HIP(gs_scalar_ref(d, w.pm, w.sc, o.tol, rule, s));
+        *pending = false;
         GS_HIP(run_xy_fft(d, w.P, w.X, d.ntraj, -1, 1.0, s));
         GS_HIP(residual_pass(w, w.sc, o.tol, 1, s));
     }
     return BEC_OK;
 }
 
-// One gradient-flow iteration in six launches: the per-trajectory scalars
+// One gradient-flow iteration in five launches: the per-trajectory scalars
 // (mu, the residual test, the renormalisation of the previous update) are
 // evaluated inside the passes that consume them.  Iteration 0 starts from
-// the normalised guess; later ones renormalise the previous update first.
+// the normalised guess; later ones from the transform the previous update left
+// in W, which they renormalise.
 int gradient_iteration(GsWork &w, const bec_gs_options &o, int it, double alpha, hipStream_t s)
 {
     const DevGroup &d = w.g.dev;
     GsTables t{w.exy, w.ez};
     const int check = o.rule == BEC_GS_RULE_RESIDUAL && (it % std::max(1, o.check_every) == 0);
-    GS_HIP(gs_xy_forward(d, w.X, w.W, w.sc, s, it > 0 ? w.pn : nullptr));
-    GS_HIP(gs_z_diag(d, w.W, w.sc, t, 0, 0.0, nullptr, s));
+    if (it == 0) GS_HIP(gs_xy_forward(d, w.X, w.W, w.sc, s));
+    GS_HIP(gs_z_diag(d, w.W, w.sc, t, 0, 0.0, nullptr, s, nullptr, it > 0 ? w.pn : nullptr));
     GS_HIP(gs_xy_hamiltonian(d, w.X, w.W, w.sc, w.ph, s));
     GS_HIP(gs_xy_residual(d, w.X, w.W, w.sc, w.pr, s, w.ph));
     // preconditioner shift: the option, else each record's Thomas-Fermi mu
@@ -356,6 +363,8 @@ int gs_solve(const bec_calc_params *params, int batch, const double *guesses, co
     if (o.method == BEC_GS_SPLIT_STEP) {
         GS_HIP(gs_xy_forward(d, w.X, w.P, w.sc, s));     // x -> hybrid, renormalised
         GS_HIP(gs_apply_scale(d, w.X, w.sc, s));          // keeps X consistent, s <- 1
+        GS_HIP(w.alloc(&w.Q, elem_size(o.precision) * n));
+        GS_HIP(gs_z_imag(d, w.P, w.Q, w.sc, s));          // the first half step
     } else {
         GS_HIP(gs_apply_scale(d, w.X, w.sc, s));
         GS_HIP(hipMemcpyAsync(w.P, w.X, elem_size(o.precision) * n, hipMemcpyDeviceToDevice, s));
@@ -366,15 +375,18 @@ int gs_solve(const bec_calc_params *params, int batch, const double *guesses, co
     GS_HIP(hipEventRecord(e0, s));
     std::vector<int> done(ntraj, 0);
     int it = 0;
+    bool pending = false;
     const int block = 16;
     while (it < o.max_iter) {
         const int nb = std::min(block, o.max_iter - it);
         for (int j = 0; j < nb; ++j, ++it) {
-            st = o.method == BEC_GS_SPLIT_STEP ? split_step_iteration(w, o, it, s)
+            st = o.method == BEC_GS_SPLIT_STEP ? split_step_iteration(w, o, it, &pending, s)
                                                : gradient_iteration(w, o, it, alpha, s);
             if (st != BEC_OK) break;
         }
         if (st != BEC_OK) break;
+        if (pending) GS_HIP(gs_scalar_ref(d, w.pm, w.sc, o.tol, o.rule == BEC_GS_RULE_REFERENCE, s));
+        pending = false;
         GS_HIP(hipMemcpyAsync(done.data(), w.sc.done, sizeof(int) * ntraj, hipMemcpyDeviceToHost, s));
         GS_HIP(hipStreamSynchronize(s));
         if (std::all_of(done.begin(), done.end(), [](int v) { return v != 0; })) break;

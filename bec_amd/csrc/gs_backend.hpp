@@ -25,10 +25,15 @@ struct GsTables {
 };
 
 // ---- split step (calculateSteadyState, wigner.cu:84-175)
-// z-pass with the imaginary-time half step (and the pending scale); when
-// kcopy != nullptr it also stores the normalised k-space values.
-hipError_t gs_z_imag(const DevGroup &g, void *psi, const GsScalars &sc, void *kcopy, hipStream_t s);
-hipError_t gs_xy_nonlinear_imag(const DevGroup &g, void *psi, const GsScalars &sc, hipStream_t s);
+// z-pass with the imaginary-time half step, in -> out
+hipError_t gs_z_imag(const DevGroup &g, const void *in, void *out, const GsScalars &sc, hipStream_t s);
+// two half steps of q: the k-space values after the first to kcopy (normalised),
+// transformed back to psi; after the second transformed back to q.  e_prev <- e_ref.
+hipError_t gs_z_step(const DevGroup &g, void *q, void *psi, void *kcopy, const GsScalars &sc, hipStream_t s);
+// x-space step on psi times sc.s; pm != nullptr: first the work of gs_scalar_ref on
+// the previous iteration's partials
+hipError_t gs_xy_nonlinear_imag(const DevGroup &g, void *psi, const GsScalars &sc, hipStream_t s,
+                                const double *pm = nullptr, double tol = 0.0, int use_rule = 0);
 // partials: {sum n, sum n V, sum n^2, sum Re(psi_x psi_k k^2/2)} per workgroup
 hipError_t gs_xy_measure_ref(const DevGroup &g, const void *psi, const void *kcopy, const GsScalars &sc,
                              const GsTables &t, double *partial, hipStream_t s);
@@ -47,15 +52,15 @@ struct GsResidualTest {
 };
 
 // ---- gradient flow / residual machinery (x-space iterate psi)
-// pn != nullptr: first renormalise with the scale of the previous update's
-// partials (the work of gs_scalar_norm, counting the iteration)
-hipError_t gs_xy_forward(const DevGroup &g, const void *psi, void *w, const GsScalars &sc, hipStream_t s,
-                         const double *pn = nullptr);
+hipError_t gs_xy_forward(const DevGroup &g, const void *psi, void *w, const GsScalars &sc, hipStream_t s);
 // variant 0: multiply by k^2/2 / nz; 1: by 1 / ((alpha + k^2/2) nz), alpha
 // taken per record from alpha_rec when it is not nullptr; test != nullptr:
-// run the residual test first and skip the trajectories it stops
+// run the residual test first and skip the trajectories it stops; pn != nullptr
+// (variant 0): first renormalise with the scale of the previous update's partials
+// (the work of gs_scalar_norm, counting the iteration), applied to the values
 hipError_t gs_z_diag(const DevGroup &g, void *w, const GsScalars &sc, const GsTables &t, int variant,
-                     double alpha, const double *alpha_rec, hipStream_t s, const GsResidualTest *test = nullptr);
+                     double alpha, const double *alpha_rec, hipStream_t s, const GsResidualTest *test = nullptr,
+                     const double *pn = nullptr);
 // h = K psi + (V + g11 |psi|^2) psi; partials {Re<psi,h>, <psi,psi>, <psi,K psi>, sum V n, sum n^2}
 hipError_t gs_xy_hamiltonian(const DevGroup &g, const void *psi, void *w, const GsScalars &sc,
                              double *partial, hipStream_t s);
@@ -66,8 +71,9 @@ hipError_t gs_xy_residual(const DevGroup &g, const void *psi, void *w, const GsS
                           hipStream_t s, const double *ph = nullptr);
 hipError_t gs_scalar_residual(const DevGroup &g, const double *partial_h, const double *partial_r,
                               const GsScalars &sc, double tol, int check, hipStream_t s);
-// psi_new = s psi - tau d + beta (s psi - prev); prev <- s psi; partial {|psi_new|^2}
-hipError_t gs_xy_update(const DevGroup &g, void *psi, void *prev, const void *w, const GsScalars &sc,
+// psi_new = s psi - tau d + beta (s psi - prev); prev <- s psi; partial {|psi_new|^2};
+// w (d on entry) <- F_xy(psi_new)
+hipError_t gs_xy_update(const DevGroup &g, void *psi, void *prev, void *w, const GsScalars &sc,
                         double tau, double beta, double *partial, hipStream_t s);
 hipError_t gs_scalar_norm(const DevGroup &g, const double *partial, const GsScalars &sc, hipStream_t s);
 // s <- sqrt(N0 / (dV sum |psi|^2)) of an x-space state (no iteration count)

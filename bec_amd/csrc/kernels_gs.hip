@@ -28,33 +28,97 @@ __device__ __forceinline__ double psum(const double *partial, int per, int nsum,
     return wave_sum(s);
 }
 
+// The reference's energy integral and scale of one iteration, from the four sums
+// {sum n, sum n V, sum n^2, sum Re(psi_x psi_k k^2/2)} of its measuring pass.
+struct RefEnergy {
+    double s2, E;
+    __device__ __forceinline__ int flag(double e_prev, double tol, int use_rule) const
+    {
+        if (!(E == E) || !(s2 == s2)) return 2;   // non-finite
+        return use_rule && fabs((E - e_prev) / E) < tol ? 1 : 0;
+    }
+    __device__ __forceinline__ void record(const GsScalars &sc, int traj, int flag) const
+    {
+        sc.iters[traj] += 1;
+        if (flag) sc.done[traj] = flag;
+        sc.e_ref[traj] = E;
+        sc.s[traj] = sqrt(s2);
+    }
+};
+__device__ __forceinline__ RefEnergy ref_energy(const double *partial, int per, int traj, const TrajParams &p)
+{
+    const double2 *q = (const double2 *)(partial + (long)traj * per * 4);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int j = (int)(threadIdx.x & 63); j < per; j += 64) {
+        const double2 a = q[2 * j], b = q[2 * j + 1];
+        v[0] += a.x;
+        v[1] += a.y;
+        v[2] += b.x;
+        v[3] += b.y;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = wave_sum(v[k]);
+    const double dV = dv_of(p), s2 = p.N0 / (v[0] * dV);
+    return {s2, dV * (s2 * (v[1] + v[3]) + p.g11 * s2 * s2 * v[2] / 2.0)};
+}
+
 // --------------------------------------------------------------- z-passes
 
+// psi_k *= exp(-K dt/2) between src and dst (the first half step of a solve).
 template <typename T, int NZ, int R1> struct OpGsZImag : SkipDone {
     static constexpr int NC = 1;
     static constexpr int NW = NZ / R1, KPT = R1 / NW;
-    cpx<T> *psi;
-    const cpx<T> *kxy, *kz;   // KT_IM_HALF tables [records][...]
-    const double *scale;      // per trajectory
-    cpx<T> *kcopy;
+    const cpx<T> *in;
+    cpx<T> *out;
+    const cpx<T> *kxy, *kz;   // KT_IM_HALF tables [records][...], the kz ones over NZ
     int nxy, rec_shift;
-    __device__ const cpx<T> *src(int) const { return psi; }
-    __device__ cpx<T> *dst(int) const { return psi; }
+    __device__ const cpx<T> *src(int) const { return in; }
+    __device__ cpx<T> *dst(int) const { return out; }
     __device__ __forceinline__ void kspace(int, cpx<T> (&X)[KPT][NW], int kk0, int q, int traj) const
+    {
+        half_step(X, kk0, q, traj, (T)1);
+    }
+    __device__ __forceinline__ void half_step(cpx<T> (&X)[KPT][NW], int kk0, int q, int traj, T s) const
     {
         const int rec = traj >> rec_shift;
         cpx<T> fxy = kxy[(long)rec * nxy + q];
-        const T s = (T)scale[traj];
         fxy = mk<T>(fxy.x * s, fxy.y * s);
         const cpx<T> *kzr = kz + (long)rec * NZ;
 #pragma unroll
         for (int i = 0; i < KPT; ++i)
 #pragma unroll
-            for (int m = 0; m < NW; ++m) {
-                const int kzi = kk0 + i + R1 * m;
-                X[i][m] = cmul<T>(X[i][m], cmul<T>(fxy, kzr[kzi]));
-                if (kcopy) kcopy[((long)traj * NZ + kzi) * nxy + q] = X[i][m];
-            }
+            for (int m = 0; m < NW; ++m) X[i][m] = cmul<T>(X[i][m], cmul<T>(fxy, kzr[kk0 + i + R1 * m]));
+    }
+};
+
+// The second half step of one iteration and the first of the next in one pass:
+// psi_k (kept in kcopy for the energy integral) goes back to `psi`, the state the
+// iteration ends with, and exp(-K dt/2) psi_k to `out`, where the next one begins
+// (its renormalisation, linear, is applied to the x-space step's input).  One
+// forward transform and one launch instead of two of each per iteration.
+template <typename T, int NZ, int R1> struct OpGsZStep : OpGsZImag<T, NZ, R1> {
+    using Base = OpGsZImag<T, NZ, R1>;
+    static constexpr bool TWICE = true;
+    static constexpr int NW = Base::NW, KPT = Base::KPT;
+    cpx<T> *psi, *kcopy;
+    GsScalars sc;
+    __device__ __forceinline__ void begin(int traj, bool first)
+    {
+        // the energies of the last two iterations: e_ref has been tested by now
+        if (first && threadIdx.x == 0 && !this->done[traj]) sc.e_prev[traj] = sc.e_ref[traj];
+    }
+    __device__ cpx<T> *first(int) const { return psi; }
+    __device__ __forceinline__ void kspace(int, cpx<T> (&X)[KPT][NW], int kk0, int q, int traj) const
+    {
+        this->half_step(X, kk0, q, traj, (T)1);
+#pragma unroll
+        for (int i = 0; i < KPT; ++i)
+#pragma unroll
+            for (int m = 0; m < NW; ++m) kcopy[((long)traj * NZ + kk0 + i + R1 * m) * this->nxy + q] = X[i][m];
+    }
+    __device__ __forceinline__ void again(int, cpx<T> (&X)[KPT][NW], int kk0, int q, int traj) const
+    {
+        this->half_step(X, kk0, q, traj, (T)NZ);   // NZ a power of two: undoes the table's 1/NZ exactly
     }
 };
 
@@ -87,6 +151,31 @@ struct FusedResidual {
     }
 };
 
+// Fused renormalisation (pn != nullptr): the scale of the previous update,
+// s = sqrt(N_target / (dV sum |psi|^2)), from its partials (the sums of
+// scalar_norm_kernel); the first workgroup records s and counts the iteration.
+struct FusedRenorm {
+    const double *pn = nullptr;
+    int per = 0;
+    const TrajParams *P = nullptr;
+    GsScalars sc{};
+    double s = 1.0;
+    bool bad = false;
+    __device__ __forceinline__ void run(int traj, int rec, bool first)
+    {
+        if (!pn) return;
+        const TrajParams &p = P[rec];
+        const double n = psum(pn, per, 1, traj, 0) * dv_of(p);
+        s = sqrt((sc.target ? sc.target[traj] : p.N0) / n);
+        bad = !(n == n);
+        if (first && threadIdx.x == 0) {
+            sc.s[traj] = s;
+            sc.iters[traj] += 1;
+            if (bad) sc.done[traj] = 2;
+        }
+    }
+};
+
 template <typename T, int NZ, int R1> struct OpGsZDiag : SkipDone {
     static constexpr int NC = 1;
     static constexpr int NW = NZ / R1, KPT = R1 / NW;
@@ -96,8 +185,14 @@ template <typename T, int NZ, int R1> struct OpGsZDiag : SkipDone {
     int nxy, rec_shift, variant;
     double alpha;
     FusedResidual fr;
-    __device__ __forceinline__ void begin(int traj, bool first) { fr.run(traj, first, done); }
-    __device__ __forceinline__ bool skip(int traj) const { return (done && done[traj]) || fr.stop; }
+    FusedRenorm rn;
+    __device__ __forceinline__ void begin(int traj, bool first)
+    {
+        if (done && done[traj]) return;
+        rn.run(traj, traj >> rec_shift, first);
+        fr.run(traj, first, done);
+    }
+    __device__ __forceinline__ bool skip(int traj) const { return (done && done[traj]) || fr.stop || rn.bad; }
     __device__ const cpx<T> *src(int) const { return w; }
     __device__ cpx<T> *dst(int) const { return w; }
     __device__ __forceinline__ void kspace(int, cpx<T> (&X)[KPT][NW], int kk0, int q, int traj) const
@@ -111,7 +206,7 @@ template <typename T, int NZ, int R1> struct OpGsZDiag : SkipDone {
 #pragma unroll
             for (int m = 0; m < NW; ++m) {
                 const double e = e0 + ezr[kk0 + i + R1 * m];
-                const T f = (T)(variant == 0 ? e / NZ : 1.0 / ((al + e) * NZ));
+                const T f = (T)(variant == 0 ? e / NZ * rn.s : 1.0 / ((al + e) * NZ));
                 X[i][m] = cscale<T>(X[i][m], f);
             }
     }
@@ -119,13 +214,35 @@ template <typename T, int NZ, int R1> struct OpGsZDiag : SkipDone {
 
 // -------------------------------------------------------------- xy-passes
 
-// propagateXSpaceOneComponent (wigner_kernel.cu:154-181) + 1/(NX NY)
+// propagateXSpaceOneComponent (wigner_kernel.cu:154-181) on the renormalised
+// input, + 1/(NX NY).  Fused energy test (pm != nullptr): the previous iteration's
+// scale and energy from its partials, the first workgroup recording them.
 template <typename T, int N> struct OpGsNonlinIm : SkipDone {
     static constexpr int NC = 1, SIGN_IN = -1, SIGN_OUT = +1, NSUM = 0;
     static constexpr bool WRITE = true;
     cpx<T> *psi;
     const TrajParams *P;
     int rec_shift;
+    const double *pm = nullptr;
+    int per = 0, use_rule = 0;
+    double tol = 0.0;
+    GsScalars sc{};
+    double s_v = 1.0;
+    bool stop = false;
+    __device__ __forceinline__ void begin(int traj, bool first)
+    {
+        if (done[traj]) return;
+        if (!pm) {
+            s_v = sc.s[traj];
+            return;
+        }
+        const RefEnergy e = ref_energy(pm, per, traj, P[traj >> rec_shift]);
+        const int flag = e.flag(sc.e_prev[traj], tol, use_rule);
+        s_v = sqrt(e.s2);
+        stop = flag != 0;
+        if (first && threadIdx.x == 0) e.record(sc, traj, flag);
+    }
+    __device__ __forceinline__ bool skip(int traj) const { return done[traj] || stop; }
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return psi; }
     template <int M, class Xs>
@@ -133,12 +250,13 @@ template <typename T, int N> struct OpGsNonlinIm : SkipDone {
     {
         const TrajParams &p = P[traj >> rec_shift];
         const T hdt = (T)(0.5 * p.dt_steady), g11 = (T)p.g11, scale = (T)(1.0 / (N * N));
+        const T s_in = (T)s_v;
         const int itmax = p.itmax;
         static_for<0, M>([&](auto X_) {
             constexpr int i = decltype(X_)::value;
             const int x = xs(i);
             const T V = potential_t<T>(p, x, y, z);
-            const cpx<T> a0 = r[0][i];
+            const cpx<T> a0 = cscale<T>(r[0][i], s_in);
             cpx<T> a = a0;
             T da = (T)0;
             for (int it = 0; it < itmax; ++it) {
@@ -184,45 +302,18 @@ template <typename T, int N> struct OpGsMeasureRef : SkipDone {
 };
 
 // x-space psi * s / (NX NY) -> forward xy transform (x -> hybrid)
-// Fused renormalisation (pn != nullptr): the scale of the previous update,
-// s = sqrt(N_target / (dV sum |psi|^2)), from its partials (the sums of
-// scalar_norm_kernel); the first workgroup records s and counts the iteration.
 template <typename T, int N> struct OpGsForward : SkipDone {
     static constexpr int NC = 1, SIGN_IN = 0, SIGN_OUT = +1, NSUM = 0;
     static constexpr bool WRITE = true;
     const cpx<T> *psi;
     cpx<T> *w;
     const double *scale;
-    const double *pn = nullptr;
-    int per = 0, rec_shift = 0;
-    const TrajParams *P = nullptr;
-    GsScalars sc{};
-    double s_v = 1.0;
-    bool bad = false;
-    __device__ __forceinline__ void begin(int traj, bool first)
-    {
-        if (done && done[traj]) return;
-        if (!pn) {
-            s_v = scale[traj];
-            return;
-        }
-        const TrajParams &p = P[traj >> rec_shift];
-        const double n = psum(pn, per, 1, traj, 0) * dv_of(p);
-        s_v = sqrt((sc.target ? sc.target[traj] : p.N0) / n);
-        bad = !(n == n);
-        if (first && threadIdx.x == 0) {
-            sc.s[traj] = s_v;
-            sc.iters[traj] += 1;
-            if (bad) sc.done[traj] = 2;
-        }
-    }
-    __device__ __forceinline__ bool skip(int traj) const { return (done && done[traj]) || bad; }
     __device__ const cpx<T> *src(int) const { return psi; }
     __device__ cpx<T> *dst(int) const { return w; }
     template <int M, class Xs>
-    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int traj, long, double *) const
+    __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs, int, int, int traj, long, double *) const
     {
-        const T s = (T)(s_v / (N * N));
+        const T s = (T)(scale[traj] / (N * N));
 #pragma unroll
         for (int i = 0; i < M; ++i) r[0][i] = cscale<T>(r[0][i], s);
     }
@@ -315,16 +406,17 @@ template <typename T, int N> struct OpGsResid : SkipDone {
     }
 };
 
-// psi_new = s psi - tau d + beta (s psi - prev); prev <- s psi ; partial |psi_new|^2
+// psi_new = s psi - tau d + beta (s psi - prev); prev <- s psi ; partial |psi_new|^2 ;
+// psi_new / (NX NY) -> forward xy transform, where the next iteration begins (its
+// renormalisation, linear, is applied in k-space)
 template <typename T, int N> struct OpGsUpdate : SkipDone {
-    static constexpr int NC = 1, SIGN_IN = -1, SIGN_OUT = 0, NSUM = 1;
-    static constexpr bool WRITE = false;
-    cpx<T> *psi, *prev;
-    const cpx<T> *w;
+    static constexpr int NC = 1, SIGN_IN = -1, SIGN_OUT = +1, NSUM = 1;
+    static constexpr bool WRITE = true;
+    cpx<T> *psi, *prev, *w;
     const double *scale;
     T tau, beta;
     __device__ const cpx<T> *src(int) const { return w; }
-    __device__ cpx<T> *dst(int) const { return nullptr; }
+    __device__ cpx<T> *dst(int) const { return w; }
     template <int M, class Xs>
     __device__ __forceinline__ void apply(cpx<T> (&r)[1][M], Xs xs, int, int, int traj, long row, double *s) const
     {
@@ -339,6 +431,7 @@ template <typename T, int N> struct OpGsUpdate : SkipDone {
             prev[row + x] = ps;
             psi[row + x] = nw;
             s[0] += (double)nw.x * nw.x + (double)nw.y * nw.y;
+            r[0][i] = cscale<T>(nw, (T)(1.0 / (N * N)));
         });
     }
 };
@@ -368,20 +461,9 @@ __global__ void scalar_ref_kernel(const double *partial, int per, int ntraj, con
 {
     const int traj = blockIdx.x;   // one wave per trajectory
     if (traj >= ntraj || sc.done[traj]) return;
-    const bool lead = threadIdx.x == 0;
-    const TrajParams &p = P[traj >> rec_shift];
-    const double dV = dv_of(p);
-    const double D = psum(partial, per, 4, traj, 0), A = psum(partial, per, 4, traj, 1);
-    const double B = psum(partial, per, 4, traj, 2), C = psum(partial, per, 4, traj, 3);
-    const double s2 = p.N0 / (D * dV);
-    const double E = dV * (s2 * (A + C) + p.g11 * s2 * s2 * B / 2.0);
-    if (!lead) return;
-    sc.iters[traj] += 1;
-    if (use_rule && fabs((E - sc.e_prev[traj]) / E) < tol) sc.done[traj] = 1;
-    if (!(E == E) || !(s2 == s2)) sc.done[traj] = 2;   // non-finite
-    sc.e_prev[traj] = E;
-    sc.e_ref[traj] = E;
-    sc.s[traj] = sqrt(s2);
+    const RefEnergy e = ref_energy(partial, per, traj, P[traj >> rec_shift]);
+    if (threadIdx.x != 0) return;
+    e.record(sc, traj, e.flag(sc.e_prev[traj], tol, use_rule));
 }
 
 __global__ void scalar_mu_kernel(const double *partial, int per, int ntraj, GsScalars sc)
@@ -463,29 +545,47 @@ __global__ void tf_kernel(cpx<T> *psi, int nx, int ny, int nz, long n, const Tra
 
 // ------------------------------------------------------------- launchers
 
-hipError_t gs_z_imag(const DevGroup &g, void *psi, const GsScalars &sc, void *kcopy, hipStream_t s)
+template <class Op, typename T, int NZ> static void set_imag(Op &op, const DevGroup &g, const GsScalars &sc, const void *in, void *out)
+{
+    const int nxy = g.nx * g.ny;
+    op.done = sc.done;
+    op.in = (const cpx<T> *)in;
+    op.out = (cpx<T> *)out;
+    op.kxy = (const cpx<T> *)g.kxy + (long)KT_IM_HALF * g.n_records * nxy;
+    op.kz = (const cpx<T> *)g.kz + (long)KT_IM_HALF * g.n_records * NZ;
+    op.nxy = nxy;
+    op.rec_shift = g.rec_shift;
+}
+
+hipError_t gs_z_imag(const DevGroup &g, const void *in, void *out, const GsScalars &sc, hipStream_t s)
 {
     int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
         using T = typename decltype(Tt)::type;
         constexpr int NZ = decltype(NZt)::value;
-        constexpr int R1 = z_r1<NZ>();
-        const int nxy = g.nx * g.ny;
-        OpGsZImag<T, NZ, R1> op;
-        op.done = sc.done;
+        OpGsZImag<T, NZ, z_r1<NZ>()> op;
+        set_imag<decltype(op), T, NZ>(op, g, sc, in, out);
+        return with_pw(pw, [&](auto PWt) { return launch_z<T, NZ, decltype(PWt)::value, +1, true>(g, op, g.ntraj, s); });
+    });
+}
+
+hipError_t gs_z_step(const DevGroup &g, void *q, void *psi, void *kcopy, const GsScalars &sc, hipStream_t s)
+{
+    int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
+    return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
+        using T = typename decltype(Tt)::type;
+        constexpr int NZ = decltype(NZt)::value;
+        OpGsZStep<T, NZ, z_r1<NZ>()> op;
+        set_imag<decltype(op), T, NZ>(op, g, sc, q, q);
         op.psi = (cpx<T> *)psi;
-        op.kxy = (const cpx<T> *)g.kxy + (long)KT_IM_HALF * g.n_records * nxy;
-        op.kz = (const cpx<T> *)g.kz + (long)KT_IM_HALF * g.n_records * NZ;
-        op.scale = sc.s;
         op.kcopy = (cpx<T> *)kcopy;
-        op.nxy = nxy;
-        op.rec_shift = g.rec_shift;
+        op.sc = sc;
         return with_pw(pw, [&](auto PWt) { return launch_z<T, NZ, decltype(PWt)::value, +1, true>(g, op, g.ntraj, s); });
     });
 }
 
 hipError_t gs_z_diag(const DevGroup &g, void *w, const GsScalars &sc, const GsTables &t, int variant, double alpha,
-                     const double *alpha_rec, hipStream_t s, const GsResidualTest *test)
+                     const double *alpha_rec, hipStream_t s, const GsResidualTest *test, const double *pn)
 {
     int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
@@ -502,6 +602,12 @@ hipError_t gs_z_diag(const DevGroup &g, void *w, const GsScalars &sc, const GsTa
         op.variant = variant;
         op.alpha = alpha;
         op.alpha_rec = alpha_rec;
+        if (pn) {
+            op.rn.pn = pn;
+            op.rn.per = xy_wg_per_traj(g);
+            op.rn.P = g.params;
+            op.rn.sc = sc;
+        }
         if (test) {
             op.fr.ph = test->ph;
             op.fr.pr = test->pr;
@@ -515,7 +621,8 @@ hipError_t gs_z_diag(const DevGroup &g, void *w, const GsScalars &sc, const GsTa
     });
 }
 
-hipError_t gs_xy_nonlinear_imag(const DevGroup &g, void *psi, const GsScalars &sc, hipStream_t s)
+hipError_t gs_xy_nonlinear_imag(const DevGroup &g, void *psi, const GsScalars &sc, hipStream_t s, const double *pm,
+                                double tol, int use_rule)
 {
     return dispatch(g, [&](auto Tt, auto Nt, auto) -> hipError_t {
         using T = typename decltype(Tt)::type;
@@ -525,6 +632,11 @@ hipError_t gs_xy_nonlinear_imag(const DevGroup &g, void *psi, const GsScalars &s
         op.psi = (cpx<T> *)psi;
         op.P = g.params;
         op.rec_shift = g.rec_shift;
+        op.pm = pm;
+        op.per = xy_wg_per_traj(g);
+        op.use_rule = use_rule;
+        op.tol = tol;
+        op.sc = sc;
         return launch_xy<T, N>(g, op, g.ntraj, nullptr, s);
     });
 }
@@ -556,8 +668,7 @@ hipError_t gs_scalar_ref(const DevGroup &g, const double *partial, const GsScala
     return hipGetLastError();
 }
 
-hipError_t gs_xy_forward(const DevGroup &g, const void *psi, void *w, const GsScalars &sc, hipStream_t s,
-                         const double *pn)
+hipError_t gs_xy_forward(const DevGroup &g, const void *psi, void *w, const GsScalars &sc, hipStream_t s)
 {
     return dispatch(g, [&](auto Tt, auto Nt, auto) -> hipError_t {
         using T = typename decltype(Tt)::type;
@@ -567,11 +678,6 @@ hipError_t gs_xy_forward(const DevGroup &g, const void *psi, void *w, const GsSc
         op.psi = (const cpx<T> *)psi;
         op.w = (cpx<T> *)w;
         op.scale = sc.s;
-        op.pn = pn;
-        op.per = xy_wg_per_traj(g);
-        op.P = g.params;
-        op.rec_shift = g.rec_shift;
-        op.sc = sc;
         return launch_xy<T, N>(g, op, g.ntraj, nullptr, s);
     });
 }
@@ -629,7 +735,7 @@ hipError_t gs_scalar_residual(const DevGroup &g, const double *partial_h, const 
     return hipGetLastError();
 }
 
-hipError_t gs_xy_update(const DevGroup &g, void *psi, void *prev, const void *w, const GsScalars &sc, double tau,
+hipError_t gs_xy_update(const DevGroup &g, void *psi, void *prev, void *w, const GsScalars &sc, double tau,
                         double beta, double *partial, hipStream_t s)
 {
     return dispatch(g, [&](auto Tt, auto Nt, auto) -> hipError_t {
@@ -639,7 +745,7 @@ hipError_t gs_xy_update(const DevGroup &g, void *psi, void *prev, const void *w,
         op.done = sc.done;
         op.psi = (cpx<T> *)psi;
         op.prev = (cpx<T> *)prev;
-        op.w = (const cpx<T> *)w;
+        op.w = (cpx<T> *)w;
         op.scale = sc.s;
         op.tau = (T)tau;
         op.beta = (T)beta;

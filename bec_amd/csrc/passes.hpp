@@ -377,11 +377,13 @@ __global__ void __launch_bounds__(4 * N) xy_quad_kernel(Op op, XyGeom g, double 
 // workgroup, by every thread, before skip(): operators may compute per-
 // trajectory scalars there (first: the workgroup is its trajectory's first).
 struct NoSkip {
+    static constexpr bool TWICE = false;
     __device__ __forceinline__ void begin(int, bool) {}
     __device__ __forceinline__ bool skip(int) const { return false; }
 };
 // Operators that skip trajectories whose done flag is set.
 struct SkipDone {
+    static constexpr bool TWICE = false;
     const int *done;
     __device__ __forceinline__ void begin(int, bool) {}
     __device__ __forceinline__ bool skip(int traj) const { return done && done[traj]; }
@@ -755,6 +757,8 @@ struct ZGeom {
 //   static constexpr int NC;
 //   const cpx<T>* src(int c); cpx<T>* dst(int c);
 //   void kspace(int c, cpx<T> (&X)[KPT][NW], int kk0, int q, int traj)   (k-space values, kz = kk0+i + R1*m)
+//   TWICE: the transform back of kspace's values goes to first(c), and that of the
+//   values again() makes of them to dst(c)
 // blockIdx.y selects the first component (component-split launches of NC = 1).
 // HALF = true exchanges real and imaginary parts in two rounds through a tile
 // of NZ*PW reals (half the LDS, so more workgroups fit on a CU).
@@ -907,18 +911,35 @@ __device__ __forceinline__ void z_tile_compute(Op &op, const ZGeom &g, const cpx
         op.kspace(c, X, kk0, q, traj);
 
         if constexpr (ROUNDTRIP) {
+            auto back = [&](cpx<T> (&X)[KPT][NW]) {
 #pragma unroll
-            for (int i = 0; i < KPT; ++i) {
-                dft<T, NW, -SIGN_F>(X[i]);
+                for (int i = 0; i < KPT; ++i) {
+                    dft<T, NW, -SIGN_F>(X[i]);
 #pragma unroll
-                for (int w2 = 1; w2 < NW; ++w2) {
-                    cpx<T> f = tw[(w2 * (kk0 + i)) % NZ];
-                    if (SIGN_F > 0) f.y = -f.y;
-                    X[i][w2] = cmul<T>(X[i][w2], f);
+                    for (int w2 = 1; w2 < NW; ++w2) {
+                        cpx<T> f = tw[(w2 * (kk0 + i)) % NZ];
+                        if (SIGN_F > 0) f.y = -f.y;
+                        X[i][w2] = cmul<T>(X[i][w2], f);
+                    }
                 }
+                from_k(X, v[c]);
+                dft<T, R1, -SIGN_F, NW>(v[c]);
+            };
+            if constexpr (Op::TWICE) {
+                cpx<T> Y[KPT][NW];
+#pragma unroll
+                for (int i = 0; i < KPT; ++i)
+#pragma unroll
+                    for (int m = 0; m < NW; ++m) Y[i][m] = X[i][m];
+                back(X);
+                cpx<T> *d = op.first(c + cb);
+#pragma unroll
+                for (int j = 0; j < R1; ++j) st<NT, T>(d + base + (long)(w + NW * j) * g.nxy, v[c][j]);
+                op.again(c, Y, kk0, q, traj);
+                back(Y);
+            } else {
+                back(X);
             }
-            from_k(X, v[c]);
-            dft<T, R1, -SIGN_F, NW>(v[c]);
         } else {
             cpx<T> *d = op.dst(c + cb);
 #pragma unroll
