@@ -52,6 +52,9 @@ size_t elem_size(int prec);                       // bytes of one complex value
 long xy_workgroups(const DevGroup &g, int ntraj); // partial-sum slots of an xy pass
 int xy_wg_per_traj(const DevGroup &g);
 int default_pw(int prec, int nx, int nz);
+// pencils per workgroup of the z passes that exchange whole values (a schedule's pw
+// may fit the half exchange only)
+int full_pw(const DevGroup &g);
 int default_r1(int nz);
 // the schedule candidates the hot-pass launchers are instantiated for; unless
 // `all`, without the forms that cannot win at this batch (the ones the autotuner

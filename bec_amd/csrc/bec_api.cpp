@@ -234,6 +234,47 @@ int group_build_tables(Group &g, double dt, hipStream_t s)
     return BEC_OK;
 }
 
+// The schedule a group starts with: where each choice pays, from sweeps over
+// lattices of 64..256 x 16..32^2 and 1..4096 trajectories (us per step).
+static void default_schedule(DevGroup &d)
+{
+    d.pw = 0;
+    d.z_r1 = 0;
+    d.z_split = 1;   // one component per z workgroup
+    d.nt = d.prec == 0 ? 1 : 0;
+    d.xcd = d.ntraj % 8 == 0 ? 1 : 0;
+    d.xy_minw = 1;
+    d.z_half = 0;
+    d.xy_split = 0;
+    const long nxy = (long)d.nx * d.ny;
+    const long z_wgs = 2L * d.ntraj * nxy / default_pw(d.prec, d.nx, d.nz);
+    if (d.prec != 0) {
+        // 64 pencils to a z workgroup (whole wavefronts of one z subset, so its twiddles
+        // are scalar) through the half exchange, where that still leaves a workgroup for
+        // every CU: 57.3 -> 54.6 at 64 x 128x16x16; at 8 (64 workgroups) 13.5 -> 16.0
+        if (default_pw(d.prec, d.nx, d.nz) < 64 && d.nz * 64L * 8 <= 65536 && 2L * d.ntraj * nxy / 64 >= 256) {
+            d.pw = 64;
+            d.z_half = 1;
+        }
+        return;
+    }
+    // at most half as many z workgroups as CUs: workgroups of half the pencils.  (One
+    // wavefront per component in the plane pass would also pay there, 14.7 -> 11.1 at
+    // 8 x 128x16x16 with both, but rounds differently; the autotuner offers it.)
+    if (z_wgs <= 128) d.pw = std::min(32, default_pw(0, d.nx, d.nz));
+    // the state, 67 MB and below, fits the last-level cache (256 MB) twice over either
+    // way; from there to about 400 MB temporal accesses keep part of it there between
+    // the passes (160 trajectories 70 -> 62, 256: 101 -> 93, 512: 193 -> 173, 768: 287 ->
+    // 275), beyond it streaming ones are better (1024: 366 against 374).  From 72 MB on the
+    // passes wait on memory, and half the LDS to a z workgroup puts more of them on a CU
+    // (2048: 728 -> 714); with 256 z points it does not pay beyond the cache.
+    const long mib = 16L * d.ntraj * d.nz * nxy >> 20;
+    if (mib > 72) {
+        if (mib <= 384) d.nt = 0;
+        d.z_half = mib <= 384 || d.nz <= 128 ? 1 : 0;
+    }
+}
+
 int group_setup(Group &g, const bec_calc_params &c, int prec, int ntraj, bool alloc_state)
 {
     if (!shape_supported(c.nvx, c.nvy, c.nvz)) {
@@ -251,16 +292,7 @@ int group_setup(Group &g, const bec_calc_params &c, int prec, int ntraj, bool al
     d.ntraj = ntraj;
     d.rec_shift = 30;
     d.n_records = 1;
-    // default schedule: the autotuned choice on MI355X for 128x16x16 batches
-    // (one component per z workgroup, streaming accesses, XCD-aware placement)
-    d.pw = 0;
-    d.z_r1 = 0;
-    d.z_split = 1;
-    d.nt = prec == 0 ? 1 : 0;
-    d.xcd = ntraj % 8 == 0 ? 1 : 0;
-    d.xy_minw = 1;
-    d.z_half = 0;
-    d.xy_split = 0;
+    default_schedule(d);
     d.itmax1 = c.itmax == 1 ? 1 : 0;
     const size_t es = elem_size(prec);
     if (alloc_state) {

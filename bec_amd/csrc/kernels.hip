@@ -25,6 +25,8 @@ int default_pw(int prec, int nx, int nz)
     return pw;
 }
 
+int full_pw(const DevGroup &g) { return std::min(g.pw ? g.pw : 64, default_pw(g.prec, g.nx, g.nz)); }
+
 int default_r1(int nz) { return nz == 64 ? 8 : 16; }
 
 int schedule_candidates(int prec, int nx, int nz, int ntraj, Schedule *out, int max_out, bool all)
@@ -183,7 +185,7 @@ static hipError_t launch_nonlinear(const DevGroup &g, hipStream_t s)
         if constexpr (sizeof(T) == 4 && IT1) {
             if (g.xy_split) {
                 constexpr int PPW = 64 / N;
-                XyGeom geo{g.nz, (long)g.ntraj * g.nz, (g.xcd && g.ntraj % 8 == 0) ? 1 : 0};
+                XyGeom geo{g.nz, (long)g.ntraj * g.nz, placed(g.xcd, g.ntraj)};
                 if (geo.n_planes % PPW) return hipErrorInvalidValue;
                 hipLaunchKernelGGL((xy_split_kernel<N, NT>), dim3((unsigned)(geo.n_planes / PPW)), dim3(128), 0, s,
                                    op, geo);
@@ -287,7 +289,7 @@ hipError_t run_xy_fft(const DevGroup &g, const void *in, void *out, int ntraj, i
 hipError_t run_z_fft(const DevGroup &g, const void *in, void *out, int ntraj, int sign, double scale,
                      hipStream_t s)
 {
-    int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
+    const int pw = full_pw(g);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
         using T = typename decltype(Tt)::type;
         constexpr int NZ = decltype(NZt)::value;

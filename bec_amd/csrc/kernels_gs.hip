@@ -559,7 +559,7 @@ template <class Op, typename T, int NZ> static void set_imag(Op &op, const DevGr
 
 hipError_t gs_z_imag(const DevGroup &g, const void *in, void *out, const GsScalars &sc, hipStream_t s)
 {
-    int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
+    const int pw = full_pw(g);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
         using T = typename decltype(Tt)::type;
         constexpr int NZ = decltype(NZt)::value;
@@ -571,7 +571,7 @@ hipError_t gs_z_imag(const DevGroup &g, const void *in, void *out, const GsScala
 
 hipError_t gs_z_step(const DevGroup &g, void *q, void *psi, void *kcopy, const GsScalars &sc, hipStream_t s)
 {
-    int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
+    const int pw = full_pw(g);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
         using T = typename decltype(Tt)::type;
         constexpr int NZ = decltype(NZt)::value;
@@ -587,7 +587,7 @@ hipError_t gs_z_step(const DevGroup &g, void *q, void *psi, void *kcopy, const G
 hipError_t gs_z_diag(const DevGroup &g, void *w, const GsScalars &sc, const GsTables &t, int variant, double alpha,
                      const double *alpha_rec, hipStream_t s, const GsResidualTest *test, const double *pn)
 {
-    int pw = g.pw ? g.pw : default_pw(g.prec, g.nx, g.nz);
+    const int pw = full_pw(g);
     return dispatch(g, [&](auto Tt, auto, auto NZt) -> hipError_t {
         using T = typename decltype(Tt)::type;
         constexpr int NZ = decltype(NZt)::value;

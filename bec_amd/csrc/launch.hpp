@@ -52,11 +52,14 @@ template <class F> inline hipError_t with_bool(int v, F &&f)
     return v ? f(std::true_type{}) : f(std::false_type{});
 }
 
+// XCD-aware placement (xcd_remap) of a launch over ntraj trajectories
+inline int placed(int xcd, int ntraj) { return xcd && ntraj % 8 == 0 ? 1 : 0; }
+
 // ncomp_grid > 1: component-split launch (grid.y = ncomp_grid, Op::NC == 1)
 template <typename T, int NZ, int PW, int SIGN_F, bool RT, class Op, int R1 = z_r1<NZ>(), bool NT = false,
           bool HALF = false>
 inline hipError_t launch_z(const DevGroup &g, const Op &op, int ntraj, hipStream_t s, int ncomp_grid = 1,
-                           int xcd = 0)
+                           int xcd = 1)
 {
     if constexpr ((long)NZ * PW * (HALF ? sizeof(T) : sizeof(cpx<T>)) > 65536 || (NZ / R1) * PW > 1024) {
         return hipErrorInvalidValue;   // LDS exchange tile above 64 KiB: not instantiated
@@ -64,7 +67,7 @@ inline hipError_t launch_z(const DevGroup &g, const Op &op, int ntraj, hipStream
         constexpr int NW = NZ / R1;
         const int nxy = g.nx * g.ny;
         if (nxy % PW) return hipErrorInvalidValue;
-        ZGeom geo{nxy, nxy / PW, (xcd && ntraj % 8 == 0) ? 1 : 0};
+        ZGeom geo{nxy, nxy / PW, placed(xcd, ntraj)};
         dim3 grid((unsigned)((long)ntraj * geo.tiles_per_traj), (unsigned)ncomp_grid), block(NW * PW);
         hipLaunchKernelGGL((z_kernel<T, NZ, R1, PW, SIGN_F, RT, Op, NT, HALF>), grid, block, 0, s, op, geo,
                            (const cpx<T> *)g.tw);
@@ -74,9 +77,9 @@ inline hipError_t launch_z(const DevGroup &g, const Op &op, int ntraj, hipStream
 
 template <typename T, int N, class Op, bool NT = false, int MINW = 1>
 inline hipError_t launch_xy(const DevGroup &g, const Op &op, int ntraj, double *partial, hipStream_t s,
-                            int xcd = 0)
+                            int xcd = 1)
 {
-    XyGeom geo{g.nz, (long)ntraj * g.nz, (xcd && ntraj % 8 == 0) ? 1 : 0};
+    XyGeom geo{g.nz, (long)ntraj * g.nz, placed(xcd, ntraj)};
     if constexpr (sizeof(T) == 8) {
         hipLaunchKernelGGL((xy_quad_kernel<N, Op>), dim3((unsigned)geo.n_planes), dim3(4 * N), 0, s, op, geo, partial);
     } else {

@@ -21,39 +21,27 @@
 namespace bec {
 
 // ------------------------------------------------------------ memory access
-// NT = true issues non-temporal (streaming) loads and stores: the state is
-// touched once per pass, so it should not displace reusable lines.
-typedef float v2f_t __attribute__((ext_vector_type(2)));
-typedef double v2d_t __attribute__((ext_vector_type(2)));
+// NT = true issues non-temporal (streaming) loads and stores: for states that do
+// not stay in the caches between the passes, so that they displace nothing.  Both
+// forms load the same vector type: the compiler then fuses the same products, and a
+// schedule's nt does not change the results.
+template <typename T> struct VecOf;
+template <> struct VecOf<float> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct VecOf<double> { typedef double type __attribute__((ext_vector_type(2))); };
 
 template <bool NT, typename T> __device__ __forceinline__ cpx<T> ld(const cpx<T> *p)
 {
-    if constexpr (NT) {
-        if constexpr (sizeof(T) == 4) {
-            const v2f_t r = __builtin_nontemporal_load((const v2f_t *)p);
-            return mk<T>(r.x, r.y);
-        } else {
-            const v2d_t r = __builtin_nontemporal_load((const v2d_t *)p);
-            return mk<T>(r.x, r.y);
-        }
-    } else {
-        return *p;
-    }
+    using V = typename VecOf<T>::type;
+    const V r = NT ? __builtin_nontemporal_load((const V *)p) : *(const V *)p;
+    return mk<T>(r.x, r.y);
 }
 
 template <bool NT, typename T> __device__ __forceinline__ void st(cpx<T> *p, cpx<T> v)
 {
-    if constexpr (NT) {
-        if constexpr (sizeof(T) == 4) {
-            v2f_t r = {v.x, v.y};
-            __builtin_nontemporal_store(r, (v2f_t *)p);
-        } else {
-            v2d_t r = {v.x, v.y};
-            __builtin_nontemporal_store(r, (v2d_t *)p);
-        }
-    } else {
-        *p = v;
-    }
+    using V = typename VecOf<T>::type;
+    const V r = {v.x, v.y};
+    if constexpr (NT) __builtin_nontemporal_store(r, (V *)p);
+    else *(V *)p = r;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (blockIdx % 8).  With
