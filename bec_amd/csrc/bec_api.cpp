@@ -264,10 +264,10 @@ static void default_schedule(DevGroup &d)
     if (z_wgs <= 128) d.pw = std::min(32, default_pw(0, d.nx, d.nz));
     // the state, 67 MB and below, fits the last-level cache (256 MB) twice over either
     // way; from there to about 400 MB temporal accesses keep part of it there between
-    // the passes (160 trajectories 70 -> 62, 256: 101 -> 93, 512: 193 -> 173, 768: 287 ->
-    // 275), beyond it streaming ones are better (1024: 366 against 374).  From 72 MB on the
+    // the passes (160 trajectories 70 -> 62, 256: 98 -> 92, 512: 190 -> 174, 768: 283 ->
+    // 268), beyond it streaming ones are better (2048: 725 against 761).  From 72 MB on the
     // passes wait on memory, and half the LDS to a z workgroup puts more of them on a CU
-    // (2048: 728 -> 714); with 256 z points it does not pay beyond the cache.
+    // (2048: 737 -> 725); with 256 z points it does not pay beyond the cache.
     const long mib = 16L * d.ntraj * d.nz * nxy >> 20;
     if (mib > 72) {
         if (mib <= 384) d.nt = 0;
