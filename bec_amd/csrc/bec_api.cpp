@@ -258,10 +258,12 @@ static void default_schedule(DevGroup &d)
         }
         return;
     }
-    // at most half as many z workgroups as CUs: workgroups of half the pencils.  (One
-    // wavefront per component in the plane pass would also pay there, 14.7 -> 11.1 at
-    // 8 x 128x16x16 with both, but rounds differently; the autotuner offers it.)
-    if (z_wgs <= 128) d.pw = std::min(32, default_pw(0, d.nx, d.nz));
+    // at most half as many z workgroups as CUs: workgroups of half the pencils (1, 4, 16
+    // of 128x16x16: 15.1 -> 13.8, 16.2 -> 14.9, 16.3 -> 15.1; not with 64 z points, whose
+    // threads hold 8 values: 12.1 against 12.3 at 8).  One wavefront per component in the
+    // plane pass would also pay there (8: 14.7 -> 11.1 with both), but rounds
+    // differently; the autotuner offers it.
+    if (z_wgs <= 128 && d.nz > 64) d.pw = std::min(32, default_pw(0, d.nx, d.nz));
     // the state, 67 MB and below, fits the last-level cache (256 MB) twice over either
     // way; from there to about 400 MB temporal accesses keep part of it there between
     // the passes (160 trajectories 70 -> 62, 256: 98 -> 92, 512: 190 -> 174, 768: 283 ->
