@@ -4,8 +4,9 @@
  * supplies initial guesses to bec_ground_states_two_component (bec_api.h),
  * whose Thomas-Fermi start remains the fallback.
  *
- * Every operation of the network is a strided batched GEMM on BF16 operands
- * with FP32 accumulation (bec_gemm), plus element-wise kernels:
+ * Every operation of the network is a product of BF16 operands with FP32
+ * accumulation, on fused kernels for widths 16, 32 and 64 and as strided batched
+ * GEMMs (bec_gemm) for other shapes, in the same order of additions:
  *   lift      h0 = x P + p                       (per cell, c_in -> width)
  *   layer l   h' = act(h W_l + b_l + K_l h)      (l = 0..layers-1, no act on the last)
  *   K_l h     = Re IDFT_z IDFT_xy [ R_l(k) . DFT_xy DFT_z h ](modes)
@@ -14,8 +15,8 @@
  *              both transforms scaled by 1/sqrt(cells) each)
  *   project   y = act(h Q1 + q1) Q2 + q2          (width -> hidden -> c_out)
  * act is GELU, 0.5 x (1 + erf(x / sqrt 2)).  Activations are FP32 in memory
- * and rounded to BF16 (nearest even) as GEMM operands; weights are kept as
- * FP32 masters with BF16 copies (Adam updates the masters). */
+ * and rounded to BF16 (nearest even) as operands, as are the weights, kept as
+ * FP32 masters (Adam updates the masters). */
 #ifndef BEC_FNO_H
 #define BEC_FNO_H
 
