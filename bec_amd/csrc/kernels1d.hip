@@ -37,6 +37,12 @@ namespace {
 constexpr int MAXNV = W1D_MAX_NV;
 
 __device__ __forceinline__ double2 cm(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// a (b + lo), lo below the rounding of b
+__device__ __forceinline__ double2 cm_ext(double2 a, double2 b, double2 lo)
+{
+    return make_double2(fma(a.x, b.x, fma(-a.y, b.y, fma(a.x, lo.x, -(a.y * lo.y)))),
+                        fma(a.x, b.y, fma(a.y, b.x, fma(a.x, lo.y, a.y * lo.x))));
+}
 __device__ __forceinline__ double2 cs(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
 __device__ __forceinline__ double nrm(double2 a) { return a.x * a.x + a.y * a.y; }
 
@@ -82,7 +88,7 @@ template <int NC> __device__ __forceinline__ Line make_line(int n, double2 *lds)
     l.D = l.S + NC * l.hs;
     for (int m = threadIdx.x; m < n; m += blockDim.x) {
         double s, c;
-        sincospi(2.0 * m / n, &s, &c);
+        unit_root(m, n, &c, &s);
         lds[m] = make_double2(c, s);
     }
     for (int m = threadIdx.x; m < 2 * NC * l.hs; m += blockDim.x) l.S[m] = make_double2(0.0, 0.0);
@@ -277,6 +283,15 @@ __global__ __launch_bounds__(H ? 64 : 512) void w1d_ensemble_kernel(W1dParams p,
     sincos(kv * kv * p.dt / 2.0, &sn, &co);
     const double2 kw = make_double2(co, sn);   // exp(+i k^2 dt/2)
     const double2 kwn = cs(kw, inv);
+    // What kwn leaves of kw / (n |kw|^2): the roundings of the product, of 1 / n and of
+    // kw's modulus, which every step applies again to the same mode.  With it and the
+    // factors of unit_root the norm drifts by at most 4e-17 a step at 21 to 511 cells
+    // (3.2e-16 without both, at 21); 0.4% of the time of 20 trajectories of 41 cells.
+    const double c2 = co * co, s2 = sn * sn;   // |kw|^2 - 1, exactly but for the last sum
+    const double mod = (fmax(c2, s2) - 1.0) + fmin(c2, s2) + (fma(co, co, -c2) + fma(sn, sn, -s2));
+    const double inv_lo = fma(-inv, (double)n, 1.0) * inv;
+    const double2 kwl = make_double2(fma(co, inv, -kwn.x) + co * inv_lo - kwn.x * mod,
+                                     fma(sn, inv, -kwn.y) + sn * inv_lo - kwn.y * mod);
     const double z0 = -p.zmax + p.dz * l.k, z1 = -p.zmax + p.dz * (n - l.k);
     const double base0 = p.mu - z0 * z0 / 4.0, base1 = p.mu - z1 * z1 / 4.0;
     const double gown = l.c ? p.g22 : p.g11, det = l.c ? -0.5 * p.E : 0.5 * p.E;
@@ -327,8 +342,8 @@ __global__ __launch_bounds__(H ? 64 : 512) void w1d_ensemble_kernel(W1dParams p,
             x = cm(x, e0);
             y = l.two ? cm(y, e1) : zero;
             dft_line<+1, H>(l, f, x, y);
-            x = cm(x, kwn);
-            y = l.two ? cm(y, kwn) : zero;
+            x = cm_ext(x, kwn, kwl);
+            y = l.two ? cm_ext(y, kwn, kwl) : zero;
         }
         if (nn >= 0) {   // second pulse U^+ and measurement in k-space (:358-391)
             double2 u, v;

@@ -124,3 +124,20 @@ def test_line_lengths_at_the_edges_match_oracle(bec, oracle, nv):
     ref = oracle.run1d(oracle.Params1D(**{f: getattr(p, f) for f, _ in oracle.Params1D._fields_}))
     for key, bar in (("gs", 1e-11), ("ntot", 1e-11), ("m", 1e-9), ("vis", 1e-9), ("avn", 1e-9)):
         assert _rel(got[key], ref[key]) < bar, key
+
+
+@pytest.mark.parametrize("nv", [21, 41, 63, 65, 511])
+def test_norm_does_not_drift(bec, nv):
+    """The steps are unitary: N1 + N2 of the samples is constant but for rounding.  What repeats every step
+    and so accumulates is the rounding of the DFT's factors (half an ulp each, 2 c dc averaged over a
+    column: 1.4e-17 at 21 cells, and two transforms a step); factors rounded as sincospi(2 m / n) and a
+    rounded 1 / n gave -2.7e-16 (21 and 63 cells) and +2.9e-16 (65) a step.  The rounding of the sums
+    themselves averages out over 64 trajectories and the steps."""
+    steps = 200 if nv < 200 else 40
+    p = bec.params1d(dz=1.0 if nv == 41 else 20.0 / (nv // 2 + 0.5), ne=64, ntW=steps, seed=5)
+    assert bec.cells_1d(p) == nv
+    m = bec.run_1d(p)["m"]
+    n = m[0] + m[1] + nv * 0.5 * (p.Va + p.Vb)
+    drift = (n[-1] - n[0]) / n[0] / (steps - 1)
+    print(f"{nv} cells: {drift:+.1e} a step")
+    assert abs(drift) < 1e-16
