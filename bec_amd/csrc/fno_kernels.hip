@@ -136,12 +136,15 @@ __global__ __launch_bounds__(64) void sum_partials(const float *__restrict__ par
 template <int NB, int MB, bool SPLIT>
 __global__ __launch_bounds__(256) void plane_dft_kernel(const unsigned short *__restrict__ A,
                                                         const float *__restrict__ in, float *__restrict__ out, int M,
-                                                        int K, int W, int per)
+                                                        int K, int W, int per, int m_blocks)
 {
     extern __shared__ __align__(16) unsigned short Bs[];   // [NB * 16][K + 8], column w at row (w % NB) 16 + w / NB
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ld = K + 8;
-    const int m0 = (blockIdx.x * 4 + wave) * 16 * MB;
-    const float *src = in + (long)blockIdx.y * K * W;
+    // the planes in the grid's x dimension, which alone holds more than 65535
+    const int mb = blockIdx.x % m_blocks;
+    const long plane = blockIdx.x / m_blocks;
+    const int m0 = (mb * 4 + wave) * 16 * MB;
+    const float *src = in + plane * K * W;
     // G tiles of A are in flight: the first group under the staging loads
     constexpr int G = 16 / MB;
     const int tiles = K / 32;
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(256) void plane_dft_kernel(const unsigned short *__
 #pragma unroll
             for (int i = 0; i < MB; ++i) a[g][i] = an[g][i];
     }
-    float *dst = out + (long)blockIdx.y * M * W;
+    float *dst = out + plane * M * W;
     const int w0 = (lane & 15) * NB;
 #pragma unroll
     for (int i = 0; i < MB; ++i)
@@ -889,7 +892,7 @@ bool plane_dft_covers(int M, int K, int W)
 hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, int M, int K, int W, int planes, int per,
                          hipStream_t s)
 {
-    if (!plane_dft_covers(M, K, W) || planes < 1 || planes > 65535) return hipErrorInvalidValue;
+    if (!plane_dft_covers(M, K, W) || planes < 1) return hipErrorInvalidValue;
     // 64 rows of A per wavefront while that leaves two workgroups for every CU,
     // else 16: the planes of a single sample would fill a quarter of the chip
     const bool wide = M % 64 == 0 && (long)planes * (M / 64) >= 1024;
@@ -898,8 +901,11 @@ hipError_t run_plane_dft(const unsigned short *A, const float *in, float *out, i
         const size_t lds = sizeof(unsigned short) * NB * 16 * (K + 8);
         auto go = [&](auto mb, auto split) {
             constexpr int MB = decltype(mb)::value;
-            hipLaunchKernelGGL((plane_dft_kernel<NB, MB, decltype(split)::value>),
-                               dim3((M + 64 * MB - 1) / (64 * MB), planes), dim3(256), lds, s, A, in, out, M, K, W, per);
+            const int m_blocks = (M + 64 * MB - 1) / (64 * MB);
+            const long wgs = (long)m_blocks * planes;
+            if (wgs > 0xffffffffL / 256) return hipErrorInvalidValue;   // threads of a launch
+            hipLaunchKernelGGL((plane_dft_kernel<NB, MB, decltype(split)::value>), dim3((unsigned)wgs), dim3(256), lds, s, A,
+                               in, out, M, K, W, per, m_blocks);
             return hipGetLastError();
         };
         using M1 = std::integral_constant<int, 1>;

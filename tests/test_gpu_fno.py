@@ -143,3 +143,30 @@ def test_network_shapes_match_oracle(bec, nz, n, mz, m, width, layers, c_in, hid
         a, b = g[sl], g_ref[sl]
         rel = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
         assert rel < 5e-2 and a @ b > 0.998 * np.linalg.norm(a) * np.linalg.norm(b), (name, rel)
+
+
+def test_more_planes_than_a_grid_dimension_holds(bec):
+    """batch * mz = 65,536 kz planes in one launch of the plane transforms (a network that create accepts).  A
+    sample's output does not depend on the batch it is in, so the oracle checks the first, the 2047th and the
+    last (BF16 bar as above); the gradient of the whole batch is the mean of its halves' (the same products;
+    sums of 2^20 FP32 terms in 256 ranges of 128 tiles: below 400 roundings of 6e-8 in a row)."""
+    from bec_amd import fno as F
+    from oracle import fno_oracle as FO
+    B, cells = 2048, 32 * 16
+    net = F.FNO(seed=4, nz=32, ny=4, nx=4, mz=32, my=4, mx=4, width=16, layers=1, c_in=8, c_out=2, hidden=16, max_batch=B)
+    ocfg = FO.Config.from_struct(net.cfg)
+    rng = np.random.default_rng(4)
+    x = rng.normal(size=(B, cells, 8)).astype(np.float32)
+    t = rng.normal(size=(B, cells, 2)).astype(np.float32)
+    y = net.predict(x)
+    some = [0, 2046, 2047]
+    ref = FO.forward(ocfg, net.get_params().astype(np.float64), _grid(x[some], ocfg)).reshape(3, cells, 2)
+    assert np.linalg.norm(y[some] - ref) < 2e-2 * np.linalg.norm(ref)
+    g = []
+    for at in (slice(0, B), slice(0, B // 2), slice(B // 2, B)):
+        xs, ts = np.ascontiguousarray(x[at]), np.ascontiguousarray(t[at])
+        net.loss_backward(F.DeviceArray(xs.shape, np.float32, xs), F.DeviceArray(ts.shape, np.float32, ts), len(xs))
+        g.append(net.get_grads().astype(np.float64))
+    for name, sl in _blocks(ocfg):
+        mean = (g[1][sl] + g[2][sl]) / 2
+        assert np.linalg.norm(g[0][sl] - mean) < 400 * 6e-8 * np.linalg.norm(mean), name
