@@ -506,9 +506,8 @@ class Solver:
         check(lib().bec_pulse_rotation(self._ctx, float(theta), float(phi)), "bec_pulse_rotation")
 
     def get_state(self, space=SPACE_X, group=0):
-        # one allocation: malloc then keeps as much of the heap mapped as a caller that
-        # polls the state needs, instead of returning it and faulting it in on every call
-        a, b = np.empty((2,) + tuple(self.shape(group)), dtype=np.complex128)
+        a = np.empty(self.shape(group), dtype=np.complex128)
+        b = np.empty_like(a)
         check(lib().bec_get_state(self._ctx, group, space, _ptr(a), _ptr(b)), "bec_get_state")
         return a, b
 

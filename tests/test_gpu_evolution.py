@@ -366,3 +366,13 @@ def test_fp64_planes_match_oracle(bec, oracle, nz, n, ne, itmax):
     got = np.asarray(sums).reshape(-1, ne, 4)[-1]
     np.testing.assert_allclose(got[:, 0], (np.abs(ax) ** 2).sum(axis=(1, 2, 3)), rtol=1e-12)
     np.testing.assert_allclose(got[:, 1], (np.abs(bx) ** 2).sum(axis=(1, 2, 3)), rtol=1e-12)
+
+
+def test_each_component_of_the_state_owns_its_memory(bec):
+    """A program that keeps one component of a state keeps that array alone."""
+    c = gpu_calc(bec, **config1_model(bec, N=30000, nvx=16, nvy=16, nvz=64, ne=2))
+    with bec.Solver(c, precision=bec.FP32) as s:
+        s.init_evolution(np.ones((64, 16, 16)), 3)
+        for space in (bec.SPACE_X, bec.SPACE_K, bec.SPACE_HYBRID):
+            for v in s.get_state(space):
+                assert v.base is None and v.flags.owndata and v.shape == (2, 64, 16, 16)
