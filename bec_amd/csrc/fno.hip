@@ -24,6 +24,7 @@
 #include "../../include/bec_fno.h"
 #include "fno_kernels.hpp"
 #include "host_common.hpp"
+#include "output_place.hpp"
 
 namespace bec {
 
@@ -226,6 +227,7 @@ struct bec_fno {
     std::vector<void *> owned;
     std::vector<std::pair<const char *, size_t>> extents;   // device buffers (bytes) for the host-side GEMM checks
     long adam_t = 0;
+    int device = 0;   // the device of the buffers
 };
 
 namespace bec {
@@ -611,6 +613,22 @@ hipError_t backward_impl(bec_fno *f, int B, const float *x, hipStream_t s)
     return layer_grad(f, x, c.c_in, dh, W, rows, g + f->oP, s);
 }
 
+OutputPlace output_place(const void *ptr)
+{
+    OutputPlace p;
+    hipPointerAttribute_t a{};
+    void *base = nullptr;
+    if (hipPointerGetAttributes(&a, ptr) == hipSuccess && a.type == hipMemoryTypeDevice &&
+        hipMemGetAddressRange((hipDeviceptr_t *)&base, &p.size, (hipDeviceptr_t)ptr) == hipSuccess) {
+        p.device_memory = true;
+        p.device = a.device;
+        p.base = (uintptr_t)base;
+    } else {
+        (void)hipGetLastError();
+    }
+    return p;
+}
+
 int validate(const bec_fno_config &c)
 {
     if (c.nz < 1 || c.ny < 1 || c.nx < 1 || c.width < 1 || c.layers < 1 || c.c_in < 1 || c.c_out < 1 ||
@@ -701,6 +719,7 @@ void init_params(bec_fno *f, uint64_t seed, std::vector<float> &p)
 int create(const bec_fno_config &c, uint64_t seed, bec_fno *f)
 {
     f->c = c;
+    BEC_HIP(hipGetDevice(&f->device));
     f->S = (long)c.nz * c.ny * c.nx;
     f->P = (long)c.ny * c.nx;
     f->mxy = (long)c.my * c.mx;
@@ -830,15 +849,9 @@ extern "C" int bec_fno_forward(bec_fno *f, int batch, const float *d_x, float *d
 {
     if (!f || !d_x || !d_y || batch < 1 || batch > f->c.max_batch) return BEC_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
-    const size_t out = sizeof(float) * batch * f->S * f->c.c_out;
-    bec::CallerBuffers reg(f, {{d_x, sizeof(float) * batch * f->S * f->c.c_in}, {d_y, out}});
-    // straight into the caller's buffer where it is a device allocation that holds
-    // the output; the copy reports what else it is given
-    void *base = nullptr;
-    size_t size = 0;
-    const bool direct = hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)d_y) == hipSuccess &&
-                        (uintptr_t)d_y % sizeof(float) == 0 && (char *)d_y + out <= (char *)base + size;
-    if (!direct) (void)hipGetLastError();
+    const size_t out = sizeof(float) * batch * f->S * f->c.c_out, in = sizeof(float) * batch * f->S * f->c.c_in;
+    bec::CallerBuffers reg(f, {{d_x, in}, {d_y, out}});
+    const bool direct = bec::writes_direct(bec::output_place(d_y), f->device, (uintptr_t)d_y, out, (uintptr_t)d_x, in);
     BEC_HIP(bec::forward_impl(f, batch, d_x, direct ? d_y : f->y, false, s));
     if (!direct) BEC_HIP(hipMemcpyAsync(d_y, f->y, out, hipMemcpyDeviceToDevice, s));
     return BEC_OK;

@@ -170,3 +170,39 @@ def test_more_planes_than_a_grid_dimension_holds(bec):
     for name, sl in _blocks(ocfg):
         mean = (g[1][sl] + g[2][sl]) / 2
         assert np.linalg.norm(g[0][sl] - mean) < 400 * 6e-8 * np.linalg.norm(mean), name
+
+
+def test_output_anywhere_the_copy_takes_it(bec):
+    """The output in device memory (stored by the last kernel), in pinned host memory and over the end of the
+    input (both copied): the same bits."""
+    from bec_amd import fno as F
+    batch, cells = 3, 32 * 64
+    net = F.FNO(seed=6, nz=32, ny=8, nx=8, mz=8, my=8, mx=8, width=16, layers=2, c_in=16, c_out=2, hidden=32, max_batch=batch)
+    x = np.random.default_rng(6).normal(size=(batch, cells, 16)).astype(np.float32)
+    y = net.predict(x)
+    assert np.isfinite(y).all() and np.abs(y).max() > 0
+    # pinned host memory
+    hip = F.flib()
+    pinned = F.C.c_void_p()
+    assert hip.hipHostMalloc(F.C.byref(pinned), F.C.c_size_t(y.nbytes), F.C.c_uint(0)) == 0
+    try:
+        host = np.frombuffer((F.C.c_char * y.nbytes).from_address(pinned.value), dtype=np.float32)
+        host[:] = 0
+        net.forward(F.DeviceArray(x.shape, np.float32, x), F.DeviceView(_Pinned(pinned, y.nbytes), 0), batch)
+        F.device_synchronize()
+        assert np.array_equal(host.reshape(y.shape), y)
+    finally:
+        hip.hipHostFree(pinned)
+    # over the last 16 values of the input and beyond it
+    both = F.DeviceArray((x.size + y.size,), np.float32, np.concatenate([x.ravel(), np.zeros(y.size, np.float32)]))
+    at = x.size - 16
+    net.forward(both, F.DeviceView(both, 4 * at), batch)
+    F.device_synchronize()
+    assert np.array_equal(both.download()[at:at + y.size].reshape(y.shape), y)
+
+
+class _Pinned:
+    """Pinned host memory, as a view's base."""
+
+    def __init__(self, ptr, nbytes):
+        self.ptr, self.nbytes = ptr, nbytes
