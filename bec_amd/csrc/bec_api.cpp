@@ -235,18 +235,36 @@ int group_build_tables(Group &g, double dt, hipStream_t s)
     return BEC_OK;
 }
 
+static Schedule schedule_of(const DevGroup &d)
+{
+    return {d.pw ? d.pw : default_pw(d.prec, d.nx, d.nz), d.z_r1 ? d.z_r1 : default_r1(d.nz), d.z_split, d.nt, d.xcd,
+            d.xy_minw ? d.xy_minw : 1, d.z_half, d.xy_split};
+}
+
+static void apply_schedule(DevGroup &d, const Schedule &c)
+{
+    d.pw = c.pw;
+    d.z_r1 = c.z_r1;
+    d.z_split = c.z_split;
+    d.nt = c.nt;
+    d.xcd = c.xcd;
+    d.xy_minw = c.xy_minw;
+    d.z_half = c.z_half;
+    d.xy_split = c.xy_split;
+}
+
+// The schedule that every single choice goes with: one component per z workgroup,
+// whole values exchanged, streaming accesses in FP32.
+static Schedule plain_schedule(const DevGroup &d)
+{
+    return {default_pw(d.prec, d.nx, d.nz), default_r1(d.nz), 1, d.prec == 0 ? 1 : 0, d.ntraj % 8 == 0 ? 1 : 0, 1, 0, 0};
+}
+
 // The schedule a group starts with: where each choice pays, from sweeps over
 // lattices of 64..256 x 16..32^2 and 1..4096 trajectories (us per step).
 static void default_schedule(DevGroup &d)
 {
-    d.pw = 0;
-    d.z_r1 = 0;
-    d.z_split = 1;   // one component per z workgroup
-    d.nt = d.prec == 0 ? 1 : 0;
-    d.xcd = d.ntraj % 8 == 0 ? 1 : 0;
-    d.xy_minw = 1;
-    d.z_half = 0;
-    d.xy_split = 0;
+    apply_schedule(d, plain_schedule(d));
     const long nxy = (long)d.nx * d.ny;
     const long z_wgs = 2L * d.ntraj * nxy / default_pw(d.prec, d.nx, d.nz);
     if (d.prec != 0) {
@@ -1392,21 +1410,29 @@ extern "C" int bec_set_schedule(bec_ctx *ctx, int group, const bec_schedule *sch
     Group &g = ctx->groups[group];
     Schedule cand[64];
     const int n = schedule_candidates(g.dev.prec, g.dev.nx, g.dev.nz, g.dev.ntraj, cand, 64, true);
-    bool ok = false;
-    for (int i = 0; i < n && i < 64; ++i)
-        if (cand[i].pw == sch->pw && cand[i].z_r1 == sch->z_r1 && cand[i].z_split == sch->z_split &&
-            cand[i].nt == sch->nt && cand[i].xcd == sch->xcd && cand[i].xy_minw == sch->xy_minw &&
-            cand[i].z_half == sch->z_half && cand[i].xy_split == sch->xy_split)
-            ok = true;
-    if (!ok) return BEC_ERR_UNSUPPORTED;
-    g.dev.pw = sch->pw;
-    g.dev.z_r1 = sch->z_r1;
-    g.dev.z_split = sch->z_split;
-    g.dev.nt = sch->nt;
-    g.dev.xcd = sch->xcd;
-    g.dev.xy_minw = sch->xy_minw;
-    g.dev.z_half = sch->z_half;
-    g.dev.xy_split = sch->xy_split;
+    // the fields in bec_schedule's order
+    int Schedule::*const field[8] = {&Schedule::pw, &Schedule::z_r1, &Schedule::z_split, &Schedule::nt,
+                                     &Schedule::xcd, &Schedule::xy_minw, &Schedule::z_half, &Schedule::xy_split};
+    auto supported = [&](const Schedule &c) {
+        return std::any_of(cand, cand + std::min(n, 64), [&](const Schedule &q) {
+            return std::all_of(field, field + 8, [&](int Schedule::*f) { return q.*f == c.*f; });
+        });
+    };
+    Schedule want{sch->pw, sch->z_r1, sch->z_split, sch->nt, sch->xcd, sch->xy_minw, sch->z_half, sch->xy_split};
+    // A caller changes some fields of the schedule it has read.  The others may hold what
+    // this library chose for the group's size, which need not go with the change (the
+    // unsplit z pass exchanges whole values, say): they then return to the plain schedule.
+    const Schedule have = schedule_of(g.dev), plain = plain_schedule(g.dev);
+    unsigned given = g.schedule_given;
+    for (int i = 0; i < 8; ++i)
+        if (want.*field[i] != have.*field[i]) given |= 1u << i;
+    if (!supported(want)) {
+        for (int i = 0; i < 8; ++i)
+            if (!(given >> i & 1)) want.*field[i] = plain.*field[i];
+        if (!supported(want)) return BEC_ERR_UNSUPPORTED;
+    }
+    apply_schedule(g.dev, want);
+    g.schedule_given = given;
     // a captured step graph holds the old launch configuration
     drop_graphs(ctx);
     return BEC_OK;
@@ -1416,15 +1442,15 @@ extern "C" int bec_get_schedule(bec_ctx *ctx, int group, bec_schedule *sch)
 {
     CHECK_GROUP(ctx, group);
     if (!sch) return BEC_ERR_INVALID;
-    const DevGroup &d = ctx->groups[group].dev;
-    sch->pw = d.pw ? d.pw : default_pw(d.prec, d.nx, d.nz);
-    sch->z_r1 = d.z_r1 ? d.z_r1 : default_r1(d.nz);
-    sch->z_split = d.z_split;
-    sch->nt = d.nt;
-    sch->xcd = d.xcd;
-    sch->xy_minw = d.xy_minw ? d.xy_minw : 1;
-    sch->z_half = d.z_half;
-    sch->xy_split = d.xy_split;
+    const Schedule c = schedule_of(ctx->groups[group].dev);
+    sch->pw = c.pw;
+    sch->z_r1 = c.z_r1;
+    sch->z_split = c.z_split;
+    sch->nt = c.nt;
+    sch->xcd = c.xcd;
+    sch->xy_minw = c.xy_minw;
+    sch->z_half = c.z_half;
+    sch->xy_split = c.xy_split;
     sch->ms_per_step = 0;
     return BEC_OK;
 }

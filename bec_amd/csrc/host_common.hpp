@@ -24,6 +24,7 @@ struct Group {
     double *d_proj = nullptr;    // projection workspace (projection_doubles), allocated on first use
     void *d_avg = nullptr;       // calculateAverages workspace: x-space a, b and [cells][6], on first use
     bool initialized = false;
+    unsigned schedule_given = 0; // fields of the schedule that a caller has set (bit i: field i of bec_schedule)
 };
 
 struct DeviceBuf {

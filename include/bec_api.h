@@ -414,6 +414,9 @@ typedef struct bec_schedule {
     double ms_per_step;   /* filled by bec_autotune */
 } bec_schedule;
 
+/* Fields that no call has changed yet hold the library's choice for the group's
+ * size; where that does not go with the fields that are changed, they take the
+ * plain schedule's values (bec_get_schedule returns what runs). */
 int bec_set_schedule(bec_ctx *ctx, int group, const bec_schedule *sch);
 int bec_get_schedule(bec_ctx *ctx, int group, bec_schedule *sch);
 /* Candidate schedules for the group's lattice, precision and batch (*count of

@@ -376,3 +376,30 @@ def test_each_component_of_the_state_owns_its_memory(bec):
         for space in (bec.SPACE_X, bec.SPACE_K, bec.SPACE_HYBRID):
             for v in s.get_state(space):
                 assert v.base is None and v.flags.owndata and v.shape == (2, 64, 16, 16)
+
+
+@pytest.mark.parametrize("prec,n,nz,ne,change", [
+    (0, 16, 128, 4, dict(z_split=0)), (0, 16, 128, 256, dict(z_split=0)), (0, 16, 128, 256, dict(xy_minw=5)),
+    (0, 32, 64, 64, dict(xy_minw=5)), (0, 16, 256, 128, dict(z_split=0)), (1, 32, 128, 8, dict(z_half=0)),
+    (1, 16, 128, 32, dict(z_half=0)), (0, 16, 128, 256, dict(z_half=0, z_split=0)),
+])
+def test_one_field_of_the_schedule_can_be_changed_at_any_size(bec, prec, n, nz, ne, change):
+    """A program that changes one field need not know what else the library chose for its size.  The steps
+    stay the same step (rounding apart: 1e-5 and 1e-12 after two)."""
+    c = gpu_calc(bec, **config1_model(bec, N=30000, nvx=n, nvy=n, nvz=nz, ne=ne, dt_evo=2e-5))
+    with bec.Solver(c, precision=prec) as s:
+        s.init_evolution(np.ones((nz, n, n)), 5)
+        start = s.get_state(bec.SPACE_HYBRID)
+        ref = s.propagate(2, sample_every=2)
+        for k, v in change.items():   # one after the other, each on what is set by then
+            s.set_schedule(**{k: v})
+        assert all(s.schedule()[k] == v for k, v in change.items())
+        s.set_state(*start, space=bec.SPACE_HYBRID)
+        assert rel_l2(s.propagate(2, sample_every=2), ref) < (1e-5 if prec == 0 else 1e-12)
+        kept = s.schedule()
+        for bad in (dict(xy_minw=3), dict(z_r1=12), dict(pw=128), dict(nt=2)):
+            with pytest.raises(bec.BecError):
+                s.set_schedule(**bad)
+        assert s.schedule() == kept
+        s.set_schedule(**{k: v for k, v in kept.items() if k != "ms_per_step"})
+        assert s.schedule() == kept
