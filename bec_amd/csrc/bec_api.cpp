@@ -260,9 +260,15 @@ static Schedule plain_schedule(const DevGroup &d)
     return {default_pw(d.prec, d.nx, d.nz), default_r1(d.nz), 1, d.prec == 0 ? 1 : 0, d.ntraj % 8 == 0 ? 1 : 0, 1, 0, 0};
 }
 
+static long state_bytes(const DevGroup &d) { return (d.prec == 0 ? 16L : 32L) * d.ntraj * d.nx * d.ny * d.nz; }
+
+static bool may_cache(const DevGroup &d) { return state_bytes(d) >> 20 <= 384; }
+
 // The schedule a group starts with: where each choice pays, from sweeps over
-// lattices of 64..256 x 16..32^2 and 1..4096 trajectories (us per step).
-static void default_schedule(DevGroup &d)
+// lattices of 64..256 x 16..32^2 and 1..4096 trajectories (us per step).  cached: the
+// bytes of the states, among the groups that step together, that the last-level cache
+// may hold parts of between the passes (one beyond 400 MB streams in any case).
+static void default_schedule(DevGroup &d, long cached)
 {
     apply_schedule(d, plain_schedule(d));
     const long nxy = (long)d.nx * d.ny;
@@ -288,11 +294,16 @@ static void default_schedule(DevGroup &d)
     // the passes (160 trajectories 70 -> 62, 256: 98 -> 92, 512: 190 -> 174, 768: 283 ->
     // 268), beyond it streaming ones are better (2048: 725 against 761).  From 72 MB on the
     // passes wait on memory, and half the LDS to a z workgroup puts more of them on a CU
-    // (2048: 737 -> 725); with 256 z points it does not pay beyond the cache.
-    const long mib = 16L * d.ntraj * d.nz * nxy >> 20;
+    // (2048: 737 -> 725); with 256 z points it does not pay beyond the cache.  Groups that
+    // step together share the cache and stream from half a GB of them on, the larger
+    // lattices sooner (streaming against temporal: two groups of 512 of 128x16x16 359,
+    // 348 and four 730, 743; five of 512 of 64x16x16 452, 434 and three of 1200 641, 649;
+    // two of 320 of 64x32x32 453, 464; two of 56 of 256x32x32 359, 356 and of 64 408, 416).
+    const long mib = state_bytes(d) >> 20, cells = d.nz * nxy;
     if (mib > 72) {
-        if (mib <= 384) d.nt = 0;
-        d.z_half = mib <= 384 || d.nz <= 128 ? 1 : 0;
+        const bool temporal = may_cache(d) && cached >> 20 <= (cells <= 16384 ? 640 : cells <= 131072 ? 512 : 448);
+        if (temporal) d.nt = 0;
+        d.z_half = temporal || d.nz <= 128 ? 1 : 0;
     }
 }
 
@@ -313,7 +324,7 @@ int group_setup(Group &g, const bec_calc_params &c, int prec, int ntraj, bool al
     d.ntraj = ntraj;
     d.rec_shift = 30;
     d.n_records = 1;
-    default_schedule(d);
+    default_schedule(d, state_bytes(d));
     d.itmax1 = c.itmax == 1 ? 1 : 0;
     const size_t es = elem_size(prec);
     if (alloc_state) {
@@ -490,6 +501,9 @@ extern "C" int bec_create_groups(const bec_calc_params *groups, int n_groups, in
             return st;
         }
     }
+    long cached = 0;
+    for (const auto &g : ctx->groups) cached += may_cache(g.dev) ? state_bytes(g.dev) : 0;
+    for (auto &g : ctx->groups) default_schedule(g.dev, cached);
     if (hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming) != hipSuccess) {
         bec_destroy(ctx);

@@ -125,3 +125,18 @@ def test_full_size_fp32_populations_match_fp64(full_runs):
             for k in ("N1", "N2", "Na", "Nb"):
                 assert abs(o32[g][k] - o64[g][k]) < 1e-4 * abs(N), (losses, g, k)
             assert abs(o32[g]["visibility"] - o64[g]["visibility"]) < 1e-4, (losses, g)
+
+
+@pytest.mark.parametrize("n,nz,ne,n_groups,nt", [
+    (16, 128, 512, 1, 0), (16, 128, 160, 2, 0), (16, 128, 512, 2, 0), (16, 128, 512, 4, 1), (16, 64, 512, 5, 0),
+    (32, 64, 320, 2, 1), (32, 256, 56, 2, 0), (32, 256, 64, 2, 1), (16, 128, 1024, 1, 1)])
+def test_access_type_follows_the_sum_of_the_groups(bec, n, nz, ne, n_groups, nt):
+    """Groups that step together share the cache: streaming accesses from half a GB of states on (by lattice),
+    although each group alone would keep temporal ones up to 400 MB."""
+    c = gpu_calc(bec, **config1_model(bec, N=30000, nvx=n, nvy=n, nvz=nz, ne=ne, dt_evo=DT))
+    with bec.Solver(None, groups=[c] * n_groups, precision=bec.FP32) as s:
+        assert [s.schedule(g)["nt"] for g in range(n_groups)] == [nt] * n_groups
+    # a group that streams by itself takes no cache from the others
+    big = gpu_calc(bec, **config1_model(bec, N=30000, nvx=32, nvy=32, nvz=256, ne=128, dt_evo=DT))
+    with bec.Solver(None, groups=[c, big], precision=bec.FP32) as s:
+        assert [s.schedule(g)["nt"] for g in (0, 1)] == [int(ne == 1024), 1]
