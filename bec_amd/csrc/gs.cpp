@@ -18,7 +18,7 @@ namespace {
 
 struct GsWork {
     Group g;
-    void *X = nullptr, *W = nullptr, *P = nullptr, *KC = nullptr, *Q = nullptr;
+    void *X = nullptr, *W = nullptr, *P = nullptr, *KC = nullptr;
     double *ph = nullptr, *pr = nullptr, *pm = nullptr, *pn = nullptr;
     double *sums = nullptr;        // [batch][8] reduced sums
     double *exy = nullptr, *ez = nullptr, *mu_tf = nullptr, *ones = nullptr;
@@ -169,23 +169,23 @@ int setup_work(GsWork &w, const bec_calc_params *params, int batch, int prec, hi
     return BEC_OK;
 }
 
-// Residual machinery on the x-space iterate X (scale sc.s pending).
-hipError_t residual_pass(GsWork &w, const GsScalars &sc, double tol, int check, hipStream_t s)
+// Residual machinery on the x-space iterate X (scale sc.s pending), in the workspace `work`.
+hipError_t residual_pass(GsWork &w, void *work, const GsScalars &sc, double tol, int check, hipStream_t s)
 {
     const DevGroup &d = w.g.dev;
     GsTables t{w.exy, w.ez};
     hipError_t e;
-    if ((e = gs_xy_forward(d, w.X, w.W, sc, s)) != hipSuccess) return e;
-    if ((e = gs_z_diag(d, w.W, sc, t, 0, 0.0, nullptr, s)) != hipSuccess) return e;
-    if ((e = gs_xy_hamiltonian(d, w.X, w.W, sc, w.ph, s)) != hipSuccess) return e;
+    if ((e = gs_xy_forward(d, w.X, work, sc, s)) != hipSuccess) return e;
+    if ((e = gs_z_diag(d, work, sc, t, 0, 0.0, nullptr, s)) != hipSuccess) return e;
+    if ((e = gs_xy_hamiltonian(d, w.X, work, sc, w.ph, s)) != hipSuccess) return e;
     if ((e = gs_scalar_mu(d, w.ph, sc, s)) != hipSuccess) return e;
-    if ((e = gs_xy_residual(d, w.X, w.W, sc, w.pr, s)) != hipSuccess) return e;
+    if ((e = gs_xy_residual(d, w.X, work, sc, w.pr, s)) != hipSuccess) return e;
     return gs_scalar_residual(d, w.ph, w.pr, sc, tol, check, s);
 }
 
-// One split-step iteration in three launches: the x-space step (on Q, where the
+// One split-step iteration in three launches: the x-space step (on W, where the
 // previous z pass left the state half a kinetic step ahead), the z pass that ends
-// this iteration in P and begins the next in Q, and the energy integral.  Its
+// this iteration in P and begins the next in W, and the energy integral.  Its
 // test and renormalisation run inside the next x-space step (*pending: they are
 // still to do), so nothing waits on a launch of its own: five launches before,
 // each about 2 us behind the other for a state that fills few CUs.
@@ -194,15 +194,15 @@ int split_step_iteration(GsWork &w, const bec_gs_options &o, int it, bool *pendi
     const DevGroup &d = w.g.dev;
     const int rule = o.rule == BEC_GS_RULE_REFERENCE;
     GsTables t{w.exy, w.ez};
-    GS_HIP(gs_xy_nonlinear_imag(d, w.Q, w.sc, s, *pending ? w.pm : nullptr, o.tol, rule));
-    GS_HIP(gs_z_step(d, w.Q, w.P, w.KC, w.sc, s));
+    GS_HIP(gs_xy_nonlinear_imag(d, w.W, w.sc, s, *pending ? w.pm : nullptr, o.tol, rule));
+    GS_HIP(gs_z_step(d, w.W, w.P, w.KC, w.sc, s));
     GS_HIP(gs_xy_measure_ref(d, w.P, w.KC, w.sc, t, w.pm, s));
     *pending = true;
     if (o.rule == BEC_GS_RULE_RESIDUAL && (it + 1) % std::max(1, o.check_every) == 0) {
         GS_HIP(gs_scalar_ref(d, w.pm, w.sc, o.tol, rule, s));
         *pending = false;
         GS_HIP(run_xy_fft(d, w.P, w.X, d.ntraj, -1, 1.0, s));
-        GS_HIP(residual_pass(w, w.sc, o.tol, 1, s));
+        GS_HIP(residual_pass(w, w.KC, w.sc, o.tol, 1, s));   // W holds the next iteration's start; KC is read out
     }
     return BEC_OK;
 }
@@ -235,7 +235,7 @@ int final_report(GsWork &w, const bec_calc_params *params, int batch, hipStream_
     GsScalars sc = w.sc;
     sc.done = w.zero_done;
     sc.s = w.ones;
-    GS_HIP(residual_pass(w, sc, 0.0, 0, s));
+    GS_HIP(residual_pass(w, w.W, sc, 0.0, 0, s));
     const int per = xy_wg_per_traj(d);
     std::vector<double> h5(5 * (size_t)batch), r1(batch), m4(4 * (size_t)batch), mu(batch), res(batch);
     GS_HIP(run_reduce_partials(w.ph, per, batch, 5, w.sums, s));
@@ -278,7 +278,7 @@ int final_report2(GsWork &w, const bec_calc_params *params, int batch, hipStream
     GsScalars sc = w.sc;
     sc.done = w.zero_done;
     sc.s = w.ones;
-    GS_HIP(residual_pass(w, sc, 0.0, 0, s));
+    GS_HIP(residual_pass(w, w.W, sc, 0.0, 0, s));
     const int per = xy_wg_per_traj(d);
     std::vector<double> h5(5 * (size_t)ntraj), mu(ntraj), res(ntraj);
     GS_HIP(run_reduce_partials(w.ph, per, ntraj, 5, w.sums, s));
@@ -363,8 +363,7 @@ int gs_solve(const bec_calc_params *params, int batch, const double *guesses, co
     if (o.method == BEC_GS_SPLIT_STEP) {
         GS_HIP(gs_xy_forward(d, w.X, w.P, w.sc, s));     // x -> hybrid, renormalised
         GS_HIP(gs_apply_scale(d, w.X, w.sc, s));          // keeps X consistent, s <- 1
-        GS_HIP(w.alloc(&w.Q, elem_size(o.precision) * n));
-        GS_HIP(gs_z_imag(d, w.P, w.Q, w.sc, s));          // the first half step
+        GS_HIP(gs_z_imag(d, w.P, w.W, w.sc, s));          // the first half step
     } else {
         GS_HIP(gs_apply_scale(d, w.X, w.sc, s));
         GS_HIP(hipMemcpyAsync(w.P, w.X, elem_size(o.precision) * n, hipMemcpyDeviceToDevice, s));
@@ -456,7 +455,7 @@ int gs_residual_of(const bec_calc_params &c, int prec, const double *psi_x, hipS
     GsScalars sc = w.sc;
     sc.done = w.zero_done;
     sc.s = w.ones;
-    GS_HIP(residual_pass(w, sc, 0.0, 0, s));
+    GS_HIP(residual_pass(w, w.W, sc, 0.0, 0, s));
     double r = 0, m = 0;
     GS_HIP(hipMemcpyAsync(&r, sc.res, sizeof(double), hipMemcpyDeviceToHost, s));
     GS_HIP(hipMemcpyAsync(&m, sc.mu, sizeof(double), hipMemcpyDeviceToHost, s));

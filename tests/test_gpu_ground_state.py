@@ -51,3 +51,25 @@ def test_batched_ground_states_match_single(bec, oracle):
         r, _ = oracle.residual(oc, out[i])
         assert r < 1.05e-6, (i, r)
         assert reps[i]["converged"]
+
+
+SETS = [(20000, 11.96), (95000, 6.0), (8000, 19.0), (30000, 8.0), (60000, 14.0), (12000, 10.0), (5000, 20.0), (45000, 9.0)]
+
+
+def _sets(bec, oracle, nz, n, sets):
+    models = [config1_model(oracle, ne=1, nvx=n, nvy=n, nvz=nz, N=N, fz=fz) for N, fz in SETS[:sets]]
+    return [gpu_calc(bec, **m) for m in models], [oracle_calc(oracle, **m) for m in models]
+
+
+@pytest.mark.parametrize("nz,n", [(128, 16), (64, 32)])
+def test_split_step_residual_rule_every_third_iteration(bec, oracle, nz, n):
+    """The residual test between fused iterations: its workspace is neither the state the next iteration
+    starts from nor the one it returns."""
+    params, oc = _sets(bec, oracle, nz, n, 3)
+    out, reps, st = bec.ground_states_batched(params, rule=bec.GS_RULE_RESIDUAL, tol=3e-2, check_every=3, precision=bec.FP64)
+    assert st == 0
+    for psi, rep, c in zip(out, reps, oc):
+        x, orep = oracle.ground_state(c, rule=oracle.RULE_RESIDUAL, tol=3e-2, check_every=3)
+        assert rep["iterations"] == orep.iterations
+        assert rel_l2(psi, x) < 1e-10
+        assert abs(rep["residual"] - orep.residual) < 1e-6 * orep.residual
