@@ -61,6 +61,24 @@ def _sets(bec, oracle, nz, n, sets):
     return [gpu_calc(bec, **m) for m in models], [oracle_calc(oracle, **m) for m in models]
 
 
+@pytest.mark.parametrize("nz,n,sets,tol", [(128, 16, 3, 1e-5), (256, 16, 3, 1e-4), (64, 32, 3, 1e-5), (128, 16, 8, 1e-4),
+                                           (64, 16, 8, 1e-5)])
+def test_batched_split_step_matches_oracle_set_by_set(bec, oracle, nz, n, sets, tol):
+    """Sets of one solve stop at different iterations (2 to 312, in different blocks between two polls), in odd
+    and XCD-placed counts; each one's iterations, state and energies are those of its own solve, at the bars
+    of the single solve above."""
+    params, oc = _sets(bec, oracle, nz, n, sets)
+    out, reps, st = bec.ground_states_batched(params, tol=tol, precision=bec.FP64)
+    assert st == 0
+    ref = [oracle.ground_state(c, rule=oracle.RULE_REFERENCE, tol=tol) for c in oc]
+    assert [r["iterations"] for r in reps] == [r.iterations for _, r in ref]
+    assert len({r.iterations // 16 for _, r in ref}) > 1
+    for psi, rep, (x, orep) in zip(out, reps, ref):
+        assert rel_l2(psi, x) < 1e-10
+        for key in ("E_ref", "mu_ref", "E", "mu"):
+            assert abs(rep[key] - getattr(orep, key)) < 1e-9 * abs(getattr(orep, key)), key
+
+
 @pytest.mark.parametrize("nz,n", [(128, 16), (64, 32)])
 def test_split_step_residual_rule_every_third_iteration(bec, oracle, nz, n):
     """The residual test between fused iterations: its workspace is neither the state the next iteration
@@ -73,3 +91,12 @@ def test_split_step_residual_rule_every_third_iteration(bec, oracle, nz, n):
         assert rep["iterations"] == orep.iterations
         assert rel_l2(psi, x) < 1e-10
         assert abs(rep["residual"] - orep.residual) < 1e-6 * orep.residual
+
+
+def test_fp32_split_step_follows_the_fp64_one(bec, oracle):
+    """40 iterations of eight sets in FP32: about a dozen roundings of 6e-8 a cell and iteration, which the
+    contracting steps don't amplify: 40 x sqrt(12) x 6e-8 = 8e-6 at most, were they all to add up."""
+    params, _ = _sets(bec, oracle, 128, 16, 8)
+    got = [bec.ground_states_batched(params, tol=1e-30, max_iter=40, precision=p) for p in (bec.FP32, bec.FP64)]
+    assert all(r["iterations"] == 40 for _, reps, _ in got for r in reps)
+    assert rel_l2(got[0][0], got[1][0], axis=(1, 2, 3)).max() < 8e-6
