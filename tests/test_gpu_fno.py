@@ -206,3 +206,40 @@ class _Pinned:
 
     def __init__(self, ptr, nbytes):
         self.ptr, self.nbytes = ptr, nbytes
+
+
+@pytest.mark.parametrize(
+    "ny,nx,width,batch,wide",
+    [
+        (16, 16, 16, 32, True),    # 64 rows per wavefront, forward and adjoint, at every width
+        (16, 16, 32, 32, True),
+        (16, 16, 64, 32, True),    # 66,560 bytes of staged columns
+        (16, 32, 32, 1, False),    # 66,048
+        (16, 32, 64, 2, False),    # 132,096: the longest plane at the largest width
+    ],
+)
+def test_plane_transform_forms_match_oracle(bec, ny, nx, width, batch, wide):
+    """The plane transforms that take 64 rows of the DFT matrix per wavefront (a thousand workgroups and more)
+    and those that stage more than 64 KiB, at the bars of the network shapes above."""
+    from bec_amd import fno as F
+    from oracle import fno_oracle as FO
+    nz, mz, m = 32, 16, 8
+    planes, rows = batch * mz, (2 * m * m, 2 * ny * nx)   # of the two directions
+    assert all((r % 64 == 0 and planes * (r // 64) >= 1024) == wide for r in rows)
+    cells = nz * ny * nx
+    net = F.FNO(seed=8, nz=nz, ny=ny, nx=nx, mz=mz, my=m, mx=m, width=width, layers=1, c_in=8, c_out=2, hidden=16, max_batch=batch)
+    ocfg = FO.Config.from_struct(net.cfg)
+    rng = np.random.default_rng(8)
+    x = rng.normal(size=(batch, cells, 8)).astype(np.float32)
+    t = rng.normal(size=(batch, cells, 2)).astype(np.float32)
+    flat = net.get_params().astype(np.float64)
+    y = net.predict(x)
+    ref = FO.forward(ocfg, flat, _grid(x, ocfg)).reshape(y.shape)
+    assert np.linalg.norm(y - ref) < 2e-2 * np.linalg.norm(ref)
+    net.loss_backward(F.DeviceArray(x.shape, np.float32, x), F.DeviceArray(t.shape, np.float32, t), batch)
+    g = net.get_grads().astype(np.float64)
+    _, g_ref = FO.loss_and_grads(ocfg, flat, _grid(x, ocfg), _grid(t, ocfg))
+    for name, sl in _blocks(ocfg):
+        a, b = g[sl], g_ref[sl]
+        rel = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+        assert rel < 5e-2 and a @ b > 0.998 * np.linalg.norm(a) * np.linalg.norm(b), (name, rel)
