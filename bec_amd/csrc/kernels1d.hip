@@ -25,6 +25,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
+
 #include "backend1d.hpp"
 #include "fastmath.hpp"
 #include "fft_reg.hpp"
@@ -269,11 +271,11 @@ __global__ __launch_bounds__(H ? 64 : 256) void w1d_ground_state_kernel(W1dParam
 // x-space density minus the vacuum term after the last step.
 template <int H>
 __global__ __launch_bounds__(H ? 64 : 512) void w1d_ensemble_kernel(W1dParams p, int n, const double2 *gs, double *meas,
-                                                           double *avn, uint32_t k0, uint32_t k1)
+                                                           double *avn, uint32_t k0, uint32_t k1, int first)
 {
     extern __shared__ double2 lds[];
     __shared__ double scratch[64];
-    const int traj = blockIdx.x;
+    const int traj = first + blockIdx.x;
     const Line l = make_line<2>(n, lds);
     Factors<H> f;
     f.load(l);
@@ -421,12 +423,11 @@ template <class Fn> static hipError_t with_terms(int n, Fn &&f)
 {
     const int h = n / 2;
     if (n > MAXNV) return hipErrorInvalidValue;
-    if (h <= 8) f(std::integral_constant<int, 8>{});
-    else if (h <= 16) f(std::integral_constant<int, 16>{});
-    else if (h <= 24) f(std::integral_constant<int, 24>{});
-    else if (h <= 31) f(std::integral_constant<int, 32>{});
-    else f(std::integral_constant<int, 0>{});
-    return hipGetLastError();
+    if (h <= 8) return f(std::integral_constant<int, 8>{});
+    if (h <= 16) return f(std::integral_constant<int, 16>{});
+    if (h <= 24) return f(std::integral_constant<int, 24>{});
+    if (h <= 31) return f(std::integral_constant<int, 32>{});
+    return f(std::integral_constant<int, 0>{});
 }
 
 hipError_t run_w1d_ground_state(const W1dParams &p, int n, double2 *gs_out, double *ntot, double *rep_out,
@@ -436,6 +437,7 @@ hipError_t run_w1d_ground_state(const W1dParams &p, int n, double2 *gs_out, doub
         constexpr int H = decltype(Ht)::value;
         hipLaunchKernelGGL(w1d_ground_state_kernel<H>, dim3(1), dim3(threads_for(n, 1)), lds_bytes(n, 1), s, p, n, gs_out,
                            ntot, rep_out);
+        return hipGetLastError();
     });
 }
 
@@ -444,8 +446,15 @@ hipError_t run_w1d_ensemble(const W1dParams &p, int n, const double2 *gs, double
     const uint32_t k0 = (uint32_t)p.seed, k1 = (uint32_t)(p.seed >> 32);
     return with_terms(n, [&](auto Ht) {
         constexpr int H = decltype(Ht)::value;
-        hipLaunchKernelGGL(w1d_ensemble_kernel<H>, dim3((unsigned)p.ne), dim3(threads_for(n, 2)), lds_bytes(n, 2), s, p, n,
-                           gs, meas, avn, k0, k1);
+        // a launch holds less than 2^32 threads: 8.4 million trajectories of 511 cells
+        const int threads = threads_for(n, 2), most = (int)(0xffffffffL / threads);
+        hipError_t e = hipSuccess;
+        for (int first = 0; first < p.ne && e == hipSuccess; first += most) {
+            hipLaunchKernelGGL(w1d_ensemble_kernel<H>, dim3((unsigned)std::min(most, p.ne - first)), dim3(threads),
+                               lds_bytes(n, 2), s, p, n, gs, meas, avn, k0, k1, first);
+            e = hipGetLastError();
+        }
+        return e;
     });
 }
 

@@ -141,3 +141,15 @@ def test_norm_does_not_drift(bec, nv):
     drift = (n[-1] - n[0]) / n[0] / (steps - 1)
     print(f"{nv} cells: {drift:+.1e} a step")
     assert abs(drift) < 1e-16
+
+
+def test_more_trajectories_than_a_launch_holds_threads(bec):
+    """8.4 million trajectories of 511 cells, 2^32 threads and more: every one contributes (means of the samples
+    and of the densities within six standard errors of a tenth of a million's; the sums are the same seed's)."""
+    kw = dict(dz=20.0 / 255.5, ntW=1, tmaxGP=0.01, seed=5)
+    few, many = (bec.run_1d(bec.params1d(ne=ne, **kw)) for ne in (100_000, 8_400_000))
+    assert np.all(np.abs(many["m"] - few["m"]) < 6 * few["var"])
+    assert np.all(many["var"] < few["var"] / 8)
+    # a cell's density n + vacuum has at most the deviation of an exponential distribution, its mean
+    dens = few["avn"] + 0.75 / 2 / kw["dz"]
+    assert np.all(np.abs(many["avn"] - few["avn"]) < 6 * dens / np.sqrt(100_000))
