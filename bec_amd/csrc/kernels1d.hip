@@ -10,11 +10,11 @@
 //   X_{n-k} = the same with the other sign,
 // so a thread that owns cells k and n - k of one component forms both outputs
 // with 4 multiply-adds per j, a quarter of the plain sum's.  It stages its own
-// S_k and D_k into LDS; the j loop reads them as broadcasts.  Up to h = 32 the
+// S_k and D_k into LDS; the j loop reads them as broadcasts.  Up to h = 31 the
 // thread keeps its cosines and sines in registers; longer lattices step
 // the index (j k) mod n into a table in LDS.  The components meet through their
 // densities (nonlinear step) and at the pulses, exchanged through LDS.  The
-// samples' six sums are reduced together, halving the values a lane carries
+// samples' five sums are reduced together, halving the values a lane carries
 // while the lanes combine, and the square root and division of a sample wait
 // until the run is over, when the lanes do them in parallel.
 //

@@ -23,8 +23,8 @@
 // stay in registers.
 //
 // Bound: FP64 issue and the LDS latency of two wavefronts per SIMD.  A step of
-// 32 trajectories at 64 x 64 takes 17.1 us (82 us with the radix-2 passes), an
-// imaginary-time step of the ground state 9.6 us.
+// 32 trajectories at 64 x 64 takes 15.2 us (82 us with the radix-2 passes), an
+// imaginary-time step of the ground state 8.7 us.
 //
 // Conventions of the program (and of the oracle's restatement): the k-space
 // kinetic factor is -k^2 with k = dk i for 2i <= n else dk (i - n),

@@ -267,7 +267,7 @@ int bec_run_2d(const bec_2d_params *p, double *m, double *var, double *vis, doub
  * programs/bec_wigner_2d.cpp/wigner_1d.cpp on the GPU, FP64 (the scheme of the
  * Scilab prototype programs/bec_wigner_1d.scilab/WignerSplitFFT.sce):
  * calculate_steady_state (:166-243) then main_loop (:245-445) for ne
- * trajectories, one wavefront per trajectory.  Field meanings are the
+ * trajectories, one workgroup per trajectory.  Field meanings are the
  * program's file-scope constants (:93-130): the lattice has
  * nv = 1 + 2 (int)(zmax / dz) cells at z = -zmax + dz j (any nv from 1 to
  * 512, the program's is 41), ntG counts the ground-state loop including its

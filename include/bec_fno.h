@@ -6,7 +6,8 @@
  *
  * Every operation of the network is a product of BF16 operands with FP32
  * accumulation, on fused kernels for widths 16, 32 and 64 and as strided batched
- * GEMMs (bec_gemm) for other shapes, in the same order of additions:
+ * GEMMs (bec_gemm) for other shapes, in the same order of additions but for two
+ * sums (the mixing R_l of a single sample at width 32, and IDFT_z from 64 modes on):
  *   lift      h0 = x P + p                       (per cell, c_in -> width)
  *   layer l   h' = act(h W_l + b_l + K_l h)      (l = 0..layers-1, no act on the last)
  *   K_l h     = Re IDFT_z IDFT_xy [ R_l(k) . DFT_xy DFT_z h ](modes)

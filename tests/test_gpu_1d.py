@@ -131,7 +131,7 @@ def test_norm_does_not_drift(bec, nv):
     """The steps are unitary: N1 + N2 of the samples is constant but for rounding.  What repeats every step
     and so accumulates is the rounding of the DFT's factors (half an ulp each, 2 c dc averaged over a
     column: 1.4e-17 at 21 cells, and two transforms a step); factors rounded as sincospi(2 m / n) and a
-    rounded 1 / n gave -2.7e-16 (21 and 63 cells) and +2.9e-16 (65) a step.  The rounding of the sums
+    rounded 1 / n gave -3.2e-16 (21 cells), -2.0e-16 (63) and +1.7e-16 (65) a step.  The rounding of the sums
     themselves averages out over 64 trajectories and the steps."""
     steps = 200 if nv < 200 else 40
     p = bec.params1d(dz=1.0 if nv == 41 else 20.0 / (nv // 2 + 0.5), ne=64, ntW=steps, seed=5)
