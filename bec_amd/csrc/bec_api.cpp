@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -26,7 +27,6 @@ struct bec_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double *d_samples = nullptr;
     size_t sample_bytes = 0;
-    std::vector<float> stage;   // FP32 values on their way to the caller (STAGE_FLOATS, on first use)
     // hipGraph of STEP_BLOCK full steps [K N] over all groups; kernel
     // arguments are device pointers only, so it stays valid when dt changes
     hipGraph_t body_graph = nullptr;
@@ -394,30 +394,17 @@ int download_complex(const void *d, double *h, long n, int prec, hipStream_t s)
         BEC_HIP(hipStreamSynchronize(s));
         return BEC_OK;
     }
-    std::vector<float> f(2 * n);
-    BEC_HIP(hipMemcpyAsync(f.data(), d, sizeof(float) * 2 * n, hipMemcpyDeviceToHost, s));
-    BEC_HIP(hipStreamSynchronize(s));
-    for (long i = 0; i < 2 * n; ++i) h[i] = f[i];
-    return BEC_OK;
-}
-
-// One component into the caller's array.  FP32 values pass through a buffer that the
-// context keeps, 512 KiB at a time (copies that the runtime stages itself; 1 MiB at a
-// time a context's first call took 1.3 ms longer).  A fresh array as large as the
-// component cost its page faults on every call: both components of 64 trajectories of
-// 128x16x16 7.0 -> 5.9 ms, of 3 of 128x32x32 0.82 -> 0.61.
-constexpr long STAGE_FLOATS = 1L << 17;
-
-static int download_component(bec_ctx *ctx, const void *d, double *h, long n)
-{
-    if (ctx->prec == 1) return download_complex(d, h, n, 1, ctx->stream);
-    ctx->stage.resize(STAGE_FLOATS);
-    float *in = ctx->stage.data();
-    for (long at = 0; at < 2 * n; at += STAGE_FLOATS) {
-        const long m = std::min(STAGE_FLOATS, 2 * n - at);
-        BEC_HIP(hipMemcpyAsync(in, (const float *)d + at, sizeof(float) * m, hipMemcpyDeviceToHost, ctx->stream));
-        BEC_HIP(hipStreamSynchronize(ctx->stream));
-        for (long i = 0; i < m; ++i) h[at + i] = in[i];
+    // FP32 values 512 KiB at a time (copies that the runtime stages itself; 1 MiB at a time
+    // a first call took 1.3 ms longer).  An array of all of them cost its page faults on
+    // every call: both components of 64 trajectories of 128x16x16 7.0 -> 5.9 ms, of 3 of
+    // 128x32x32 0.78 -> 0.65.
+    constexpr long PIECE = 1L << 17;
+    std::unique_ptr<float[]> f(new float[std::min(PIECE, 2 * n)]);
+    for (long at = 0; at < 2 * n; at += PIECE) {
+        const long m = std::min(PIECE, 2 * n - at);
+        BEC_HIP(hipMemcpyAsync(f.get(), (const float *)d + at, sizeof(float) * m, hipMemcpyDeviceToHost, s));
+        BEC_HIP(hipStreamSynchronize(s));
+        for (long i = 0; i < m; ++i) h[at + i] = f[i];
     }
     return BEC_OK;
 }
@@ -1154,8 +1141,8 @@ extern "C" int bec_get_state(bec_ctx *ctx, int group, int space, double *a, doub
     if (!g.initialized) return BEC_ERR_STATE;
     const long n = g.cells * g.dev.ntraj;
     if (space == BEC_SPACE_HYBRID) {   // the stored representation, exact (FP32 values widen exactly)
-        int st = a ? download_component(ctx, g.dev.a, a, n) : BEC_OK;
-        if (st == BEC_OK && b) st = download_component(ctx, g.dev.b, b, n);
+        int st = a ? download_complex(g.dev.a, a, n, g.dev.prec, ctx->stream) : BEC_OK;
+        if (st == BEC_OK && b) st = download_complex(g.dev.b, b, n, g.dev.prec, ctx->stream);
         return st;
     }
     void *tmp = nullptr;
@@ -1173,7 +1160,7 @@ extern "C" int bec_get_state(bec_ctx *ctx, int group, int space, double *a, doub
             st = hip_status(e);
             break;
         }
-        st = download_component(ctx, tmp, h, n);
+        st = download_complex(tmp, h, n, g.dev.prec, ctx->stream);
     }
     dev_free(tmp);
     return st;

@@ -378,6 +378,20 @@ def test_each_component_of_the_state_owns_its_memory(bec):
                 assert v.base is None and v.flags.owndata and v.shape == (2, 64, 16, 16)
 
 
+def test_two_threads_read_the_state_of_one_context(bec):
+    """The calls of two threads on one context share its stream, not their buffers."""
+    from concurrent.futures import ThreadPoolExecutor
+    c = gpu_calc(bec, **config1_model(bec, N=30000, nvx=16, nvy=16, nvz=128, ne=12, dt_evo=2e-5))
+    with bec.Solver(c, precision=bec.FP32) as s:
+        s.init_evolution(np.ones((128, 16, 16)), 3)
+        spaces = (bec.SPACE_X, bec.SPACE_K)
+        ref = [s.get_state(v) for v in spaces]
+        with ThreadPoolExecutor(2) as pool:
+            for _ in range(10):
+                for got, want in zip(pool.map(s.get_state, spaces), ref):
+                    assert all(np.array_equal(x, y) for x, y in zip(got, want))
+
+
 @pytest.mark.parametrize("prec,n,nz,ne,change", [
     (0, 16, 128, 4, dict(z_split=0)), (0, 16, 128, 256, dict(z_split=0)), (0, 16, 128, 256, dict(xy_minw=5)),
     (0, 32, 64, 64, dict(xy_minw=5)), (0, 16, 256, 128, dict(z_split=0)), (1, 32, 128, 8, dict(z_half=0)),
