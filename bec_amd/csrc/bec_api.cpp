@@ -394,11 +394,11 @@ int download_complex(const void *d, double *h, long n, int prec, hipStream_t s)
         BEC_HIP(hipStreamSynchronize(s));
         return BEC_OK;
     }
-    // FP32 values 512 KiB at a time (copies that the runtime stages itself; 1 MiB at a time
-    // a first call took 1.3 ms longer).  An array of all of them cost its page faults on
-    // every call: both components of 64 trajectories of 128x16x16 7.0 -> 5.9 ms, of 3 of
-    // 128x32x32 0.78 -> 0.65.
-    constexpr long PIECE = 1L << 17;
+    // FP32 values 896 KiB at a time: copies that the runtime stages itself (1 MiB at a time
+    // a first call took 1.3 ms longer; 512 KiB at a time 3 trajectories of 128x16x16 took
+    // 167 us, now 156).  An array of all of them cost its page faults on every call: both
+    // components of 8 trajectories 0.47 -> 0.38 ms, of 64 7.0 -> 5.6.
+    constexpr long PIECE = 7L << 15;
     std::unique_ptr<float[]> f(new float[std::min(PIECE, 2 * n)]);
     for (long at = 0; at < 2 * n; at += PIECE) {
         const long m = std::min(PIECE, 2 * n - at);
