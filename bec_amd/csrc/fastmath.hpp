@@ -188,8 +188,8 @@ BEC_HD inline void fast_sincos_f64(double x, double *s, double *c)
 BEC_HD inline void unit_root(int m, int n, double *c, double *s)
 {
     const int k = 2 * m > n ? n - m : m;           // the upper half mirrored
-    const int oct = (int)(8LL * k / n);            // 0..4
-    int r = (int)(8LL * k - (long long)oct * n);   // angle = (oct + r / n) pi/4
+    const int oct = 8 * k / n;                     // 0..4
+    int r = 8 * k - oct * n;                       // angle = (oct + r / n) pi/4
     if (oct & 1) r = n - r;                        // from the nearer multiple of pi/2
     const double d = 2.0 * n, q = r / d, ql = fma(-q, d, (double)r) / d;
     const double x = DPIO2_A * q, e = fma(DPIO2_A, q, -x) + (DPIO2_B * q + DPIO2_A * ql);
